@@ -27,7 +27,7 @@ struct AttnArgs {
     const _Float16* v;
     const uint16_t* mask; // F16 bits, may be null
     float* dst;           // [B][Nq][Hq][D]
-    float* ws;            // split-KV partial records (decode)
+    float* ws;            // scratch: split-KV partial records (decode), records of KV pieces (prefill)
     int64_t q_nb1, q_nb2, q_nb3;   // bytes
     int64_t k_nb1, k_nb2, k_nb3;   // bytes
     int64_t v_nb1, v_nb2, v_nb3;   // bytes
@@ -70,6 +70,7 @@ struct AttnArgs {
     // on [lo, hi] and -inf elsewhere ({n_kv, -1}: no live entry), else
     // {-2, -2}; written by a pre-pass launch into workspace scratch
     int2* mask_rows;
+    size_t ws_bytes;      // prefill: bytes at ws
 };
 
 // n / d for 0 <= n < 2^31 by a multiply-high, an add and a shift, with the
@@ -574,6 +575,8 @@ constexpr int kDecodeWaves = 4;      // wavefronts per decode workgroup
 // Floats per decode partial record: O [G][D], then m [G] and l [G], padded to
 // a multiple of 4 so every record starts 16-byte aligned.
 constexpr int dec_record_floats(int D, int G) { return G * D + ((2 * G + 3) & ~3); }
+// prefill beyond the kernels below; hd 128 with prefill128_takes (and a.mask_rows
+// set if there is a mask tensor) goes to launch_prefill128
 hipError_t launch_prefill(const AttnArgs& a, int head_dim, int waves, hipStream_t stream);
 // hd 64 prefill on the pipelined kernel: no mask, an implicit mask, or a mask
 // tensor (a.mask_rows: workspace for nq * hm * bm intervals, filled first by
@@ -592,6 +595,23 @@ hipError_t launch_mask_prep(const AttnArgs& a, const StageReq* stage, hipStream_
 hipError_t launch_prefill_pair(const AttnArgs& a, hipStream_t stream);
 // whether launch_prefill_pair takes these strides (its 32-bit offsets)
 bool prefill_pair_fits(const AttnArgs& a);
+// hd 128 prefill with the heads of a kv group sharing K/V blocks: no mask, an
+// implicit mask, or a mask tensor (a.mask_rows filled by launch_mask_prep
+// first); a.ws: scratch for the records of tiles cut into KV pieces (any
+// size; with less, fewer pieces)
+hipError_t launch_prefill128(const AttnArgs& a, hipStream_t stream);
+// its query heads per workgroup (log2): the largest power of two, up to 8,
+// that divides the GQA group
+inline uint32_t prefill128_heads_log2(const AttnArgs& a) {
+    uint32_t l = 0;
+    while (l < 3 && (a.hq / a.hkv) % (2 << l) == 0) ++l;
+    return l;
+}
+// whether launch_prefill takes an hd 128 call there: at least half of a
+// workgroup's 8 wavefronts (32 rows of a head each) have rows
+inline bool prefill128_takes(const AttnArgs& a) {
+    return ((((int64_t)a.nq + 31) / 32) << prefill128_heads_log2(a)) >= 4;
+}
 hipError_t launch_zero(float* dst, int64_t n, hipStream_t stream);
 hipError_t launch_kv_append(const AppendArgs& a, hipStream_t stream);
 // F32 -> f16 copies of K and V (StageReq above), one launch of their own

@@ -1,0 +1,702 @@
+// fa_prefill128.hip — hd 128 prefill for gfx950: the query heads of one kv
+// head share each K/V block, the KV range is cut into pieces when the query
+// rows alone leave the chip idle.
+//
+// Replaces the backend kernel of GGML_OP_FLASH_ATTN_EXT for the decoder
+// prefill calls of voxtral.cpp (src/voxtral.cpp:1802, GQA 32/8, hd 128, the
+// causal mask of :2104-2111) that the short masked kernel does not take:
+// n_kv over 512, or no mask.
+//
+// Work decomposition
+//   Workgroup = 8 wavefronts of 32 query rows, two per SIMD: HPW query heads
+//   of one kv head (the largest power of two dividing the GQA group, up to 8)
+//   x 8 / HPW row tiles, so a group of 4 takes 64 positions of 4 heads. All
+//   of them walk the same 32-position K/V blocks, read from L2 once for 256
+//   query rows and shared in LDS.
+//   A tile's live blocks are cut into pieces of at most `lp` blocks, one
+//   workgroup each (piece p of a tile with fewer pieces ends at once). A tile
+//   of one piece writes its output; otherwise every piece leaves its
+//   unnormalised O with the rows' running max and sum in the workspace, and
+//   fa_prefill128_combine merges them in piece order.
+// What bounds it: per wavefront and block 16 MFMAs (512 cycles of its SIMD's
+//   matrix pipe) against ~130 VALU instructions of softmax, so the two pipes
+//   are about even and have to overlap. PV runs one block behind:
+//     half t:  MFMA  O += V_{t-1}^T P(t-1)^T, then S(t+1) = K_{t+1} Q^T
+//              VALU  softmax of S(t) -> P(t)
+//   where no MFMA waits for that half's VALU work. K_{t+1} is read at the top
+//   of the half and lands under the PV MFMAs, V_t after them and lands under
+//   the S MFMAs.
+// K/V staging: a ring of 4 steps of 64 positions (32 KiB each), filled by
+//   global_load_lds_dwordx4; step u + 3 is issued in iteration u into the slot
+//   of step u - 1, one barrier after its last read, and has two iterations to
+//   land. One barrier per 64 positions.
+// MFMA operand layouts, LDS swizzles and the row-to-KV permutation are those
+// of fa_prefill.hip; the softmax without a block max (P against the running
+// max; the sum of P tells when a score passed it by more than 2^8) is that of
+// fa_prefill_pp.hip.
+// Masks: each lane's row has a live interval, from the formula of an implicit
+// mask or from the pre-pass over a mask tensor (launch_mask_prep); blocks not
+// wholly live for a wavefront's rows get their dead scores set to -inf. A
+// workgroup with a row that is no interval (finite values, holes) reads the
+// mask per block and skips the blocks that are dead for its rows.
+#include "fa_common.h"
+
+#include <type_traits>
+
+namespace vxfa {
+
+namespace p128 {
+constexpr int D = 128;
+constexpr int KS = D / 16;             // S-MFMA k-steps
+constexpr int DB = D / 32;             // O^T row blocks
+constexpr int BK = 32;                 // positions per block
+constexpr int ROW = D * 2;             // bytes per K/V row
+constexpr int BLK = BK * ROW;          // bytes of one matrix block (8 KiB)
+constexpr int STEP = 2 * BLK;          // one matrix of a 64-position step
+constexpr int NS = 4;                  // ring slots
+constexpr int NW = 8;
+constexpr int NT = 64 * NW;
+constexpr int REC = 64 * 64 + 64;      // floats of a wavefront's record: O, then (m, l) of 32 rows
+constexpr float TAU_SUM = 256.0f;      // 2^8
+constexpr float TAU = 8.0f;
+// 1/sqrt(128) in log2 units, as the host computes it from ggml's float scale
+constexpr float kC128 = 0.08838834764831845f * kLog2e;
+}  // namespace p128
+
+struct Pieces {
+    uint32_t hpw_log2;                 // log2 of the query heads per workgroup
+    uint32_t lp;                       // blocks per piece at most
+    DivMod np;                         // pieces per tile in the grid
+    int32_t nqt;                       // tiles
+    int32_t nhg;                       // head groups (hq / heads per workgroup)
+    int* count;                        // pieces of each tile [b][nhg][nqt]
+    float* rec;                        // records [b][nhg][nqt][np][NW][REC]
+};
+
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+    static_assert(N >= 0 && N < 16, "vmcnt range");
+    __builtin_amdgcn_s_waitcnt(N | (7 << 4) | (15 << 8));
+}
+
+__device__ __forceinline__ int wave_min32(int x) {
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) x = min(x, __shfl_xor(x, m, 64));
+    return __builtin_amdgcn_readfirstlane(x);
+}
+__device__ __forceinline__ int wave_max32(int x) {
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) x = max(x, __shfl_xor(x, m, 64));
+    return __builtin_amdgcn_readfirstlane(x);
+}
+
+// MM: 0 no mask, 1 a mask tensor (intervals in a.mask_rows), 2 implicit.
+// CL: the scale is exactly 1/sqrt(128) (c is a literal, see exps below).
+template <bool QF16, bool CL, int MM>
+__global__ __launch_bounds__(p128::NT) void fa_prefill128(AttnArgs a, GridMap gm, Pieces pc) {
+    using namespace p128;
+    __shared__ __attribute__((aligned(16))) char smem[NS * 2 * STEP];   // K steps, then V steps
+
+    int idx, hg, b, hk, bkv;
+    gm.locate(blockIdx.x, idx, hg, b, hk, bkv);
+    const int qt = (int)pc.np.div((uint32_t)idx);
+    const int piece = idx - qt * (int)pc.np.d;
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nl = lane & 31;
+    const int hh = lane >> 5;
+    const int hpw = 1 << pc.hpw_log2;
+    const int bm = 32 * (NW >> pc.hpw_log2);              // positions per workgroup
+    const int h = hg * hpw + (wave & (hpw - 1));
+    const int q0 = qt * bm;                               // the workgroup's first row
+    const int r0 = q0 + 32 * (wave >> pc.hpw_log2);       // the wavefront's first row
+    const int qrow = r0 + nl;
+    const bool qvalid = qrow < a.nq;
+    const int qld = min(qrow, a.nq - 1);
+    const char* kb = (const char*)a.k + (int64_t)hk * a.k_nb2 + (int64_t)bkv * a.k_nb3;
+    const char* vb = (const char*)a.v + (int64_t)hk * a.v_nb2 + (int64_t)bkv * a.v_nb3;
+
+    // ---- live interval of the lane's row, union over the workgroup ----------
+    // (MM = 1: 4 table entries per lane cover the workgroup's 256 rows; every
+    // wavefront reduces them itself, no barrier)
+    int rlo = 0, rhi = a.nkv - 1;                         // the lane's row
+    int lo = 0, hi = a.nkv;                               // the workgroup
+    bool slow = false;
+    if constexpr (MM == 1) {
+        const int2* tab = a.mask_rows + (int64_t)(b % a.bm) * a.hm * a.nq;
+        int2 iv[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int i = 64 * u + lane;                  // head i / bm of the workgroup, row i % bm
+            const int hi_ = i >> (8 - pc.hpw_log2), row = min(q0 + (i & (bm - 1)), a.nq - 1);
+            iv[u] = tab[(int64_t)((hg * hpw + hi_) % a.hm) * a.nq + row];
+        }
+        const int2 mine = tab[(int64_t)(h % a.hm) * a.nq + qld];
+        int tlo = 0x7fffffff, thi = -1;
+        bool non = false;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            non = non || iv[u].x == -2;
+            if (iv[u].x >= 0 && iv[u].x <= iv[u].y) {
+                tlo = min(tlo, iv[u].x);
+                thi = max(thi, iv[u].y);
+            }
+        }
+        slow = __any(non);
+        lo = wave_min32(tlo);
+        hi = wave_max32(thi) + 1;
+        rlo = mine.x;
+        rhi = mine.y;
+        if (slow) { lo = 0; hi = a.nkv; }
+    }
+    if constexpr (MM == 2) {
+        const int64_t q1 = min(q0 + bm, a.nq) - 1;        // the workgroup's last real row
+        const int64_t wb = a.im_window > 0 ? a.im_offset - a.im_window + 1 : INT64_MIN / 2;
+        auto clampkv = [&](int64_t x) { return (int)(x < -1 ? -1 : (x > a.nkv ? a.nkv : x)); };
+        lo = max(clampkv(q0 + wb), 0);
+        hi = min(clampkv(q1 + a.im_offset), a.nkv - 1) + 1;
+        rlo = clampkv(qld + wb);
+        rhi = min(clampkv(qld + a.im_offset), a.nkv - 1);
+    }
+    const int blo = hi > lo ? lo / BK : 0;
+    const int nblk = hi > lo ? (hi + BK - 1) / BK - blo : 0;
+
+    // ---- this piece's blocks [bs, bs + nb) -----------------------------------
+    int bs = blo, nb = nblk;
+    bool whole = true;
+    if (pc.np.d > 1) {
+        const int n = max((nblk + (int)pc.lp - 1) / (int)pc.lp, 1);
+        if (piece >= n) return;
+        whole = n == 1;
+        const int len = ((nblk + n - 1) / n + 1) & ~1;    // whole steps
+        bs = blo + min(piece * len, nblk);
+        nb = min(len, blo + nblk - bs);
+        if (piece == 0 && tid == 0) pc.count[((int64_t)b * pc.nhg + hg) * pc.nqt + qt] = n;
+    }
+
+    // ---- Q operand: row qrow, dims 16 ks + 8 hh .. + 7 ------------------------
+    half8 qb[KS];
+    floatx4 qraw[QF16 ? 1 : KS][2];
+    int qpos = 0;
+    {
+        const char* qp = (const char*)a.q + (int64_t)qld * a.q_nb1 + (int64_t)h * a.q_nb2 + (int64_t)b * a.q_nb3;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            if constexpr (QF16) {
+                qb[ks] = *(const half8*)(qp + (16 * ks + 8 * hh) * 2);
+            } else {
+                const floatx4* p = (const floatx4*)(qp + (16 * ks + 8 * hh) * 4);
+                qraw[ks][0] = p[0];
+                qraw[ks][1] = p[1];
+            }
+        }
+        if constexpr (!QF16) {
+            // (without a rotary embedding the first word of Q, unused: a
+            // branch would make the compiler wait for the loads before it)
+            const int* pp = a.rope_pos ? a.rope_pos + ((int64_t)b * a.nq + qld) : (const int*)a.q;
+            qpos = *pp;
+        }
+    }
+
+    // ---- step loads: global -> LDS ring ----------------------------------------
+    // Instruction i (0, 1) of wavefront w fills rows [4 (w + 8 i), + 4) of the
+    // step; lane l writes LDS chunk l % 16 of row + l / 16, which holds the
+    // row's chunk (l % 16) ^ swizzle(row). Rows at or past n_kv read row
+    // n_kv - 1.
+    const int nstep = (nb + 1) >> 1;
+    uint32_t ldk[2], ldv[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int r = 4 * (wave + NW * i) + (lane >> 4);
+        ldk[i] = (uint32_t)r * (uint32_t)a.k_nb1 + ((lane & 15) ^ swz_k<D>(r)) * 16;
+        ldv[i] = (uint32_t)r * (uint32_t)a.v_nb1 + ((lane & 15) ^ swz_v<D>(r)) * 16;
+    }
+    const uint32_t lds0 = lds_offset(smem);
+    auto issue = [&](int u) {
+        const int kv0 = (bs + 2 * u) * BK;
+        const uint32_t kd = lds0 + (u & (NS - 1)) * STEP, vd = kd + NS * STEP;
+        const char* kst = kb + (int64_t)kv0 * a.k_nb1;
+        const char* vst = vb + (int64_t)kv0 * a.v_nb1;
+        if (kv0 + 2 * BK <= a.nkv) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) dma16(kst, ldk[i], kd + 4 * (wave + NW * i) * ROW);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) dma16(vst, ldv[i], vd + 4 * (wave + NW * i) * ROW);
+        } else {
+            // (recomputed here rather than held across the loop; the empty asm
+            // keeps it here)
+            int ln = lane;
+            asm volatile("" : "+v"(ln));
+            const int rmax = a.nkv - 1 - kv0;   // kv0 < n_kv
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int r = 4 * (wave + NW * i) + (ln >> 4);
+                dma16(kst, (uint32_t)min(r, rmax) * (uint32_t)a.k_nb1 + ((ln & 15) ^ swz_k<D>(r)) * 16,
+                      kd + 4 * (wave + NW * i) * ROW);
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int r = 4 * (wave + NW * i) + (ln >> 4);
+                dma16(vst, (uint32_t)min(r, rmax) * (uint32_t)a.v_nb1 + ((ln & 15) ^ swz_v<D>(r)) * 16,
+                      vd + 4 * (wave + NW * i) * ROW);
+            }
+        }
+    };
+    for (int u = 0; u < min(nstep, NS - 1); ++u) issue(u);
+
+    // ---- Q: rotate, fold the sign of the scale in (0 for scale 0), round ------
+    const float c = a.scale_log2 != 0.f ? fabsf(a.scale_log2) : 1.0f;
+    {
+        const float sg = a.scale_log2 < 0.f ? -1.0f : (a.scale_log2 > 0.f ? 1.0f : 0.0f);
+        if constexpr (QF16) {
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) qb[ks] = qb[ks] * (_Float16)sg;
+        } else {
+            // one running product over the row's pairs, as ggml builds its
+            // cos / sin cache: pair 8 ks + o belongs to the lanes of half o / 4
+            float th = (float)qpos;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                float x[8] = {qraw[ks][0][0], qraw[ks][0][1], qraw[ks][0][2], qraw[ks][0][3],
+                              qraw[ks][1][0], qraw[ks][1][1], qraw[ks][1][2], qraw[ks][1][3]};
+                if (a.rope_pos) {
+                    float ang[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int o = 0; o < 8; ++o) {
+                        if (ks > 0 || o > 0) th *= a.rope_ts;
+                        if ((o >> 2) == hh) ang[o & 3] = th;
+                    }
+                    rope8_ang(x, ang, 16 * ks + 8 * hh, a.rope_dims);
+                }
+#pragma unroll
+                for (int e = 0; e < 8; ++e) qb[ks][e] = (_Float16)(x[e] * sg);
+            }
+        }
+    }
+
+    // ---- operand reads ------------------------------------------------------------
+    // K: A-operand row nl of a block is K row krow, chunk 2 ks + hh; the blocks
+    // and rows are 256-byte aligned, so the chunk (with its swizzle) is a field
+    // of the address and ks is an XOR of it.
+    int kbase;
+    {
+        const int am = nl >> 3, ahb = (nl >> 2) & 1, ab = nl & 3;
+        const int krow = ahb ? 16 + ((am + 2) & 3) * 4 + ab : 4 * am + ab;
+        kbase = krow * ROW + (hh ^ swz_k<D>(krow)) * 16;
+    }
+    // V^T operand (cc, db): rows (hh ? 24 - 8 cc : 8 cc) + vq, chunk 4 db + clo
+    // (cc flips bit 3 of the row, db bits 2 and 3 of the chunk)
+    int vbase;
+    {
+        const int vq = (lane & 15) >> 2;
+        const int clo = 2 * ((lane & 31) >> 4) + ((lane & 3) >> 1);
+        vbase = NS * STEP + ((hh ? 24 : 0) + vq) * ROW + (clo ^ swz_v<D>(vq)) * 16 + (lane & 1) * 8;
+    }
+    // block t of the piece
+    auto read_k = [&](int t, half8 (&kr)[KS]) {
+        const int base = kbase + (t & (2 * NS - 1)) * BLK;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) kr[ks] = *(const half8*)(smem + (base ^ (32 * ks)));
+    };
+    auto read_v = [&](int t, half8 (&vr)[2][DB]) {
+        const int base = vbase + (t & (2 * NS - 1)) * BLK;
+#pragma unroll
+        for (int cc = 0; cc < 2; ++cc)
+#pragma unroll
+            for (int db = 0; db < DB; ++db) {
+                const char* p = smem + (base ^ (8 * ROW * cc + 64 * db));
+                const half4 lo4 = lds_read_tr16(p);
+                const half4 hi4 = lds_read_tr16(p + 4 * ROW);
+                vr[cc][db] = half8{lo4[0], lo4[1], lo4[2], lo4[3], hi4[0], hi4[1], hi4[2], hi4[3]};
+            }
+    };
+    auto s_mfma = [&](floatx16& s, const half8 (&kr)[KS]) {
+        s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kr[0], qb[0], floatx16{}, 0, 0, 0);
+#pragma unroll
+        for (int ks = 1; ks < KS; ++ks) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kr[ks], qb[ks], s, 0, 0, 0);
+    };
+    floatx16 o[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db) o[db] = floatx16{};
+    auto pv_mfma = [&](const half8 (&p)[2], const half8 (&vr)[2][DB]) {
+#pragma unroll
+        for (int cc = 0; cc < 2; ++cc)
+#pragma unroll
+            for (int db = 0; db < DB; ++db) o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vr[cc][db], p[cc], o[db], 0, 0, 0);
+    };
+
+    // largest lower and smallest upper bound over the wavefront's rows: a
+    // block inside both is wholly live
+    const int last = min(a.nkv, (bs + nb) * BK) - 1;      // this piece's last position
+    rhi = min(rhi, last);
+    int hlo = 0, hhi = last;
+    if constexpr (MM == 1) {
+        hlo = wave_max32(rlo);
+        hhi = wave_min32(rhi);
+    }
+    if constexpr (MM == 2) {
+        hlo = __builtin_amdgcn_readlane(rlo, 31);
+        hhi = __builtin_amdgcn_readlane(rhi, 0);
+    }
+    auto mask_fix = [&](floatx16& sc, int t) {
+        const int kv0 = (bs + t) * BK;
+        if (!(kv0 >= hlo && kv0 + BK - 1 <= hhi)) {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                const int kv = kv0 + pf_kv_of(hh, j);
+                if constexpr (MM == 0) sc[j] = kv > last ? -INFINITY : sc[j];
+                else sc[j] = (kv < rlo || kv > rhi) ? -INFINITY : sc[j];
+            }
+        }
+    };
+
+    // ---- softmax ------------------------------------------------------------------
+    // P = 2^(c s - m) as two f16 B operands, and the lane's sum of them. With CL
+    // c is a literal: v_fmamk_f32 issues at twice the rate of the
+    // three-register FMA; -m has to reach it as a plain register.
+    const half2 ones = {(_Float16)1.0f, (_Float16)1.0f};
+    float m = -INFINITY, l = 0.f;
+    auto exps = [&](const floatx16& sc, half8 (&p)[2]) -> float {
+        float nm = (m == -INFINITY) ? 0.f : -m;
+        asm("" : "+v"(nm));
+        float ls[2] = {0.f, 0.f};
+#pragma unroll
+        for (int cc = 0; cc < 2; ++cc) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                p[cc][i] = (_Float16)exp2_fast(fmaf(sc[8 * cc + i], CL ? kC128 : c, nm));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const half2 p2 = {p[cc][2 * i], p[cc][2 * i + 1]};
+                ls[i & 1] = __builtin_amdgcn_fdot2(p2, ones, ls[i & 1], false);
+            }
+        }
+        return ls[0] + ls[1];
+    };
+    auto block_max = [&](const floatx16& sc) -> float {
+        float r = sc[0];
+#pragma unroll
+        for (int j = 1; j < 16; ++j) r = fmaxf(r, sc[j]);
+        return pair32_max(r) * c;
+    };
+    auto raise = [&](float mx) {
+        const float mnew = fmaxf(m, mx);
+        const float ms = (mnew == -INFINITY) ? 0.f : mnew;
+        const float alpha = exp2_fast(m - ms);
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+            for (int j = 0; j < 16; ++j) o[db][j] *= alpha;
+        l *= alpha;
+        m = mnew;
+    };
+    // (a row that has no live score yet takes the exact path; rows past n_q
+    // take no part in the choice)
+    auto softmax = [&](const floatx16& sc, half8 (&p)[2]) {
+        float ls = exps(sc, p);
+        bool up = !(ls <= TAU_SUM);
+        if constexpr (MM != 0) up = (up || m == -INFINITY) && qvalid;
+        if (__any(up)) {
+            raise(block_max(sc));
+            ls = exps(sc, p);
+        }
+        l += ls;
+    };
+
+    // before iteration 0: step 0 and the first half of step 1 (K), step 0 (V)
+    // (loads in flight may stay: all but step 0's and step 1's K)
+    {
+        const int npre = min(nstep, NS - 1);
+        if (npre >= 3) wait_vm<6>();
+        else if (npre == 2) wait_vm<2>();
+        else wait_vm<0>();
+    }
+    __syncthreads();
+
+    auto walk = [&](auto slow_tag) __attribute__((always_inline)) {
+        constexpr bool SLOW = decltype(slow_tag)::value;
+        half8 kr[KS], vr[2][DB], pa[2], pb[2];
+        floatx16 sa, sb;
+        if constexpr (SLOW) {
+            // each block on its own, its mask values read per row
+            const uint16_t* mr = (const uint16_t*)((const char*)a.mask + (int64_t)(h % a.hm) * a.m_nb2 +
+                                                   (int64_t)(b % a.bm) * a.m_nb3 + (int64_t)qld * a.m_nb1);
+            const float inv_c = kLog2e / c;
+            for (int u = 0; u < nstep; ++u) {
+                if (u + NS - 1 < nstep) issue(u + NS - 1);
+                for (int t = 2 * u; t < min(2 * u + 2, nb); ++t) {
+                    const int kv0 = (bs + t) * BK;
+                    uint16_t mv[16];
+                    if (a.mask_vec && kv0 + BK <= a.nkv) {
+                        const uint16_t* p = mr + kv0 + 16 * hh;
+                        const u32x4 w0 = *(const u32x4*)(p + 8 * hh), w1 = *(const u32x4*)(p + 8 - 8 * hh);
+#pragma unroll
+                        for (int w = 0; w < 4; ++w) {
+                            mv[2 * w] = (uint16_t)w0[w];
+                            mv[2 * w + 1] = (uint16_t)(w0[w] >> 16);
+                            mv[8 + 2 * w] = (uint16_t)w1[w];
+                            mv[8 + 2 * w + 1] = (uint16_t)(w1[w] >> 16);
+                        }
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < 16; ++j) mv[j] = mr[min(kv0 + pf_kv_of(hh, j), a.nkv - 1)];
+#pragma unroll
+                        for (int j = 0; j < 16; ++j)
+                            if (kv0 + pf_kv_of(hh, j) >= a.nkv) mv[j] = kF16NegInf;
+                    }
+                    bool live = false;
+#pragma unroll
+                    for (int j = 0; j < 16; ++j) live |= mv[j] != kF16NegInf;
+                    if (!__any(live && qvalid)) continue;
+                    read_k(t, kr);
+                    s_mfma(sa, kr);
+                    read_v(t, vr);
+#pragma unroll
+                    for (int j = 0; j < 16; ++j)
+                        sa[j] = mv[j] == kF16NegInf ? -INFINITY : fmaf(f16_bits_to_f32(mv[j]), inv_c, sa[j]);
+                    const float mx = block_max(sa);
+                    if (__any(mx > m + TAU && qvalid)) raise(mx);
+                    l += exps(sa, pa);
+                    pv_mfma(pa, vr);
+                }
+                wait_vm<0>();
+                __syncthreads();
+            }
+        } else {
+            if (nb == 0) return;
+            // PV of the block before the first adds zero
+#pragma unroll
+            for (int cc = 0; cc < 2; ++cc) {
+                pb[cc] = half8{};
+#pragma unroll
+                for (int db = 0; db < DB; ++db) vr[cc][db] = half8{};
+            }
+            read_k(0, kr);
+            s_mfma(sa, kr);
+            mask_fix(sa, 0);
+            m = block_max(sa);
+            // half t: PV(t - 1), S(t + 1) and the softmax of S(t)
+            auto half = [&](int t, floatx16& scur, floatx16& snext, half8 (&pcur)[2], half8 (&pprev)[2]) {
+                mask_fix(scur, t);
+                read_k(t + 1, kr);
+                pv_mfma(pprev, vr);
+                __builtin_amdgcn_sched_barrier(0x6);   // VALU and SALU may cross
+                read_v(t, vr);
+                s_mfma(snext, kr);
+                softmax(scur, pcur);
+            };
+            // (whole steps: a second block past nb has no live score, and the last
+            // half's S is not used)
+            for (int u = 0; u < nstep; ++u) {
+                if (u + NS - 1 < nstep) issue(u + NS - 1);
+                half(2 * u, sa, sb, pa, pb);
+                half(2 * u + 1, sb, sa, pb, pa);
+                // K of step u + 2 and V of step u + 1 have landed: at most the
+                // loads of step u + 3 and V of step u + 2 are in flight
+                if (u + 3 < nstep) wait_vm<6>();
+                else if (u + 2 < nstep) wait_vm<2>();
+                else wait_vm<0>();
+                __syncthreads();
+            }
+            pv_mfma(pb, vr);
+        }
+    };
+    if constexpr (MM == 1) {
+        if (slow) walk(std::true_type{});
+        else walk(std::false_type{});
+    } else {
+        walk(std::false_type{});
+    }
+
+    // ---- output, or this piece's record --------------------------------------------
+    const float lt = pair32_sum(l);
+    if (whole) {
+        const float inv = (lt == 0.f) ? 0.f : 1.0f / lt;
+        if (qvalid) {
+            float* out = a.dst + (((int64_t)b * a.nq + qrow) * a.hq + h) * D;
+#pragma unroll
+            for (int db = 0; db < DB; ++db)
+#pragma unroll
+                for (int a4 = 0; a4 < 4; ++a4)
+                    *(floatx4*)(out + 32 * db + 8 * a4 + 4 * hh) =
+                        floatx4{o[db][4 * a4] * inv, o[db][4 * a4 + 1] * inv, o[db][4 * a4 + 2] * inv,
+                                o[db][4 * a4 + 3] * inv};
+        }
+    } else {
+        const int64_t ri = ((((int64_t)b * pc.nhg + hg) * pc.nqt + qt) * pc.np.d + piece) * NW + wave;
+        float* rec = pc.rec + ri * REC;
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+            for (int a4 = 0; a4 < 4; ++a4)
+                *(floatx4*)(rec + (4 * db + a4) * 256 + 4 * lane) =
+                    floatx4{o[db][4 * a4], o[db][4 * a4 + 1], o[db][4 * a4 + 2], o[db][4 * a4 + 3]};
+        if (hh == 0) *(float2*)(rec + 4096 + 2 * nl) = float2{m, lt};
+    }
+}
+
+// Merge of the pieces of a tile: workgroup = one wavefront tile (32 rows of a
+// head), wavefront = 32 output dims; lane layout as in the records.
+__global__ __launch_bounds__(256) void fa_prefill128_combine(AttnArgs a, Pieces pc) {
+    using namespace p128;
+    const int lane = threadIdx.x & 63, db = threadIdx.x >> 6;
+    const int nl = lane & 31, hh = lane >> 5;
+    const int64_t tile = blockIdx.x / NW;                 // (b nhg + hg) nqt + qt
+    const int wave = blockIdx.x % NW;
+    const int n = pc.count[tile];
+    if (n <= 1) return;
+    const int qt = (int)(tile % pc.nqt);
+    const int hg = (int)(tile / pc.nqt % pc.nhg), b = (int)(tile / pc.nqt / pc.nhg);
+    const int hpw = 1 << pc.hpw_log2;
+    const int h = hg * hpw + (wave & (hpw - 1));
+    const int qrow = qt * 32 * (NW >> pc.hpw_log2) + 32 * (wave >> pc.hpw_log2) + nl;
+    if (qrow - nl >= a.nq) return;
+    const float* rec = pc.rec + (tile * pc.np.d * NW + wave) * REC;
+    const int64_t stride = (int64_t)NW * REC;
+    float M = -INFINITY, L = 0.f;
+    floatx4 acc[4];
+#pragma unroll
+    for (int a4 = 0; a4 < 4; ++a4) acc[a4] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int p0 = 0; p0 < n; p0 += 4) {
+        float2 ml[4];
+        floatx4 v[4][4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float* r = rec + min(p0 + i, n - 1) * stride;
+            ml[i] = *(const float2*)(r + 4096 + 2 * nl);
+#pragma unroll
+            for (int a4 = 0; a4 < 4; ++a4) v[i][a4] = *(const floatx4*)(r + (4 * db + a4) * 256 + 4 * lane);
+        }
+        float mn = M;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (p0 + i >= n) ml[i] = float2{-INFINITY, 0.f};
+            mn = fmaxf(mn, ml[i].x);
+        }
+        const float ms = mn == -INFINITY ? 0.f : mn;
+        const float al = exp2_fast(M - ms);
+        L *= al;
+#pragma unroll
+        for (int a4 = 0; a4 < 4; ++a4) acc[a4] *= al;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float w = exp2_fast(ml[i].x - ms);
+            L = fmaf(w, ml[i].y, L);
+            if (p0 + i < n) {
+#pragma unroll
+                for (int a4 = 0; a4 < 4; ++a4)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[a4][e] = fmaf(w, v[i][a4][e], acc[a4][e]);
+            }
+        }
+        M = mn;
+    }
+    if (qrow < a.nq) {
+        const float inv = (L == 0.f) ? 0.f : 1.0f / L;
+        float* out = a.dst + (((int64_t)b * a.nq + qrow) * a.hq + h) * D + 32 * db + 4 * hh;
+#pragma unroll
+        for (int a4 = 0; a4 < 4; ++a4) *(floatx4*)(out + 8 * a4) = acc[a4] * inv;
+    }
+}
+
+// Blocks per piece and pieces per tile. `len(t)` is the block count of tile t.
+// (Any mask is taken for a causal one that ends at n_kv, as voxtral's are;
+// another only balances worse. An implicit mask and the tensor that it stands
+// for so get the same pieces, and the same bits.) Time in units of a block (~0.75 us):
+// a workgroup costs its blocks plus kWg, and 256 run at once; merging costs
+// a launch and the records' traffic.
+static void choose_pieces(const AttnArgs& a, int bm, int nqt, int64_t groups, size_t ws_bytes, uint32_t& lp,
+                          uint32_t& np) {
+    constexpr double kWg = 4.0, kLaunch = 4.0, kRecord = 0.05;
+    const int nblk = (a.nkv + p128::BK - 1) / p128::BK;
+    auto len = [&](int t) -> int {
+        int64_t hi = a.nkv;
+        if ((a.mask || a.im_causal) && a.nkv >= a.nq) {
+            const int64_t q1 = (int64_t)(t + 1) * bm < a.nq ? (int64_t)(t + 1) * bm : a.nq;
+            hi = q1 + (a.nkv - a.nq);
+        }
+        return (int)((hi + p128::BK - 1) / p128::BK);
+    };
+    lp = (uint32_t)nblk;
+    np = 1;
+    if (groups * nqt >= 1024) return;
+    int longest = 1;
+    for (int t = 0; t < nqt; ++t) { const int n = len(t); longest = n > longest ? n : longest; }
+    double best = 1e30;
+    static const int cand[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32, 48, 64};
+    for (int P : cand) {
+        if (P > 1 && longest < 2 * P) break;
+        const int l = ((longest + P - 1) / P + 1) & ~1;
+        // pieces per tile: the kernel's own count for the longest possible tile
+        const int pn = P == 1 ? 1 : (nblk + l - 1) / l;
+        const size_t need = (size_t)groups * nqt * (sizeof(int) + (size_t)pn * p128::NW * p128::REC * sizeof(float)) + 256;
+        if (P > 1 && need > ws_bytes) break;
+        int64_t total = 0, count = 0, recs = 0;
+        for (int t = 0; t < nqt; ++t) {
+            const int n = len(t), k = n > l ? (n + l - 1) / l : 1;
+            total += n;
+            count += k;
+            if (k > 1) recs += k;
+        }
+        total *= groups;
+        count *= groups;
+        recs *= groups;
+        const double rounds = (double)((count + 255) / 256);
+        const double mean = (double)total / (double)count;
+        double cost = rounds * (mean + kWg);
+        if (cost < l + kWg) cost = l + kWg;
+        if (recs) cost += kLaunch + kRecord * (double)recs;
+        if (cost < best) {
+            best = cost;
+            lp = (uint32_t)(P == 1 ? nblk : l);
+            np = (uint32_t)pn;
+        }
+    }
+}
+
+template <int MM>
+static void launch_p128_mm(const AttnArgs& a, const GridMap& gm, const Pieces& pc, bool cl, unsigned nwg,
+                           hipStream_t st) {
+    const dim3 grid(nwg), block(p128::NT);
+    if (a.q_f16) {
+        if (cl) hipLaunchKernelGGL((fa_prefill128<true, true, MM>), grid, block, 0, st, a, gm, pc);
+        else hipLaunchKernelGGL((fa_prefill128<true, false, MM>), grid, block, 0, st, a, gm, pc);
+    } else {
+        if (cl) hipLaunchKernelGGL((fa_prefill128<false, true, MM>), grid, block, 0, st, a, gm, pc);
+        else hipLaunchKernelGGL((fa_prefill128<false, false, MM>), grid, block, 0, st, a, gm, pc);
+    }
+}
+
+hipError_t launch_prefill128(const AttnArgs& a, hipStream_t st) {
+    if (a.mask && !a.mask_rows) return hipErrorInvalidValue;
+    if (!prefill128_takes(a) || a.nkv <= 0) return hipErrorInvalidValue;
+    Pieces pc;
+    pc.hpw_log2 = prefill128_heads_log2(a);
+    const int hpw = 1 << pc.hpw_log2, bm = 32 * (p128::NW >> pc.hpw_log2);
+    const int nqt = (a.nq + bm - 1) / bm, nhg = a.hq / hpw;
+    const int64_t groups = (int64_t)nhg * a.b;
+    uint32_t np = 1;
+    choose_pieces(a, bm, nqt, groups, a.ws ? a.ws_bytes : 0, pc.lp, np);
+    pc.np = DivMod::make(np);
+    pc.nqt = nqt;
+    pc.nhg = nhg;
+    pc.count = reinterpret_cast<int*>(a.ws);
+    pc.rec = a.ws + (((size_t)groups * nqt + 63) & ~(size_t)63);
+    const int64_t nwg = groups * nqt * np;
+    if (nwg <= 0 || nwg > 0x7fffffff) return hipErrorInvalidValue;
+    const bool masked = a.mask || a.im_causal;
+    const GridMap gm = masked ? GridMap::make_tiles_desc((int)nwg, nqt * (int)np, nhg, a.hkv, a.b, a.bk)
+                              : GridMap::make((int)nwg, nqt * (int)np, nhg, a.hkv, a.b, a.bk);
+    const bool cl = fabsf(a.scale_log2) == p128::kC128;
+    if (a.mask) launch_p128_mm<1>(a, gm, pc, cl, (unsigned)nwg, st);
+    else if (a.im_causal) launch_p128_mm<2>(a, gm, pc, cl, (unsigned)nwg, st);
+    else launch_p128_mm<0>(a, gm, pc, cl, (unsigned)nwg, st);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || np == 1) return e;
+    hipLaunchKernelGGL(fa_prefill128_combine, dim3((unsigned)(groups * nqt * p128::NW)), dim3(256), 0, st, a, pc);
+    return hipGetLastError();
+}
+
+}  // namespace vxfa

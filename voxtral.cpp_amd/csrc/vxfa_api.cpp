@@ -54,10 +54,11 @@ struct Tuning {
 // message: a context's workspace, or the library's static scratch array.
 struct Workspace {
     int device;
-    float* rec;           // split-KV partial records
-    size_t rec_bytes;
-    _Float16* stage;      // f16 staging of F32 K/V (prefill)
-    size_t stage_bytes;
+    char* base;           // one area, 256-byte aligned: a decode call's split-KV
+    size_t bytes;         // records, or a prefill call's staged K/V, mask row
+                          // intervals and piece records, in that order
+    size_t rec_bytes;     // of it, most that decode records take
+    size_t stage_bytes;   // of it, most that staged F32 K/V take
     char* err;            // message of the last failure
     size_t err_len;
     Tuning tune;
@@ -65,13 +66,12 @@ struct Workspace {
 
 struct vxfa_ctx {
     int device = 0;
-    char* ws = nullptr;           // one device allocation holding both regions
-    float* rec = nullptr;         // kRecordBytes of partial records
-    _Float16* stage = nullptr;    // kStageBytes of f16 K/V staging
+    char* ws = nullptr;           // kRecordBytes + kStageBytes of device memory
     char last_error[256] = {0};
     Tuning tune;                  // read once when the context is created
     Workspace view() {
-        return Workspace{device, rec, kRecordBytes, stage, kStageBytes, last_error, sizeof(last_error), tune};
+        return Workspace{device, ws, kRecordBytes + kStageBytes, kRecordBytes, kStageBytes, last_error,
+                         sizeof(last_error), tune};
     }
 };
 
@@ -303,8 +303,6 @@ vxfa_ctx* vxfa_ctx_create(int device) {
         delete c;
         return nullptr;
     }
-    c->rec = reinterpret_cast<float*>(c->ws);
-    c->stage = reinterpret_cast<_Float16*>(c->ws + kRecordBytes);
     return c;
 }
 
@@ -506,7 +504,7 @@ int run(Workspace& w, const vxfa_tensor* q, const vxfa_tensor* k, const vxfa_ten
         S = fit_split(S, B * Hkv, vxfa::dec_record_floats((int)D, (int)G), w.rec_bytes);
         a.n_split = S;
         a.dec_t16 = t16 ? 1 : 0;
-        a.ws = w.rec;
+        a.ws = reinterpret_cast<float*>(w.base);
         e = vxfa::launch_decode(a, (int)D, (int)G, st);
     } else {
         size_t staged = 0;   // bytes of the staging area this call fills
@@ -524,8 +522,8 @@ int run(Workspace& w, const vxfa_tensor* q, const vxfa_tensor* k, const vxfa_ten
                         (long long)(2 * per * (int64_t)sizeof(_Float16)), w.stage_bytes);
                 return VXFA_NO_WORKSPACE;
             }
-            _Float16* sk = w.stage;
-            _Float16* sv = w.stage + per;
+            _Float16* sk = reinterpret_cast<_Float16*>(w.base);
+            _Float16* sv = sk + per;
             stage = vxfa::StageReq{static_cast<const float*>(k->data), (int64_t)k->nb[1], (int64_t)k->nb[2],
                                    (int64_t)k->nb[3], static_cast<const float*>(v->data), (int64_t)v->nb[1],
                                    (int64_t)v->nb[2], (int64_t)v->nb[3], (int)D, (int)Nkv, (int)Hkv, (int)Bk, sk,
@@ -538,16 +536,18 @@ int run(Workspace& w, const vxfa_tensor* q, const vxfa_tensor* k, const vxfa_ten
             a.k_nb3 = a.v_nb3 = Nkv * Hkv * D * 2;
             a.kv_f32 = 0;
         }
-        // a mask tensor with a pre-pass (the pipelined hd 64 kernel; the short
-        // masked prefill when F32 K/V are staged): the live interval of each
-        // mask row (8 bytes a row) in the records region, unused by a prefill
-        // call; where records and staging share one area (the no-alloc
-        // scratch), after the staged K/V
+        size_t used = (staged + 255) & ~(size_t)255;
+        bool stage_done = false;
+        // a mask tensor with a pre-pass (the pipelined hd 64 kernel, the grouped
+        // hd 128 one, the short masked prefill when F32 K/V are staged): the
+        // live interval of each mask row (8 bytes a row), after the staged K/V
         int2* mrows = nullptr;
         if (mask) {
-            const size_t off = w.rec == reinterpret_cast<float*>(w.stage) ? (staged + 255) & ~(size_t)255 : 0;
-            const size_t need = (size_t)(Nq * a.hm * a.bm) * sizeof(int2);
-            if (off + need <= w.rec_bytes) mrows = reinterpret_cast<int2*>(reinterpret_cast<char*>(w.rec) + off);
+            const size_t need = ((size_t)(Nq * a.hm * a.bm) * sizeof(int2) + 255) & ~(size_t)255;
+            if (used + need <= w.bytes) {
+                mrows = reinterpret_cast<int2*>(w.base + used);
+                used += need;
+            }
         }
         const bool pp_mask_fits = mrows != nullptr;
         if (D == 64 && (!mask || pp_mask_fits) && !rope && scale != 0.0f && w.tune.pp_enabled) {
@@ -562,16 +562,20 @@ int run(Workspace& w, const vxfa_tensor* q, const vxfa_tensor* k, const vxfa_ten
         } else {
             const bool pair = D == 128 && (mask || implicit) && Nkv <= 512 && w.tune.pair_enabled &&
                               vxfa::prefill_pair_fits(a);
-            if (pair && staged && mask && mrows && w.tune.pair_intervals) {
-                // the decoder prefill as voxtral calls it (F32 cache, F16 mask):
-                // the staging launch also finds the mask rows' intervals, from
-                // which the short masked prefill takes its block classes
+            // hd 128 beyond the short masked prefill: the kernel whose workgroups
+            // share K/V blocks among the heads of a kv group (a mask tensor
+            // needs its intervals table)
+            const bool grouped = D == 128 && !pair && (!mask || mrows) && vxfa::prefill128_takes(a);
+            if (mask && mrows && ((pair && staged && w.tune.pair_intervals) || grouped)) {
+                // the mask rows' intervals, in one launch with the staging:
+                // for the decoder prefill as voxtral calls it (F32 cache, F16
+                // mask), and for the grouped kernel
                 a.mask_rows = mrows;
-                e = vxfa::launch_mask_prep(a, &stage, st);
-                if (e != hipSuccess) { set_err(w, "F32 K/V staging: %s", hipGetErrorString(e)); return VXFA_HIP_ERROR; }
-                staged = 0;   // (done in that launch)
+                e = vxfa::launch_mask_prep(a, staged ? &stage : nullptr, st);
+                if (e != hipSuccess) { set_err(w, "mask pre-pass: %s", hipGetErrorString(e)); return VXFA_HIP_ERROR; }
+                if (staged) stage_done = true;
             }
-            if (staged) {
+            if (staged && !stage_done) {
                 e = vxfa::launch_to_f16_kv(stage, st);
                 if (e != hipSuccess) { set_err(w, "F32 K/V staging: %s", hipGetErrorString(e)); return VXFA_HIP_ERROR; }
             }
@@ -580,6 +584,8 @@ int run(Workspace& w, const vxfa_tensor* q, const vxfa_tensor* k, const vxfa_ten
                 // tiles, every live block on its own wavefront
                 e = vxfa::launch_prefill_pair(a, st);
             } else {
+                a.ws = reinterpret_cast<float*>(w.base + used);
+                a.ws_bytes = w.bytes - used;
                 // query-row wavefronts per workgroup (each with its KV partner
                 // wavefronts): 4 shares every staged K/V step among 128 query rows;
                 // hd 128 and small grids (fewer than 128 workgroups of 128 rows) use 2
@@ -729,10 +735,8 @@ int vxfa_flash_attn_ext_noalloc(const vxfa_tensor* q, const vxfa_tensor* k, cons
         t.read_env();
         return t;
     }();
-    // records (decode) and staging (prefill with F32 K/V) are never needed
-    // by one call together: both use the whole array
-    Workspace w{device, static_cast<float*>(ptr), kScratchBytes, static_cast<_Float16*>(ptr), kScratchBytes,
-                t_noalloc_err, sizeof(t_noalloc_err), tune};
+    Workspace w{device, static_cast<char*>(ptr), kScratchBytes, kScratchBytes, kScratchBytes, t_noalloc_err,
+                sizeof(t_noalloc_err), tune};
     return run(w, q, k, v, mask, nullptr, dst, scale, max_bias, logit_softcap, stream);
 }
 
