@@ -70,6 +70,7 @@ struct AttnArgs {
     // on [lo, hi] and -inf elsewhere ({n_kv, -1}: no live entry), else
     // {-2, -2}; written by a pre-pass launch into workspace scratch
     int2* mask_rows;
+    int32_t mask_rows_ready;   // host: mask_rows has been filled by an earlier launch of this call
     size_t ws_bytes;      // prefill: bytes at ws
 };
 
@@ -265,6 +266,18 @@ struct AppendArgs {
     const int32_t* rope_pos;
     float rope_ts;
     int32_t rope_dims;
+    // the rest of a prefill call's preparation, in the same launch (null: none):
+    // F32 query rows (hq heads, token t of batch b one of the n_new new rows)
+    // rotated like K and rounded to f16, to q_out [b][t][hq][d]
+    const float* q;
+    int64_t q_nb1, q_nb2, q_nb3;
+    _Float16* q_out;
+    int32_t hq;
+    // and the live intervals of a mask tensor's rows (fa_mask_rows.h)
+    const uint16_t* mask;
+    int64_t m_nb1, m_nb2, m_nb3;
+    int32_t m_n, m_nq, m_hm, m_rows;
+    int2* m_out;
 };
 
 // Rotary embedding as ggml_rope_ext computes it for mode 0 with

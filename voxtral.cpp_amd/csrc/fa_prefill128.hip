@@ -92,10 +92,13 @@ __device__ __forceinline__ int wave_max32(int x) {
 
 // MM: 0 no mask, 1 a mask tensor (intervals in a.mask_rows), 2 implicit.
 // CL: the scale is exactly 1/sqrt(128) (c is a literal, see exps below).
-template <bool QF16, bool CL, int MM>
+// QT: 0 F32 rows, 1 f16 rows, 2 F32 rows to rotate (a call whose rotated rows
+// do not fit the scratch; 14 KB of code that the others do not fetch).
+template <int QT, bool CL, int MM>
 __global__ __launch_bounds__(p128::NT) void fa_prefill128(AttnArgs a, GridMap gm, Pieces pc) {
     using namespace p128;
-    __shared__ __attribute__((aligned(16))) char smem[NS * 2 * STEP];   // K steps, then V steps
+    // K steps, V steps, and half of the Q staging (160 KiB: all of a CU's LDS)
+    __shared__ __attribute__((aligned(16))) char smem[NS * 2 * STEP + (QT == 2 ? 0 : 4 * BLK)];
 
     int idx, hg, b, hk, bkv;
     gm.locate(blockIdx.x, idx, hg, b, hk, bkv);
@@ -114,6 +117,7 @@ __global__ __launch_bounds__(p128::NT) void fa_prefill128(AttnArgs a, GridMap gm
     const int r0 = q0 + 32 * (wave >> pc.hpw_log2);       // the wavefront's first row
     const int qrow = r0 + nl;
     const bool qvalid = qrow < a.nq;
+    const bool active = r0 < a.nq;                        // the wavefront has rows
     const int qld = min(qrow, a.nq - 1);
     const char* kb = (const char*)a.k + (int64_t)hk * a.k_nb2 + (int64_t)bkv * a.k_nb3;
     const char* vb = (const char*)a.v + (int64_t)hk * a.v_nb2 + (int64_t)bkv * a.v_nb3;
@@ -176,27 +180,29 @@ __global__ __launch_bounds__(p128::NT) void fa_prefill128(AttnArgs a, GridMap gm
         if (piece == 0 && tid == 0) pc.count[((int64_t)b * pc.nhg + hg) * pc.nqt + qt] = n;
     }
 
-    // ---- Q operand: row qrow, dims 16 ks + 8 hh .. + 7 ------------------------
-    half8 qb[KS];
-    floatx4 qraw[QF16 ? 1 : KS][2];
+    // ---- Q loads -----------------------------------------------------------------
+    // Whole rows of the wavefront's 32 (rows past n_q read the last one), turned
+    // into the operand layout through LDS below: a load of the operand layout
+    // touches 32 rows per instruction, and its 16 instructions of 8 wavefronts
+    // kept the CU's address unit busy for ~2 us. QT 2 (rotation) needs a row's
+    // pairs together and loads the operand layout.
+    constexpr int QL = QT == 2 ? 2 * KS : (QT == 1 ? KS : 2 * KS);   // 16-byte loads per lane
+    constexpr int QCH = QT == 1 ? 16 : 32;                            // 16-byte chunks per row
+    floatx4 qraw[QL];
     int qpos = 0;
     {
-        const char* qp = (const char*)a.q + (int64_t)qld * a.q_nb1 + (int64_t)h * a.q_nb2 + (int64_t)b * a.q_nb3;
+        const char* qp = (const char*)a.q + (int64_t)h * a.q_nb2 + (int64_t)b * a.q_nb3;
+        if constexpr (QT == 2) {
+            const char* p = qp + (int64_t)qld * a.q_nb1 + 32 * hh;
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            if constexpr (QF16) {
-                qb[ks] = *(const half8*)(qp + (16 * ks + 8 * hh) * 2);
-            } else {
-                const floatx4* p = (const floatx4*)(qp + (16 * ks + 8 * hh) * 4);
-                qraw[ks][0] = p[0];
-                qraw[ks][1] = p[1];
+            for (int u = 0; u < QL; ++u) qraw[u] = *(const floatx4*)(p + 64 * (u >> 1) + 16 * (u & 1));
+            qpos = a.rope_pos[(int64_t)b * a.nq + qld];
+        } else {
+#pragma unroll
+            for (int u = 0; u < QL; ++u) {
+                const int row = min(r0 + (64 / QCH) * u + lane / QCH, a.nq - 1);
+                qraw[u] = __builtin_nontemporal_load((const floatx4*)(qp + (int64_t)row * a.q_nb1) + lane % QCH);
             }
-        }
-        if constexpr (!QF16) {
-            // (without a rotary embedding the first word of Q, unused: a
-            // branch would make the compiler wait for the loads before it)
-            const int* pp = a.rope_pos ? a.rope_pos + ((int64_t)b * a.nq + qld) : (const int*)a.q;
-            qpos = *pp;
         }
     }
 
@@ -244,35 +250,56 @@ __global__ __launch_bounds__(p128::NT) void fa_prefill128(AttnArgs a, GridMap gm
             }
         }
     };
-    for (int u = 0; u < min(nstep, NS - 1); ++u) issue(u);
+    for (int u = 0; u < min(nstep, 2); ++u) issue(u);
 
-    // ---- Q: rotate, fold the sign of the scale in (0 for scale 0), round ------
+    // ---- Q operand: row qrow, dims 16 ks + 8 hh .. + 7, rounded to f16; the sign
+    // of the scale folded in (0 for scale 0) -----------------------------------------
     const float c = a.scale_log2 != 0.f ? fabsf(a.scale_log2) : 1.0f;
+    half8 qb[KS];
     {
         const float sg = a.scale_log2 < 0.f ? -1.0f : (a.scale_log2 > 0.f ? 1.0f : 0.0f);
-        if constexpr (QF16) {
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) qb[ks] = qb[ks] * (_Float16)sg;
-        } else {
+        if constexpr (QT == 2) {
             // one running product over the row's pairs, as ggml builds its
             // cos / sin cache: pair 8 ks + o belongs to the lanes of half o / 4
             float th = (float)qpos;
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) {
-                float x[8] = {qraw[ks][0][0], qraw[ks][0][1], qraw[ks][0][2], qraw[ks][0][3],
-                              qraw[ks][1][0], qraw[ks][1][1], qraw[ks][1][2], qraw[ks][1][3]};
-                if (a.rope_pos) {
-                    float ang[4] = {0.f, 0.f, 0.f, 0.f};
+                float x[8];
 #pragma unroll
-                    for (int o = 0; o < 8; ++o) {
-                        if (ks > 0 || o > 0) th *= a.rope_ts;
-                        if ((o >> 2) == hh) ang[o & 3] = th;
-                    }
-                    rope8_ang(x, ang, 16 * ks + 8 * hh, a.rope_dims);
+                for (int e = 0; e < 8; ++e) x[e] = qraw[2 * ks + (e >> 2)][e & 3];
+                float ang[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int o = 0; o < 8; ++o) {
+                    if (ks > 0 || o > 0) th *= a.rope_ts;
+                    if ((o >> 2) == hh) ang[o & 3] = th;
                 }
+                rope8_ang(x, ang, 16 * ks + 8 * hh, a.rope_dims);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) qb[ks][e] = (_Float16)(x[e] * sg);
             }
+        } else {
+            // the wavefront's 8 KiB: row r at 256 r, 16-byte chunk j at j ^ (r & 15);
+            // wavefronts 0-3 in ring slot 3 (filled from iteration 0 on), 4-7 past
+            // the ring
+            char* qs = smem + (wave < 2 ? 3 * STEP + wave * BLK
+                                        : (wave < 4 ? (NS + 3) * STEP + (wave - 2) * BLK
+                                                    : 2 * NS * STEP + (wave - 4) * BLK));
+#pragma unroll
+            for (int u = 0; u < QL; ++u) {
+                const int r = (64 / QCH) * u + lane / QCH, j = lane % QCH;
+                if constexpr (QT == 1) {
+                    *(half8*)(qs + r * ROW + ((j ^ (r & 15)) * 16)) = __builtin_bit_cast(half8, qraw[u]) * (_Float16)sg;
+                } else {
+                    half4 y;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) y[e] = (_Float16)(qraw[u][e] * sg);
+                    *(half4*)(qs + r * ROW + (((j >> 1) ^ (r & 15)) * 16) + (j & 1) * 8) = y;
+                }
+            }
+            __builtin_amdgcn_wave_barrier();   // (one wavefront's LDS accesses run in order)
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+                qb[ks] = *(const half8*)(qs + nl * ROW + (((2 * ks + hh) ^ (nl & 15)) * 16));
         }
     }
 
@@ -405,13 +432,13 @@ __global__ __launch_bounds__(p128::NT) void fa_prefill128(AttnArgs a, GridMap gm
         l += ls;
     };
 
-    // before iteration 0: step 0 and the first half of step 1 (K), step 0 (V)
-    // (loads in flight may stay: all but step 0's and step 1's K)
-    {
-        const int npre = min(nstep, NS - 1);
-        if (npre >= 3) wait_vm<6>();
-        else if (npre == 2) wait_vm<2>();
-        else wait_vm<0>();
+    // before iteration 0: steps 0 and 1 (step 2's loads, issued after the wait
+    // for Q, may stay in flight)
+    if (nstep > 2) {
+        issue(2);
+        wait_vm<4>();
+    } else {
+        wait_vm<0>();
     }
     __syncthreads();
 
@@ -426,7 +453,7 @@ __global__ __launch_bounds__(p128::NT) void fa_prefill128(AttnArgs a, GridMap gm
             const float inv_c = kLog2e / c;
             for (int u = 0; u < nstep; ++u) {
                 if (u + NS - 1 < nstep) issue(u + NS - 1);
-                for (int t = 2 * u; t < min(2 * u + 2, nb); ++t) {
+                for (int t = 2 * u; active && t < min(2 * u + 2, nb); ++t) {
                     const int kv0 = (bs + t) * BK;
                     uint16_t mv[16];
                     if (a.mask_vec && kv0 + BK <= a.nkv) {
@@ -491,8 +518,10 @@ __global__ __launch_bounds__(p128::NT) void fa_prefill128(AttnArgs a, GridMap gm
             // half's S is not used)
             for (int u = 0; u < nstep; ++u) {
                 if (u + NS - 1 < nstep) issue(u + NS - 1);
-                half(2 * u, sa, sb, pa, pb);
-                half(2 * u + 1, sb, sa, pb, pa);
+                if (active) {
+                    half(2 * u, sa, sb, pa, pb);
+                    half(2 * u + 1, sb, sa, pb, pa);
+                }
                 // K of step u + 2 and V of step u + 1 have landed: at most the
                 // loads of step u + 3 and V of step u + 2 are in flight
                 if (u + 3 < nstep) wait_vm<6>();
@@ -524,7 +553,7 @@ __global__ __launch_bounds__(p128::NT) void fa_prefill128(AttnArgs a, GridMap gm
                         floatx4{o[db][4 * a4] * inv, o[db][4 * a4 + 1] * inv, o[db][4 * a4 + 2] * inv,
                                 o[db][4 * a4 + 3] * inv};
         }
-    } else {
+    } else if (active) {
         const int64_t ri = ((((int64_t)b * pc.nhg + hg) * pc.nqt + qt) * pc.np.d + piece) * NW + wave;
         float* rec = pc.rec + ri * REC;
 #pragma unroll
@@ -537,42 +566,50 @@ __global__ __launch_bounds__(p128::NT) void fa_prefill128(AttnArgs a, GridMap gm
     }
 }
 
-// Merge of the pieces of a tile: workgroup = one wavefront tile (32 rows of a
-// head), wavefront = 32 output dims; lane layout as in the records.
+// Merge of the pieces of a tile; lane layout as in the records. A wavefront
+// takes 32 output dims of one wavefront tile (32 rows of a head) and every
+// SP-th piece, with UP records' loads in flight; the SP wavefronts of a
+// workgroup then merge through LDS (SP = 1: a workgroup is the four dim
+// groups of a wavefront tile).
+template <int SP, int UP>
 __global__ __launch_bounds__(256) void fa_prefill128_combine(AttnArgs a, Pieces pc) {
     using namespace p128;
-    const int lane = threadIdx.x & 63, db = threadIdx.x >> 6;
+    static_assert(SP == 1 || SP == 4, "wavefronts per tile and dims");
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nl = lane & 31, hh = lane >> 5;
-    const int64_t tile = blockIdx.x / NW;                 // (b nhg + hg) nqt + qt
-    const int wave = blockIdx.x % NW;
+    const uint32_t wt = SP == 1 ? blockIdx.x : blockIdx.x / DB;         // wavefront tile
+    const int db = SP == 1 ? w : (int)(blockIdx.x % DB);
+    const int sp = SP == 1 ? 0 : w;
+    const int64_t tile = wt / NW;                         // (b nhg + hg) nqt + qt
+    const int wave = wt % NW;
     const int n = pc.count[tile];
-    if (n <= 1) return;
     const int qt = (int)(tile % pc.nqt);
     const int hg = (int)(tile / pc.nqt % pc.nhg), b = (int)(tile / pc.nqt / pc.nhg);
     const int hpw = 1 << pc.hpw_log2;
     const int h = hg * hpw + (wave & (hpw - 1));
     const int qrow = qt * 32 * (NW >> pc.hpw_log2) + 32 * (wave >> pc.hpw_log2) + nl;
-    if (qrow - nl >= a.nq) return;
+    if (n <= 1 || qrow - nl >= a.nq) return;
     const float* rec = pc.rec + (tile * pc.np.d * NW + wave) * REC;
     const int64_t stride = (int64_t)NW * REC;
     float M = -INFINITY, L = 0.f;
     floatx4 acc[4];
 #pragma unroll
     for (int a4 = 0; a4 < 4; ++a4) acc[a4] = floatx4{0.f, 0.f, 0.f, 0.f};
-    for (int p0 = 0; p0 < n; p0 += 4) {
-        float2 ml[4];
-        floatx4 v[4][4];
+    for (int p0 = sp; p0 < n; p0 += SP * UP) {
+        float2 ml[UP];
+        floatx4 v[UP][4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float* r = rec + min(p0 + i, n - 1) * stride;
+        for (int i = 0; i < UP; ++i) {
+            const float* r = rec + min(p0 + SP * i, n - 1) * stride;
             ml[i] = *(const float2*)(r + 4096 + 2 * nl);
 #pragma unroll
             for (int a4 = 0; a4 < 4; ++a4) v[i][a4] = *(const floatx4*)(r + (4 * db + a4) * 256 + 4 * lane);
         }
         float mn = M;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            if (p0 + i >= n) ml[i] = float2{-INFINITY, 0.f};
+        for (int i = 0; i < UP; ++i) {
+            if (p0 + SP * i >= n) ml[i] = float2{-INFINITY, 0.f};
             mn = fmaxf(mn, ml[i].x);
         }
         const float ms = mn == -INFINITY ? 0.f : mn;
@@ -581,19 +618,45 @@ __global__ __launch_bounds__(256) void fa_prefill128_combine(AttnArgs a, Pieces 
 #pragma unroll
         for (int a4 = 0; a4 < 4; ++a4) acc[a4] *= al;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float w = exp2_fast(ml[i].x - ms);
-            L = fmaf(w, ml[i].y, L);
-            if (p0 + i < n) {
+        for (int i = 0; i < UP; ++i) {
+            const float wt_ = exp2_fast(ml[i].x - ms);
+            L = fmaf(wt_, ml[i].y, L);
+            if (p0 + SP * i < n) {
 #pragma unroll
                 for (int a4 = 0; a4 < 4; ++a4)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) acc[a4][e] = fmaf(w, v[i][a4][e], acc[a4][e]);
+                    for (int e = 0; e < 4; ++e) acc[a4][e] = fmaf(wt_, v[i][a4][e], acc[a4][e]);
             }
         }
         M = mn;
     }
-    if (qrow < a.nq) {
+    if constexpr (SP > 1) {
+        __shared__ floatx4 xo[SP][4][64];
+        __shared__ float2 xm[SP][64];
+#pragma unroll
+        for (int a4 = 0; a4 < 4; ++a4) xo[sp][a4][lane] = acc[a4];
+        xm[sp][lane] = float2{M, L};
+        __syncthreads();
+        // wavefront w merges quarter w of the 16 dims a lane holds
+        float mm = -INFINITY;
+#pragma unroll
+        for (int s = 0; s < SP; ++s) mm = fmaxf(mm, xm[s][lane].x);
+        const float ms = mm == -INFINITY ? 0.f : mm;
+        L = 0.f;
+        floatx4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < SP; ++s) {
+            const float f = exp2_fast(xm[s][lane].x - ms);
+            L = fmaf(f, xm[s][lane].y, L);
+            const floatx4 x = xo[s][w][lane];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = fmaf(f, x[e], o[e]);
+        }
+        if (qrow < a.nq) {
+            const float inv = (L == 0.f) ? 0.f : 1.0f / L;
+            *(floatx4*)(a.dst + (((int64_t)b * a.nq + qrow) * a.hq + h) * D + 32 * db + 8 * w + 4 * hh) = o * inv;
+        }
+    } else if (qrow < a.nq) {
         const float inv = (L == 0.f) ? 0.f : 1.0f / L;
         float* out = a.dst + (((int64_t)b * a.nq + qrow) * a.hq + h) * D + 32 * db + 4 * hh;
 #pragma unroll
@@ -656,17 +719,12 @@ static void choose_pieces(const AttnArgs& a, int bm, int nqt, int64_t groups, si
     }
 }
 
-template <int MM>
-static void launch_p128_mm(const AttnArgs& a, const GridMap& gm, const Pieces& pc, bool cl, unsigned nwg,
-                           hipStream_t st) {
+template <int QT, bool CL>
+static void launch_p128(const AttnArgs& a, const GridMap& gm, const Pieces& pc, unsigned nwg, hipStream_t st) {
     const dim3 grid(nwg), block(p128::NT);
-    if (a.q_f16) {
-        if (cl) hipLaunchKernelGGL((fa_prefill128<true, true, MM>), grid, block, 0, st, a, gm, pc);
-        else hipLaunchKernelGGL((fa_prefill128<true, false, MM>), grid, block, 0, st, a, gm, pc);
-    } else {
-        if (cl) hipLaunchKernelGGL((fa_prefill128<false, true, MM>), grid, block, 0, st, a, gm, pc);
-        else hipLaunchKernelGGL((fa_prefill128<false, false, MM>), grid, block, 0, st, a, gm, pc);
-    }
+    if (a.mask) hipLaunchKernelGGL((fa_prefill128<QT, CL, 1>), grid, block, 0, st, a, gm, pc);
+    else if (a.im_causal) hipLaunchKernelGGL((fa_prefill128<QT, CL, 2>), grid, block, 0, st, a, gm, pc);
+    else hipLaunchKernelGGL((fa_prefill128<QT, CL, 0>), grid, block, 0, st, a, gm, pc);
 }
 
 hipError_t launch_prefill128(const AttnArgs& a, hipStream_t st) {
@@ -690,12 +748,21 @@ hipError_t launch_prefill128(const AttnArgs& a, hipStream_t st) {
     const GridMap gm = masked ? GridMap::make_tiles_desc((int)nwg, nqt * (int)np, nhg, a.hkv, a.b, a.bk)
                               : GridMap::make((int)nwg, nqt * (int)np, nhg, a.hkv, a.b, a.bk);
     const bool cl = fabsf(a.scale_log2) == p128::kC128;
-    if (a.mask) launch_p128_mm<1>(a, gm, pc, cl, (unsigned)nwg, st);
-    else if (a.im_causal) launch_p128_mm<2>(a, gm, pc, cl, (unsigned)nwg, st);
-    else launch_p128_mm<0>(a, gm, pc, cl, (unsigned)nwg, st);
+    if (a.q_f16) {
+        if (cl) launch_p128<1, true>(a, gm, pc, (unsigned)nwg, st);
+        else launch_p128<1, false>(a, gm, pc, (unsigned)nwg, st);
+    } else if (a.rope_pos) {
+        if (cl) launch_p128<2, true>(a, gm, pc, (unsigned)nwg, st);
+        else launch_p128<2, false>(a, gm, pc, (unsigned)nwg, st);
+    } else {
+        if (cl) launch_p128<0, true>(a, gm, pc, (unsigned)nwg, st);
+        else launch_p128<0, false>(a, gm, pc, (unsigned)nwg, st);
+    }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || np == 1) return e;
-    hipLaunchKernelGGL(fa_prefill128_combine, dim3((unsigned)(groups * nqt * p128::NW)), dim3(256), 0, st, a, pc);
+    const unsigned nwt = (unsigned)(groups * nqt * p128::NW);
+    if (np <= 4) hipLaunchKernelGGL((fa_prefill128_combine<1, 4>), dim3(nwt), dim3(256), 0, st, a, pc);
+    else hipLaunchKernelGGL((fa_prefill128_combine<4, 4>), dim3(nwt * p128::DB), dim3(256), 0, st, a, pc);
     return hipGetLastError();
 }
 

@@ -410,13 +410,21 @@ int run(Workspace& w, const vxfa_tensor* q, const vxfa_tensor* k, const vxfa_ten
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     // rotary embedding: ggml's theta scale, computed as ggml_rope_ext's CPU path does
     const float rope_ts = rope ? powf(rope->freq_base, -2.0f / (float)rope->n_dims) : 0.0f;
-    if (append && !fuse_append) {
-        vxfa::AppendArgs ap = append_args(k, v, k_new, v_new);
+    // the append launch of a call that does not fuse it: before a decode call
+    // or an early end; a prefill call adds to it first (below)
+    const bool separate = append && !fuse_append;
+    vxfa::AppendArgs ap;
+    if (separate) {
+        ap = append_args(k, v, k_new, v_new);
         if (rope) {
             ap.rope_pos = rope->positions;
             ap.rope_ts = rope_ts;
             ap.rope_dims = rope->n_dims;
         }
+    }
+    const bool decode = Nq == 1 && (Gq == 1 || Gq == 2 || Gq == 4);
+    const bool empty = Nq * Hq * B == 0 || Nkv == 0;
+    if (separate && (decode || empty)) {
         e = vxfa::launch_kv_append(ap, st);
         if (e != hipSuccess) { set_err(w, "kv append: %s", hipGetErrorString(e)); return VXFA_HIP_ERROR; }
     }
@@ -472,8 +480,8 @@ int run(Workspace& w, const vxfa_tensor* q, const vxfa_tensor* k, const vxfa_ten
         a.im_offset = im->offset;
     }
 
-    const int64_t G = Hq / Hkv;
-    if (Nq == 1 && (G == 1 || G == 2 || G == 4)) {
+    const int64_t G = Gq;
+    if (decode) {
         if (implicit) {
             // the one query row attends [offset - W + 1, offset], clipped to [0, n_kv)
             int64_t lo = im->window > 0 ? im->offset - im->window + 1 : 0;
@@ -549,8 +557,44 @@ int run(Workspace& w, const vxfa_tensor* q, const vxfa_tensor* k, const vxfa_ten
                 used += need;
             }
         }
-        const bool pp_mask_fits = mrows != nullptr;
-        if (D == 64 && (!mask || pp_mask_fits) && !rope && scale != 0.0f && w.tune.pp_enabled) {
+        const bool pair = D == 128 && (mask || implicit) && Nkv <= 512 && w.tune.pair_enabled &&
+                          vxfa::prefill_pair_fits(a);
+        // hd 128 beyond the short masked prefill: the kernel whose workgroups
+        // share K/V blocks among the heads of a kv group (a mask tensor needs
+        // its intervals table)
+        const bool grouped = D == 128 && !pair && (!mask || mrows) && vxfa::prefill128_takes(a);
+        const bool pp = D == 64 && (!mask || mrows) && scale != 0.0f && w.tune.pp_enabled;
+        if (separate) {
+            // the append launch also rotates Q into scratch as f16 (else the
+            // attention kernel rotates it in each workgroup, and hd 64 goes to
+            // the general kernel), and finds the mask rows' intervals
+            if (rope) {
+                const size_t need = ((size_t)(B * Nq * Hq * D) * sizeof(_Float16) + 255) & ~(size_t)255;
+                if (used + need <= w.bytes && (pair || grouped || pp)) {
+                    ap.q = static_cast<const float*>(q->data);
+                    ap.q_nb1 = a.q_nb1; ap.q_nb2 = a.q_nb2; ap.q_nb3 = a.q_nb3;
+                    ap.q_out = reinterpret_cast<_Float16*>(w.base + used);
+                    ap.hq = (int32_t)Hq;
+                    used += need;
+                    a.q = ap.q_out;
+                    a.q_f16 = 1;
+                    a.q_nb1 = Hq * D * 2; a.q_nb2 = D * 2; a.q_nb3 = Nq * Hq * D * 2;
+                    a.rope_pos = nullptr;
+                }
+            }
+            const int64_t nrows = Nq * a.hm * a.bm;
+            if (mask && mrows && (grouped || pp || (pair && w.tune.pair_intervals)) && nrows < 0x7fffffff - 15) {
+                ap.mask = a.mask;
+                ap.m_nb1 = a.m_nb1; ap.m_nb2 = a.m_nb2; ap.m_nb3 = a.m_nb3;
+                ap.m_n = a.nkv; ap.m_nq = a.nq; ap.m_hm = a.hm; ap.m_rows = (int32_t)nrows;
+                ap.m_out = mrows;
+                a.mask_rows = mrows;
+                a.mask_rows_ready = 1;
+            }
+            e = vxfa::launch_kv_append(ap, st);
+            if (e != hipSuccess) { set_err(w, "kv append: %s", hipGetErrorString(e)); return VXFA_HIP_ERROR; }
+        }
+        if (pp && !a.rope_pos) {
             a.mask_rows = mrows;
             // (scale 0 goes to the general kernel: the pipelined one folds the
             // scale into the exponent and scores the partial block's dead rows -inf)
@@ -560,13 +604,7 @@ int run(Workspace& w, const vxfa_tensor* q, const vxfa_tensor* k, const vxfa_ten
             // pre-pass's launch when there is one
             e = vxfa::launch_prefill64_pp(a, staged ? &stage : nullptr, st);
         } else {
-            const bool pair = D == 128 && (mask || implicit) && Nkv <= 512 && w.tune.pair_enabled &&
-                              vxfa::prefill_pair_fits(a);
-            // hd 128 beyond the short masked prefill: the kernel whose workgroups
-            // share K/V blocks among the heads of a kv group (a mask tensor
-            // needs its intervals table)
-            const bool grouped = D == 128 && !pair && (!mask || mrows) && vxfa::prefill128_takes(a);
-            if (mask && mrows && ((pair && staged && w.tune.pair_intervals) || grouped)) {
+            if (mask && mrows && !a.mask_rows_ready && ((pair && staged && w.tune.pair_intervals) || grouped)) {
                 // the mask rows' intervals, in one launch with the staging:
                 // for the decoder prefill as voxtral calls it (F32 cache, F16
                 // mask), and for the grouped kernel
