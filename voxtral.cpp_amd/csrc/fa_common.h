@@ -37,6 +37,7 @@ struct AttnArgs {
     int32_t kv_f32;       // k and v element type is F32 (else f16)
     int32_t n_split;      // decode: workgroups per (batch, kv head)
     int32_t dec_t16;      // decode, f16 K/V: 16-position tiles (short spans) instead of 32
+    int32_t dec_chunk;    // decode with mask_rows: positions per split at most
     int32_t mask_vec;     // mask data and strides 16-byte aligned (128-bit mask loads)
     float scale_log2;     // scale * log2(e)
     // implicit causal / window mask (instead of a mask tensor): query row i
@@ -68,7 +69,8 @@ struct AttnArgs {
     // prefill after F32 staging): per mask row (batch bm_i, plane p, row q at
     // (bm_i * hm + p) * nq + q) the live interval {lo, hi} when the row is 0
     // on [lo, hi] and -inf elsewhere ({n_kv, -1}: no live entry), else
-    // {-2, -2}; written by a pre-pass launch into workspace scratch
+    // {-2, -2}; written by a pre-pass launch into workspace scratch.
+    // Batched decode with a mask tensor: the rows' live ranges (fa_decode.hip)
     int2* mask_rows;
     int32_t mask_rows_ready;   // host: mask_rows has been filled by an earlier launch of this call
     size_t ws_bytes;      // prefill: bytes at ws

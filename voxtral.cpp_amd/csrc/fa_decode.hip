@@ -68,6 +68,7 @@
 // implicit causal / window mask leaves to the query) and sizes the splits to
 // it, so no scan runs.
 #include "fa_common.h"
+#include "fa_mask_rows.h"
 
 #include <type_traits>
 
@@ -75,6 +76,29 @@ namespace vxfa {
 
 constexpr int DEC_WAVES = kDecodeWaves;
 constexpr int DEC_THREADS = 64 * DEC_WAVES;
+
+// Batches with a mask tensor (streams of ragged lengths): a pre-pass leaves
+// each mask row's live range in a.mask_rows ({lo, hi} inclusive, {0, -1} when
+// empty; lo complemented when the row holds anything but 0 inside it), and
+// each stream's range is cut into as many splits of about a.dec_chunk
+// positions as it needs: the grid's splits past those end at once.
+struct RowSplit {
+    int lo, hi;    // live positions [lo, hi)
+    bool exact;    // every entry in it is 0
+    int n, size;   // splits, positions per split (whole workgroup rounds)
+};
+__device__ __forceinline__ RowSplit row_split(const AttnArgs& a, int row) {
+    const int2 r = a.mask_rows[row];
+    RowSplit s;
+    s.exact = r.x >= 0;
+    s.lo = s.exact ? r.x : ~r.x;
+    s.hi = r.y + 1;
+    const int span = s.hi - s.lo;
+    s.n = max((span + a.dec_chunk - 1) / a.dec_chunk, 1);
+    const int unit = a.dec_t16 || a.kv_f32 ? 16 : 32;
+    s.size = ((span + s.n - 1) / s.n + unit - 1) & ~(unit - 1);
+    return s;
+}
 
 // Log-sum-exp merge of the n_split partial records, one wavefront per
 // (query head, 32 output dims):
@@ -88,7 +112,7 @@ constexpr int DEC_THREADS = 64 * DEC_WAVES;
 // row rotation and two lane-swap instructions, on the VALU: the former
 // 64-lane LDS shuffles made three dependent chains of up to six round
 // trips). Fixed order: the output is deterministic.
-template <int D, int G, int MAXS>
+template <int D, int G, int MAXS, bool TAB>
 __global__ __launch_bounds__(64) void fa_decode_combine(AttnArgs a) {
     constexpr int CSUB = D / 32;                  // 32-dim slices per head
     constexpr int CF4 = 8;                        // float4 per slice
@@ -106,8 +130,13 @@ __global__ __launch_bounds__(64) void fa_decode_combine(AttnArgs a) {
     const int h = rest / CSUB, sl = rest % CSUB;
     const int hq = g * G + h;
     const int b = blockIdx.y;
-    const int ns = a.n_split;
-    const float* base = a.ws + (int64_t)(b * a.hkv + g) * ns * RS;
+    int ns = a.n_split;
+    if constexpr (TAB) {
+        const RowSplit rs = row_split(a, b % a.bm);
+        ns = rs.n;
+        if (ns <= 1) return;   // the one split wrote the output
+    }
+    const float* base = a.ws + (int64_t)(b * a.hkv + g) * a.n_split * RS;
     const int f = lane % CF4, grp = lane / CF4;
 
     floatx4 o[MAXS];
@@ -171,10 +200,27 @@ struct DecodeDivs {
     DivMod hkv, split, bgrp, hm, bm;
 };
 
-// two wavefronts per SIMD (256 registers per lane, arch + accumulation): the
-// masked f16 variant otherwise took 256 + 2 and ran one per SIMD
-template <int D, int G, bool QF16, bool MASK, bool KV32, bool RING, bool T16>
-__global__ __launch_bounds__(DEC_THREADS, 2) void fa_decode(AttnArgs a, DecodeDivs dv) {
+// LDS of one decode workgroup.
+template <int D, int G, bool KV32, int TP>
+struct DecodeLds {
+    floatx4 p[DEC_WAVES][TP];
+    float acc[DEC_WAVES][G][D];
+    float m[DEC_WAVES][G];
+    float l[DEC_WAVES][G];
+    int red[2 * DEC_WAVES];
+    // the group's query heads [G][D]: f16 against f16 K, F32 against F32 K
+    __align__(16) char q_raw[G * D * (KV32 ? 4 : 2)];
+    float2 rope[D / 2];   // cos / sin of each pair's rotary angle (with rope_pos)
+    // each wavefront's K tile: TP rows of f16 (f16 K) or F32 (F32 K), 8 KiB either way
+    __align__(16) char kt_raw[DEC_WAVES * TP * D * (KV32 ? 4 : 2)];
+};
+
+// The workgroup's split `split` of n_split over the live positions [lo, hi)
+// (MASK: they are found here by a scan of the mask row(s) unless `scanned`);
+// size > 0: split s takes the size positions from lo + s size.
+template <int D, int G, bool QF16, bool MASK, bool KV32, bool RING, bool T16, class Lds>
+__device__ __forceinline__ void decode_body(const AttnArgs& a, const DecodeDivs& dv, Lds& lds, int g, int b, int split,
+                                            int n_split, int lo, int hi, int size) {
     static_assert(D == 64 || D == 128, "head dim");
     static_assert(G == 1 || G == 2 || G == 4, "GQA group");
     constexpr int KS = D / 32;        // MFMA k-steps of 32 dims
@@ -189,25 +235,20 @@ __global__ __launch_bounds__(DEC_THREADS, 2) void fa_decode(AttnArgs a, DecodeDi
     constexpr int ESZ = KV32 ? 4 : 2; // K/V element size
     constexpr int NCH = D / 8;        // 16-byte chunks of an f16 row
 
-    __shared__ floatx4 lds_p[DEC_WAVES][TP];
-    __shared__ float lds_acc[DEC_WAVES][G][D];
-    __shared__ float lds_m[DEC_WAVES][G];
-    __shared__ float lds_l[DEC_WAVES][G];
-    __shared__ int lds_red[2 * DEC_WAVES];
-    // the group's query heads [G][D]: f16 against f16 K, F32 against F32 K
-    __shared__ __align__(16) char lds_q_raw[G * D * (KV32 ? 4 : 2)];
-    __shared__ float2 lds_rope[D / 2];   // cos / sin of each pair's rotary angle (with rope_pos)
-    // each wavefront's K tile: TP rows of f16 (f16 K) or F32 (F32 K), 8 KiB either way
-    __shared__ __align__(16) char lds_kt_raw[DEC_WAVES * TP * D * ESZ];
+    auto& lds_p = lds.p;
+    auto& lds_acc = lds.acc;
+    auto& lds_m = lds.m;
+    auto& lds_l = lds.l;
+    auto& lds_red = lds.red;
+    auto& lds_q_raw = lds.q_raw;
+    auto& lds_rope = lds.rope;
+    auto& lds_kt_raw = lds.kt_raw;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     // wave-uniform (a scalar register): tile indices, row bases and loop
     // bounds derived from it stay on the scalar unit
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int g = (int)dv.hkv.mod(blockIdx.x);
-    const int split = (int)dv.hkv.div(blockIdx.x);
-    const int b = blockIdx.y;
     const int bkv = (int)dv.bgrp.div(b);
     constexpr bool masked = MASK;  // compile time, like QF16, so no load is conditional at run time
     // rotary position of the query token (also the appended row's: the host
@@ -229,8 +270,7 @@ __global__ __launch_bounds__(DEC_THREADS, 2) void fa_decode(AttnArgs a, DecodeDi
     // ---- live range of the KV axis -------------------------------------
     // The mask rows of this group's query heads: planes (g G + j) % hm of
     // batch b % bm. One scan when they are one plane or consecutive planes.
-    int lo = a.kv_lo, hi = a.kv_hi;   // without a mask tensor the host gives the live range
-    if constexpr (masked) {
+    if (masked && size == 0) {
         const char* mb = (const char*)a.mask + (int64_t)dv.bm.mod(b) * a.m_nb3;
         const int p0 = (int)dv.hm.mod(g * G);
         const int np = a.hm == 1 ? 1 : (p0 + G <= a.hm ? G : 0);
@@ -259,12 +299,15 @@ __global__ __launch_bounds__(DEC_THREADS, 2) void fa_decode(AttnArgs a, DecodeDi
     const int ntiles = (span + TP - 1) / TP;
     // (ntiles * n_split < 2^31 but for caches of more than 2^30 positions)
     int t_begin, t_end;
-    if (ntiles < (1 << 25)) {
+    if (size > 0) {
+        t_begin = min(split * (size / TP), ntiles);
+        t_end = min(t_begin + size / TP, ntiles);
+    } else if (ntiles < (1 << 25)) {
         t_begin = (int)dv.split.div((uint32_t)(ntiles * split));
         t_end = (int)dv.split.div((uint32_t)(ntiles * (split + 1)));
     } else {
-        t_begin = (int)(((int64_t)ntiles * split) / a.n_split);
-        t_end = (int)(((int64_t)ntiles * (split + 1)) / a.n_split);
+        t_begin = (int)(((int64_t)ntiles * split) / n_split);
+        t_end = (int)(((int64_t)ntiles * (split + 1)) / n_split);
     }
 
     const char* kb = (const char*)a.k + (int64_t)g * a.k_nb2 + (int64_t)bkv * a.k_nb3;
@@ -615,7 +658,7 @@ __global__ __launch_bounds__(DEC_THREADS, 2) void fa_decode(AttnArgs a, DecodeDi
     // The lanes holding each element once write the rounded row to the cache.
     // (f16 caches only; the host rejects an append to an F32 cache.)
     if constexpr (!KV32) {
-        if (a.append && split == a.n_split - 1 && wave == 0) {
+        if (a.append && split == n_split - 1 && wave == 0) {
             const int pn = a.nkv - 1;
             const float* kn = (const float*)((const char*)a.k_new + (int64_t)bkv * a.kn_nb3) + g * D;
             const float* vn = (const float*)((const char*)a.v_new + (int64_t)bkv * a.vn_nb3) + g * D;
@@ -722,7 +765,7 @@ __global__ __launch_bounds__(DEC_THREADS, 2) void fa_decode(AttnArgs a, DecodeDi
     __syncthreads();
 
     float* rec = nullptr;
-    if (a.n_split > 1)
+    if (n_split > 1)
         rec = a.ws + ((int64_t)(b * a.hkv + g) * a.n_split + split) * dec_record_floats(D, G);
     for (int o = tid; o < G * D; o += DEC_THREADS) {
         const int h = o / D, d = o % D;
@@ -746,30 +789,90 @@ __global__ __launch_bounds__(DEC_THREADS, 2) void fa_decode(AttnArgs a, DecodeDi
     }
 }
 
+// MM: 0 no mask tensor (the host gives the live range), 1 a mask tensor whose
+// row(s) every workgroup scans, 2 a mask tensor with its rows' live ranges in
+// a.mask_rows (one head plane); ranges of zeros then take the maskless path.
+// Two wavefronts per SIMD (256 registers per lane, arch + accumulation): the
+// masked f16 variant otherwise took 256 + 2 and ran one per SIMD
+template <int D, int G, bool QF16, int MM, bool KV32, bool RING, bool T16>
+__global__ __launch_bounds__(DEC_THREADS, 2) void fa_decode(AttnArgs a, DecodeDivs dv) {
+    __shared__ DecodeLds<D, G, KV32, (KV32 || T16) ? 16 : 32> lds;
+    const int g = (int)dv.hkv.mod(blockIdx.x);
+    const int split = (int)dv.hkv.div(blockIdx.x);
+    const int b = blockIdx.y;
+    if constexpr (MM == 2) {
+        const RowSplit rs = row_split(a, (int)dv.bm.mod(b));
+        if (split >= rs.n) return;
+        if (rs.exact) decode_body<D, G, QF16, false, KV32, RING, T16>(a, dv, lds, g, b, split, rs.n, rs.lo, rs.hi, rs.size);
+        else decode_body<D, G, QF16, true, KV32, RING, T16>(a, dv, lds, g, b, split, rs.n, rs.lo, rs.hi, rs.size);
+    } else {
+        decode_body<D, G, QF16, MM == 1, KV32, RING, T16>(a, dv, lds, g, b, split, a.n_split, a.kv_lo, a.kv_hi, 0);
+    }
+}
+
+// The live range of each mask row (one query row per stream, one head plane:
+// row = mask batch), for MM 2 above: one workgroup per row.
+constexpr int DEC_MR_THREADS = 512;
+__global__ __launch_bounds__(DEC_MR_THREADS) void decode_mask_rows_kernel(AttnArgs a) {
+    __shared__ int red[4][DEC_MR_THREADS / 64];
+    const MaskRowArgs m{a.mask, a.m_nb1, a.m_nb2, a.m_nb3, a.nkv, 1, 1, a.bm, a.mask_rows};
+    const MaskRowPart p = mask_row_part<DEC_MR_THREADS>(m, blockIdx.x, threadIdx.x);
+    const int wave = threadIdx.x >> 6;
+    const int lo = wave_min_dpp(p.lo), hi = wave_max_dpp(p.hi), cnt = wave_sum_dpp(p.cnt);
+    const int nz = wave_max_dpp(p.nz != 0 ? 1 : 0);
+    if ((threadIdx.x & 63) == 0) {
+        red[0][wave] = lo;
+        red[1][wave] = hi;
+        red[2][wave] = cnt;
+        red[3][wave] = nz;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int l = red[0][0], h = red[1][0], c = red[2][0], z = red[3][0];
+        for (int w = 1; w < DEC_MR_THREADS / 64; ++w) {
+            l = min(l, red[0][w]);
+            h = max(h, red[1][w]);
+            c += red[2][w];
+            z |= red[3][w];
+        }
+        a.mask_rows[blockIdx.x] = h < l ? int2{0, -1} : int2{(z || c != h - l + 1) ? ~l : l, h};
+    }
+}
+
 template <int D, int G, bool KV32, bool T16>
 static hipError_t launch_dgk(const AttnArgs& a, hipStream_t st) {
     const dim3 grid(a.n_split * a.hkv, a.b), block(DEC_THREADS);
     const DecodeDivs dv = {DivMod::make(a.hkv), DivMod::make(a.n_split), DivMod::make(a.b / a.bk),
                            DivMod::make(a.hm > 0 ? a.hm : 1), DivMod::make(a.bm > 0 ? a.bm : 1)};
-    if (a.mask) {
-        if (a.q_f16) hipLaunchKernelGGL((fa_decode<D, G, true, true, KV32, false, T16>), grid, block, 0, st, a, dv);
-        else hipLaunchKernelGGL((fa_decode<D, G, false, true, KV32, false, T16>), grid, block, 0, st, a, dv);
+    const bool tab = a.mask && a.mask_rows;
+    if (tab) {
+        hipLaunchKernelGGL(decode_mask_rows_kernel, dim3(a.bm), dim3(DEC_MR_THREADS), 0, st, a);
+        if (a.q_f16) hipLaunchKernelGGL((fa_decode<D, G, true, 2, KV32, false, T16>), grid, block, 0, st, a, dv);
+        else hipLaunchKernelGGL((fa_decode<D, G, false, 2, KV32, false, T16>), grid, block, 0, st, a, dv);
+    } else if (a.mask) {
+        if (a.q_f16) hipLaunchKernelGGL((fa_decode<D, G, true, 1, KV32, false, T16>), grid, block, 0, st, a, dv);
+        else hipLaunchKernelGGL((fa_decode<D, G, false, 1, KV32, false, T16>), grid, block, 0, st, a, dv);
     } else if (a.ring_cap > 0) {
         // a ring: f16 cache, no mask tensor (the host rejects anything else)
         if constexpr (!KV32) {
-            if (a.q_f16) hipLaunchKernelGGL((fa_decode<D, G, true, false, false, true, T16>), grid, block, 0, st, a, dv);
-            else hipLaunchKernelGGL((fa_decode<D, G, false, false, false, true, T16>), grid, block, 0, st, a, dv);
+            if (a.q_f16) hipLaunchKernelGGL((fa_decode<D, G, true, 0, false, true, T16>), grid, block, 0, st, a, dv);
+            else hipLaunchKernelGGL((fa_decode<D, G, false, 0, false, true, T16>), grid, block, 0, st, a, dv);
         }
     } else {
-        if (a.q_f16) hipLaunchKernelGGL((fa_decode<D, G, true, false, KV32, false, T16>), grid, block, 0, st, a, dv);
-        else hipLaunchKernelGGL((fa_decode<D, G, false, false, KV32, false, T16>), grid, block, 0, st, a, dv);
+        if (a.q_f16) hipLaunchKernelGGL((fa_decode<D, G, true, 0, KV32, false, T16>), grid, block, 0, st, a, dv);
+        else hipLaunchKernelGGL((fa_decode<D, G, false, 0, KV32, false, T16>), grid, block, 0, st, a, dv);
     }
     // the combine loads ceil(n_split / 8) partial slices per lane
     const dim3 cgrid(a.hkv * G * (D / 32), a.b);
-    if (a.n_split > 32) hipLaunchKernelGGL((fa_decode_combine<D, G, 8>), cgrid, dim3(64), 0, st, a);
-    else if (a.n_split > 16) hipLaunchKernelGGL((fa_decode_combine<D, G, 4>), cgrid, dim3(64), 0, st, a);
-    else if (a.n_split > 8) hipLaunchKernelGGL((fa_decode_combine<D, G, 2>), cgrid, dim3(64), 0, st, a);
-    else if (a.n_split > 1) hipLaunchKernelGGL((fa_decode_combine<D, G, 1>), cgrid, dim3(64), 0, st, a);
+    auto merge = [&](auto tab_tag) {
+        constexpr bool TAB = decltype(tab_tag)::value;
+        if (a.n_split > 32) hipLaunchKernelGGL((fa_decode_combine<D, G, 8, TAB>), cgrid, dim3(64), 0, st, a);
+        else if (a.n_split > 16) hipLaunchKernelGGL((fa_decode_combine<D, G, 4, TAB>), cgrid, dim3(64), 0, st, a);
+        else if (a.n_split > 8) hipLaunchKernelGGL((fa_decode_combine<D, G, 2, TAB>), cgrid, dim3(64), 0, st, a);
+        else if (a.n_split > 1) hipLaunchKernelGGL((fa_decode_combine<D, G, 1, TAB>), cgrid, dim3(64), 0, st, a);
+    };
+    if (tab) merge(std::true_type{});
+    else merge(std::false_type{});
     return hipGetLastError();
 }
 template <int D, int G>
@@ -784,6 +887,11 @@ hipError_t launch_decode(const AttnArgs& a, int head_dim, int group, hipStream_t
     if (a.b > 65535 || (int64_t)a.n_split * a.hkv > 0x7fffffff) return hipErrorInvalidValue;
     if (a.kv_f32 && a.append) return hipErrorInvalidValue;
     if (a.ring_cap > 0 && (a.kv_f32 || a.mask)) return hipErrorInvalidValue;
+    // row ranges: one head plane; dec_chunk positions a split at most, all of
+    // n_kv within n_split of them
+    if (a.mask && a.mask_rows && (a.hm != 1 || a.dec_chunk < 1 || a.bm < 1 ||
+                                  ((int64_t)a.nkv + a.dec_chunk - 1) / a.dec_chunk > a.n_split))
+        return hipErrorInvalidValue;
     // the kernel's 32-bit lane offsets: row strides below 2^24 bytes; a ring
     // of fewer than 2^24 rows spanning less than 2^31 bytes
     if (a.k_nb1 < 0 || a.k_nb1 >= (1 << 24) || a.v_nb1 < 0 || a.v_nb1 >= (1 << 24)) return hipErrorInvalidValue;

@@ -64,17 +64,21 @@ __device__ __forceinline__ int wave_sum_dpp(int x) {
 // SIMD issues at about half the SIMD's rate (1500 realtime-encoder rows:
 // 4.8 us with 16 lanes and 12 chunks per lane).
 constexpr int kMaskRowChunks = 3;    // chunks per lane per round
-constexpr int kMaskRowRound = 64 * kMaskRowChunks;
 struct MaskRowArgs {
     const uint16_t* mask;
     int64_t nb1, nb2, nb3;
     int n, nq, hm, nrows;
     int2* out;
 };
-// Mask row w (w < nrows, uniform over the wavefront) by lane s (0..63);
-// every lane calls it (waves past the last row pass w = nrows - 1 and store
-// nothing).
-__device__ __forceinline__ void mask_row_interval(const MaskRowArgs& m, int w, int s, bool store) {
+// What thread s of NT sees of mask row w: first and last live column, their
+// count, and whether one is not zero.
+struct MaskRowPart {
+    int lo, hi, cnt;
+    uint32_t nz;
+};
+template <int NT>
+__device__ __forceinline__ MaskRowPart mask_row_part(const MaskRowArgs& m, int w, int s) {
+    constexpr int kMaskRowRound = NT * kMaskRowChunks;
     const int q = w % m.nq, pb = w / m.nq, p = pb % m.hm, bb = pb / m.hm;
     const char* rowp = (const char*)m.mask + (int64_t)q * m.nb1 + (int64_t)p * m.nb2 + (int64_t)bb * m.nb3;
     const int mis = (int)(reinterpret_cast<uintptr_t>(rowp) & 15);   // even: the mask is 2-byte aligned
@@ -87,10 +91,10 @@ __device__ __forceinline__ void mask_row_interval(const MaskRowArgs& m, int w, i
     for (int c0 = 0; c0 < nchmax; c0 += kMaskRowRound) {
         u32x4 wv[kMaskRowChunks];
 #pragma unroll
-        for (int u = 0; u < kMaskRowChunks; ++u) wv[u] = *(const u32x4*)(base + 16 * min(c0 + 64 * u + s, nch - 1));
+        for (int u = 0; u < kMaskRowChunks; ++u) wv[u] = *(const u32x4*)(base + 16 * min(c0 + NT * u + s, nch - 1));
 #pragma unroll
         for (int u = 0; u < kMaskRowChunks; ++u) {
-            const int col0 = 8 * (c0 + 64 * u + s) - mis / 2;      // column of the chunk's first entry
+            const int col0 = 8 * (c0 + NT * u + s) - mis / 2;      // column of the chunk's first entry
             const int elo = max(-col0, 0), ehi = min(n - col0, 8);  // entries [elo, ehi) lie in the row
             const uint32_t valid = ehi > elo ? ((1u << ehi) - 1u) & ~((1u << elo) - 1u) : 0u;
             uint32_t live = 0, nz = 0;
@@ -110,12 +114,19 @@ __device__ __forceinline__ void mask_row_interval(const MaskRowArgs& m, int w, i
             cnt += __builtin_popcount(live);
         }
     }
-    lo = wave_min_dpp(lo);
-    hi = wave_max_dpp(hi);
-    cnt = wave_sum_dpp(cnt);
-    const int nonzero = wave_max_dpp(nzall != 0 ? 1 : 0);
+    return MaskRowPart{lo, hi, cnt, nzall};
+}
+// Mask row w (w < nrows, uniform over the wavefront) by lane s (0..63);
+// every lane calls it (waves past the last row pass w = nrows - 1 and store
+// nothing).
+__device__ __forceinline__ void mask_row_interval(const MaskRowArgs& m, int w, int s, bool store) {
+    const MaskRowPart p = mask_row_part<64>(m, w, s);
+    const int lo = wave_min_dpp(p.lo);
+    const int hi = wave_max_dpp(p.hi);
+    const int cnt = wave_sum_dpp(p.cnt);
+    const int nonzero = wave_max_dpp(p.nz != 0 ? 1 : 0);
     if (s == 0 && store)
-        m.out[w] = hi < lo ? int2{n, -1} : ((nonzero || cnt != hi - lo + 1) ? int2{-2, -2} : int2{lo, hi});
+        m.out[w] = hi < lo ? int2{m.n, -1} : ((nonzero || cnt != hi - lo + 1) ? int2{-2, -2} : int2{lo, hi});
 }
 
 // mask rows [4 bx, 4 bx + 4), one per wavefront

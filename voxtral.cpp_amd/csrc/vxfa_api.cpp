@@ -500,19 +500,38 @@ int run(Workspace& w, const vxfa_tensor* q, const vxfa_tensor* k, const vxfa_ten
         // keep every wavefront busy on a window's share (2048 of 16384 rows in
         // 32 splits: 10.29 -> 9.83 us)
         if (mask && B == 1 && !a.kv_f32) t16 = true;
-        if (mask && B > 1) {
-            // streams of ragged lengths (a mask row each): the longest sets the
-            // time, so split every stream finer, about 2048 workgroups in all
-            const int64_t s2 = (2048 + B * Hkv - 1) / (B * Hkv);
-            if (s2 > S) S = (int)(s2 < (Nkv + 63) / 64 ? s2 : (Nkv + 63) / 64);
+        size_t used = 0;
+        if (mask && B > 1 && a.hm == 1 && Nkv < (1 << 30)) {
+            // streams of ragged lengths (a mask row each): the rows' live ranges
+            // by a pre-pass, then splits of up to `chunk` positions, about
+            // 4096 workgroups in all if every stream were full: the streams'
+            // lengths differ, so the splits have to be fine for the last round
+            const int64_t pairs = B * Hkv;
+            int64_t s2 = w.tune.split_override > 0 ? w.tune.split_override : (4096 + pairs - 1) / pairs;
+            if (s2 > vxfa::kDecodeMaxSplit) s2 = vxfa::kDecodeMaxSplit;
+            used = ((size_t)a.bm * sizeof(int2) + 255) & ~(size_t)255;
+            s2 = fit_split((int)s2, pairs, vxfa::dec_record_floats((int)D, (int)G), w.rec_bytes - used);
+            // whole rounds of the four wavefronts' tiles
+            int64_t chunk = (Nkv + s2 - 1) / s2;
+            t16 = !a.kv_f32 && chunk <= 64;
+            const int64_t round = vxfa::kDecodeWaves * (t16 || a.kv_f32 ? 16 : 32);
+            chunk = (chunk + round - 1) / round * round;
+            S = (int)((Nkv + chunk - 1) / chunk);
+            a.dec_chunk = (int32_t)chunk;
+            a.mask_rows = reinterpret_cast<int2*>(w.base);
+        } else {
+            if (mask && B > 1) {
+                const int64_t s2 = (2048 + B * Hkv - 1) / (B * Hkv);
+                if (s2 > S) S = (int)(s2 < (Nkv + 63) / 64 ? s2 : (Nkv + 63) / 64);
+            }
+            if (mask && S > kMaskedSplitCap) S = kMaskedSplitCap;
+            if (w.tune.split_override > 0) S = w.tune.split_override;
+            if (S > vxfa::kDecodeMaxSplit) S = vxfa::kDecodeMaxSplit;
+            S = fit_split(S, B * Hkv, vxfa::dec_record_floats((int)D, (int)G), w.rec_bytes);
         }
-        if (mask && S > kMaskedSplitCap) S = kMaskedSplitCap;
-        if (w.tune.split_override > 0) S = w.tune.split_override;
-        if (S > vxfa::kDecodeMaxSplit) S = vxfa::kDecodeMaxSplit;
-        S = fit_split(S, B * Hkv, vxfa::dec_record_floats((int)D, (int)G), w.rec_bytes);
         a.n_split = S;
         a.dec_t16 = t16 ? 1 : 0;
-        a.ws = reinterpret_cast<float*>(w.base);
+        a.ws = reinterpret_cast<float*>(w.base + used);
         e = vxfa::launch_decode(a, (int)D, (int)G, st);
     } else {
         size_t staged = 0;   // bytes of the staging area this call fills
