@@ -291,7 +291,7 @@ __device__ __forceinline__ void decode_body(const AttnArgs& a, const DecodeDivs&
     }
 
     // With a fused append the new row (n_kv - 1) is not read from the cache:
-    // every workgroup walks [lo, hi_main) and wavefront 0 of the last split
+    // every workgroup walks [lo, hi_main) and a wavefront of the last split
     // folds the new row in afterwards, from the F32 source.
     const bool new_live = a.append && hi == a.nkv;
     const int hi_main = a.append ? min(hi, a.nkv - 1) : hi;
@@ -299,16 +299,20 @@ __device__ __forceinline__ void decode_body(const AttnArgs& a, const DecodeDivs&
     const int ntiles = (span + TP - 1) / TP;
     // (ntiles * n_split < 2^31 but for caches of more than 2^30 positions)
     int t_begin, t_end;
+    // (an appended row counts as one more tile, the last: it falls to the last
+    // split, and there to the wavefront whose turn it would be)
+    const int nall = ntiles + (a.append ? 1 : 0);
     if (size > 0) {
         t_begin = min(split * (size / TP), ntiles);
         t_end = min(t_begin + size / TP, ntiles);
-    } else if (ntiles < (1 << 25)) {
-        t_begin = (int)dv.split.div((uint32_t)(ntiles * split));
-        t_end = (int)dv.split.div((uint32_t)(ntiles * (split + 1)));
+    } else if (nall < (1 << 25)) {
+        t_begin = (int)dv.split.div((uint32_t)(nall * split));
+        t_end = min((int)dv.split.div((uint32_t)(nall * (split + 1))), ntiles);
     } else {
-        t_begin = (int)(((int64_t)ntiles * split) / n_split);
-        t_end = (int)(((int64_t)ntiles * (split + 1)) / n_split);
+        t_begin = (int)(((int64_t)nall * split) / n_split);
+        t_end = (int)min(((int64_t)nall * (split + 1)) / n_split, (int64_t)ntiles);
     }
+    const bool appends = a.append && split == n_split - 1 && wave == (t_end - t_begin) % DEC_WAVES;
 
     const char* kb = (const char*)a.k + (int64_t)g * a.k_nb2 + (int64_t)bkv * a.k_nb3;
     const char* vb = (const char*)a.v + (int64_t)g * a.v_nb2 + (int64_t)bkv * a.v_nb3;
@@ -630,6 +634,26 @@ __device__ __forceinline__ void decode_body(const AttnArgs& a, const DecodeDivs&
         __builtin_amdgcn_wave_barrier();
     };
 
+    // The new row's F32 loads: with the 16-position tiles of short spans ahead
+    // of the main loop, where they cost no round trip of their own (the larger
+    // tiles have no registers left for them). With its own turn among the
+    // wavefronts, n_kv 435 in 8 splits: append 6.96 -> 6.14 us per layer, rope
+    // + append 7.64 -> 6.73 (it was wavefront 0 of the last split's fifth tile,
+    // its loads after the loop).
+    floatx4 new_k[2], new_v[2];
+    auto load_new = [&]() {
+        const floatx4* kn = (const floatx4*)((const char*)a.k_new + (int64_t)bkv * a.kn_nb3 + (g * D + vcol) * 4);
+        const floatx4* vn = (const floatx4*)((const char*)a.v_new + (int64_t)bkv * a.vn_nb3 + (g * D + vcol) * 4);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            new_k[u] = kn[u];
+            new_v[u] = vn[u];
+        }
+    };
+    if constexpr (!KV32 && T16) {
+        if (appends) load_new();
+    }
+
     // ---- main loop: two register sets, the next tile loads during compute ----
     // (The next tile's loads sit under a branch, so at the join the compiler
     // counts loads in flight as on the path without them: in a walk of
@@ -652,23 +676,15 @@ __device__ __forceinline__ void decode_body(const AttnArgs& a, const DecodeDivs&
     }
 
     // ---- fused append: the new row, from the F32 sources --------------------
-    // Every lane reads the new row in its own K and V operand layout (all
+    // Every lane holds the new row in its own K and V operand layout (all
     // positions of the one-row tile clamp to it; only position n_kv - 1 is
     // valid in process()), rounded to f16 exactly as the cache will hold it.
     // The lanes holding each element once write the rounded row to the cache.
     // (f16 caches only; the host rejects an append to an F32 cache.)
     if constexpr (!KV32) {
-        if (a.append && split == n_split - 1 && wave == 0) {
+        if (appends) {
             const int pn = a.nkv - 1;
-            const float* kn = (const float*)((const char*)a.k_new + (int64_t)bkv * a.kn_nb3) + g * D;
-            const float* vn = (const float*)((const char*)a.v_new + (int64_t)bkv * a.vn_nb3) + g * D;
-            // every load of the row first (one round trip), then rotation (K,
-            // with rope_pos; the table holds the row's angles) and rounding
-            floatx4 kr[2], vr[2];
-            kr[0] = *(const floatx4*)(kn + vcol);
-            kr[1] = *(const floatx4*)(kn + vcol + 4);
-            vr[0] = *(const floatx4*)(vn + vcol);
-            vr[1] = *(const floatx4*)(vn + vcol + 4);
+            if constexpr (!T16) load_new();
             auto cvt8 = [&](const floatx4 (&r)[2], int d0, bool rot) {
                 float x[8] = {r[0][0], r[0][1], r[0][2], r[0][3], r[1][0], r[1][1], r[1][2], r[1][3]};
                 if (rot) rope8_tab(x, d0, lds_rope, a.rope_dims);
@@ -678,8 +694,8 @@ __device__ __forceinline__ void decode_body(const AttnArgs& a, const DecodeDivs&
                 return y;
             };
             const bool rot = a.rope_pos != nullptr;
-            const half8 kx = cvt8(kr, vcol, rot);
-            const half8 vx = cvt8(vr, vcol, false);
+            const half8 kx = cvt8(new_k, vcol, rot);
+            const half8 vx = cvt8(new_v, vcol, false);
 #pragma unroll
             for (int i = 0; i < NV; ++i) {
                 TA.k[i] = kx;

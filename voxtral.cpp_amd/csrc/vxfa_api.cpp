@@ -495,6 +495,15 @@ int run(Workspace& w, const vxfa_tensor* q, const vxfa_tensor* k, const vxfa_ten
         }
         bool t16 = false;
         int S = choose_split(B * Hkv, a.kv_hi - a.kv_lo, a.kv_f32 != 0, &t16);
+        // an appended row is a tile of its own: where the other tiles fill every
+        // wavefront, one more split, while there is a CU for it (n_kv 435: 8
+        // splits rope + append 6.73 us, 7 7.63; a full 2048-row ring would
+        // need 264 workgroups, 7.49 us against 7.41)
+        if (fuse_append && t16 && S > 1) {
+            const int64_t tiles = (a.kv_hi - a.kv_lo - 1 + 15) / 16 + 1;
+            const int64_t s1 = (tiles + vxfa::kDecodeWaves - 1) / vxfa::kDecodeWaves;
+            if (s1 > S && s1 * B * Hkv <= 256) S = (int)s1;
+        }
         // one mask row (a sliding window over a longer cache): the live span,
         // which sets the tiles per split, is found by the kernel; tiles of 16
         // keep every wavefront busy on a window's share (2048 of 16384 rows in
