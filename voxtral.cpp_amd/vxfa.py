@@ -112,6 +112,10 @@ def load() -> ctypes.CDLL:
     if not os.path.exists(LIB_PATH):
         raise RuntimeError(f"{LIB_PATH} is missing: build it with `make -C {HERE}` "
                            "(or __graft_entry__.build()); there is no fallback path")
+    # Descriptors are passed as they are: ctypes hands a structure to a
+    # POINTER parameter by reference itself, after its type check. (byref
+    # objects made per argument and a c_void_p per stream cost 1.2 of the 2.2
+    # us that a call spent in Python.)
     L = ctypes.CDLL(LIB_PATH)
     P = ctypes.POINTER(VxfaTensor)
     L.vxfa_ctx_create.argtypes = [ctypes.c_int]
@@ -171,13 +175,9 @@ def desc(ptr: int, type_: int, ne, nb) -> VxfaTensor:
     return t
 
 
-def _ref(t):
-    return ctypes.byref(t) if t is not None else None
-
-
 def check_mask_desc(m) -> int:
     """Host-only validation of a mask descriptor (VxfaMaskDesc or None)."""
-    return load().vxfa_check_mask_desc(_ref(m))
+    return load().vxfa_check_mask_desc(m)
 
 
 def flash_attn_ext_noalloc(q, k, v, mask, dst, scale: float, max_bias: float = 0.0, logit_softcap: float = 0.0,
@@ -186,8 +186,8 @@ def flash_attn_ext_noalloc(q, k, v, mask, dst, scale: float, max_bias: float = 0
     context; scratch in the library's static per-GPU array (calls that
     overlap on one GPU race)."""
     L = load()
-    rc = L.vxfa_flash_attn_ext_noalloc(_ref(q), _ref(k), _ref(v), _ref(mask), _ref(dst), scale, max_bias,
-                                       logit_softcap, ctypes.c_void_p(stream))
+    rc = L.vxfa_flash_attn_ext_noalloc(q, k, v, mask, dst, scale, max_bias,
+                                       logit_softcap, stream)
     if check and rc != OK:
         raise VxfaError(rc, L.vxfa_last_error(None).decode())
     return rc
@@ -195,7 +195,7 @@ def flash_attn_ext_noalloc(q, k, v, mask, dst, scale: float, max_bias: float = 0
 
 def supports(q, k, v, mask, dst, scale: float, max_bias: float = 0.0, logit_softcap: float = 0.0) -> int:
     """Host-only capability check (ggml supports_op analogue)."""
-    return load().vxfa_supports(_ref(q), _ref(k), _ref(v), _ref(mask), _ref(dst), scale, max_bias, logit_softcap)
+    return load().vxfa_supports(q, k, v, mask, dst, scale, max_bias, logit_softcap)
 
 
 class Context:
@@ -209,8 +209,8 @@ class Context:
 
     def flash_attn_ext(self, q, k, v, mask, dst, scale: float, max_bias: float = 0.0,
                        logit_softcap: float = 0.0, stream: int = 0, check: bool = True) -> int:
-        rc = self._lib.vxfa_flash_attn_ext(self._h, _ref(q), _ref(k), _ref(v), _ref(mask), _ref(dst),
-                                           scale, max_bias, logit_softcap, ctypes.c_void_p(stream))
+        rc = self._lib.vxfa_flash_attn_ext(self._h, q, k, v, mask, dst,
+                                           scale, max_bias, logit_softcap, stream)
         if check and rc != OK:
             raise VxfaError(rc, self.last_error())
         return rc
@@ -218,15 +218,15 @@ class Context:
     def flash_attn_ext_implicit(self, q, k, v, mask_desc, dst, scale: float, max_bias: float = 0.0,
                                 logit_softcap: float = 0.0, stream: int = 0, check: bool = True) -> int:
         """The op with an implicit causal / window mask (a VxfaMaskDesc, or None)."""
-        rc = self._lib.vxfa_flash_attn_ext_implicit(self._h, _ref(q), _ref(k), _ref(v), _ref(mask_desc), _ref(dst),
-                                                    scale, max_bias, logit_softcap, ctypes.c_void_p(stream))
+        rc = self._lib.vxfa_flash_attn_ext_implicit(self._h, q, k, v, mask_desc, dst,
+                                                    scale, max_bias, logit_softcap, stream)
         if check and rc != OK:
             raise VxfaError(rc, self.last_error())
         return rc
 
     def kv_append(self, k_new, v_new, k, v, stream: int = 0, check: bool = True) -> int:
         """F32 -> F16 append of new K/V rows into the last rows of the cache views k, v."""
-        rc = self._lib.vxfa_kv_append(self._h, _ref(k_new), _ref(v_new), _ref(k), _ref(v), ctypes.c_void_p(stream))
+        rc = self._lib.vxfa_kv_append(self._h, k_new, v_new, k, v, stream)
         if check and rc != OK:
             raise VxfaError(rc, self.last_error())
         return rc
@@ -234,9 +234,9 @@ class Context:
     def flash_attn_ext_append(self, q, k, v, k_new, v_new, mask, dst, scale: float, max_bias: float = 0.0,
                               logit_softcap: float = 0.0, stream: int = 0, check: bool = True) -> int:
         """kv_append then flash_attn_ext, fused for a single-token decode step."""
-        rc = self._lib.vxfa_flash_attn_ext_append(self._h, _ref(q), _ref(k), _ref(v), _ref(k_new), _ref(v_new),
-                                                  _ref(mask), _ref(dst), scale, max_bias, logit_softcap,
-                                                  ctypes.c_void_p(stream))
+        rc = self._lib.vxfa_flash_attn_ext_append(self._h, q, k, v, k_new, v_new,
+                                                  mask, dst, scale, max_bias, logit_softcap,
+                                                  stream)
         if check and rc != OK:
             raise VxfaError(rc, self.last_error())
         return rc
@@ -244,9 +244,9 @@ class Context:
     def flash_attn_ext_ring(self, q, k, v, ring_desc, k_new, v_new, dst, scale: float, max_bias: float = 0.0,
                             logit_softcap: float = 0.0, stream: int = 0, check: bool = True) -> int:
         """A decode step over a ring-buffer cache (k_new / v_new: the step's new row, or None)."""
-        rc = self._lib.vxfa_flash_attn_ext_ring(self._h, _ref(q), _ref(k), _ref(v), _ref(ring_desc), _ref(k_new),
-                                                _ref(v_new), _ref(dst), scale, max_bias, logit_softcap,
-                                                ctypes.c_void_p(stream))
+        rc = self._lib.vxfa_flash_attn_ext_ring(self._h, q, k, v, ring_desc, k_new,
+                                                v_new, dst, scale, max_bias, logit_softcap,
+                                                stream)
         if check and rc != OK:
             raise VxfaError(rc, self.last_error())
         return rc
@@ -254,9 +254,9 @@ class Context:
     def flash_attn_ext_rope(self, q, k, v, k_new, v_new, rope_desc, mask, dst, scale: float, max_bias: float = 0.0,
                             logit_softcap: float = 0.0, stream: int = 0, check: bool = True) -> int:
         """Rotate q and the new K rows (mode 0), append the new rows, attend."""
-        rc = self._lib.vxfa_flash_attn_ext_rope(self._h, _ref(q), _ref(k), _ref(v), _ref(k_new), _ref(v_new),
-                                                _ref(rope_desc), _ref(mask), _ref(dst), scale, max_bias,
-                                                logit_softcap, ctypes.c_void_p(stream))
+        rc = self._lib.vxfa_flash_attn_ext_rope(self._h, q, k, v, k_new, v_new,
+                                                rope_desc, mask, dst, scale, max_bias,
+                                                logit_softcap, stream)
         if check and rc != OK:
             raise VxfaError(rc, self.last_error())
         return rc
