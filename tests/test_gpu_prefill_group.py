@@ -1,5 +1,5 @@
 """The hd 128 prefill whose workgroups share K/V blocks among the heads of a
-kv group (fa_prefill128.hip): tile, block and piece edges, GQA groups, mask
+kv group (fa_prefill_group.hip): tile, block and piece edges, GQA groups, mask
 forms, types and scratch limits, against the exact float64 reference.
 
 Bound: Q, K, V and P are rounded to f16 (relative 2^-11 each), sums are F32;
@@ -150,3 +150,40 @@ def test_f16_q_and_rows_that_raise_the_maximum(runner):
     b, _, ne, nb, off = c.views["q"]
     c.views["q"] = (b, oracle.F16, ne, tuple(x // 2 for x in nb), off)
     run(runner, c, atol=8e-3, rel=3e-3)
+
+
+# hd 64 (4 wavefronts, no pieces) takes masked calls of at least 384
+# workgroups: 128 rows of a head each, or 32 of a group of four
+def _hd64(kind, n, heads, q_f16=False, kv_f32=False):
+    c = cases.encoder_case(n, heads, 64, seed=3100 + n, window=750 if kind == "window" else None, q_f16=q_f16,
+                           kv_f32=kv_f32, name=f"hd64 {kind} {n}x{heads}")
+    if kind == "window":
+        return c
+    rng = np.random.default_rng(3101)
+    m = cases.implicit_mask(n, n, 0)
+    if kind == "finite":
+        m = np.where(m == 0, rng.normal(0, 2, m.shape).astype(np.float16).view(np.uint16), m).astype(np.uint16)
+    elif kind == "dead rows":
+        m[:130] = cases.NEG_INF_F16
+        m[300] = cases.NEG_INF_F16
+    return cases.with_mask(c, m)
+
+
+@pytest.mark.parametrize("kind,n,heads,kw", [("window", 1057, 44, {}), ("causal", 513, 80, {}), ("finite", 481, 96, {}),
+                                             ("dead rows", 500, 96, {"q_f16": True}),
+                                             ("window", 1100, 43, {"kv_f32": True})])
+def test_hd64(runner, kind, n, heads, kw):
+    c = _hd64(kind, n, heads, **kw)
+    out = run(runner, c)
+    if kind == "dead rows":
+        assert not out[0, :130].any() and not out[0, 300].any()
+    if kind in ("window", "causal"):
+        rc, out2 = runner.run_implicit(c, vx.mask_desc(vx.MASK_CAUSAL, 750 if kind == "window" else 0, 0))
+        assert rc == 0 and np.array_equal(out, out2)
+
+
+def test_hd64_group_and_scale(runner):
+    c = cases.prefill_case(1530, hq=32, hkv=8, hd=64, kv_offset=70, seed=3200, name="hd64 32/8")
+    run(runner, c)
+    c.scale = cases.f32(-0.2)
+    run(runner, c, rel=3e-3)

@@ -585,13 +585,14 @@ __device__ __forceinline__ float pair32_sum(float x) {
 // Host-side launchers (implemented in the kernel translation units).
 namespace vxfa {
 hipError_t launch_decode(const AttnArgs& a, int head_dim, int group, hipStream_t stream);
+constexpr int64_t kGroup64Min = 384;   // hd 64: workgroups from which launch_prefill_group is the better
 constexpr int kDecodeMaxSplit = 64;  // split workgroups per (batch, kv head)
 constexpr int kDecodeWaves = 4;      // wavefronts per decode workgroup
 // Floats per decode partial record: O [G][D], then m [G] and l [G], padded to
 // a multiple of 4 so every record starts 16-byte aligned.
 constexpr int dec_record_floats(int D, int G) { return G * D + ((2 * G + 3) & ~3); }
-// prefill beyond the kernels below; hd 128 with prefill128_takes (and a.mask_rows
-// set if there is a mask tensor) goes to launch_prefill128
+// prefill beyond the kernels below; hd 128 with prefill_group_takes (and
+// a.mask_rows set if there is a mask tensor) goes to launch_prefill_group
 hipError_t launch_prefill(const AttnArgs& a, int head_dim, int waves, hipStream_t stream);
 // hd 64 prefill on the pipelined kernel: no mask, an implicit mask, or a mask
 // tensor (a.mask_rows: workspace for nq * hm * bm intervals, filled first by
@@ -610,22 +611,37 @@ hipError_t launch_mask_prep(const AttnArgs& a, const StageReq* stage, hipStream_
 hipError_t launch_prefill_pair(const AttnArgs& a, hipStream_t stream);
 // whether launch_prefill_pair takes these strides (its 32-bit offsets)
 bool prefill_pair_fits(const AttnArgs& a);
-// hd 128 prefill with the heads of a kv group sharing K/V blocks: no mask, an
-// implicit mask, or a mask tensor (a.mask_rows filled by launch_mask_prep
-// first); a.ws: scratch for the records of tiles cut into KV pieces (any
-// size; with less, fewer pieces)
-hipError_t launch_prefill128(const AttnArgs& a, hipStream_t stream);
-// its query heads per workgroup (log2): the largest power of two, up to 8,
-// that divides the GQA group
-inline uint32_t prefill128_heads_log2(const AttnArgs& a) {
+// Prefill with a workgroup's wavefronts (32 query rows each, of the heads of a
+// kv group) sharing K/V blocks. hd 128: no mask, an implicit mask, or a mask
+// tensor (a.mask_rows filled first); a.ws: scratch for the records of tiles
+// cut into KV pieces (any size; with less, fewer pieces). hd 64: masked calls
+// without a rotary embedding.
+hipError_t launch_prefill_group(const AttnArgs& a, int head_dim, hipStream_t stream);
+// its query heads per workgroup of nw wavefronts (log2): the largest power of
+// two, up to nw, that divides the GQA group
+inline uint32_t prefill_group_heads_log2(const AttnArgs& a, int nw) {
     uint32_t l = 0;
-    while (l < 3 && (a.hq / a.hkv) % (2 << l) == 0) ++l;
+    while ((2 << l) <= nw && (a.hq / a.hkv) % (2 << l) == 0) ++l;
     return l;
 }
-// whether launch_prefill takes an hd 128 call there: at least half of a
-// workgroup's 8 wavefronts (32 rows of a head each) have rows
-inline bool prefill128_takes(const AttnArgs& a) {
-    return ((((int64_t)a.nq + 31) / 32) << prefill128_heads_log2(a)) >= 4;
+// Whether the launchers take a call there. hd 128: at least half of a
+// workgroup's 8 wavefronts have rows. hd 64 (4 wavefronts, two workgroups a CU,
+// each walking its whole range): masked calls of 384 workgroups or more, which
+// the pipelined kernel (one workgroup of 128 rows and 4 KV groups a CU, ~8 us of
+// it outside the loop) runs in two rounds. Measured, us per layer, pipelined ->
+// this: 32 heads, window 750, mask tensor and F32 K/V, 1500 frames 38.3 -> 34.4;
+// implicit mask 1500 frames 26.5 -> 25.1, 4000 70.9 -> 56.2; below the line 1400
+// frames 23.7 -> 24.8, 1200 20.9 -> 23.6. A walk of 47 blocks (causal, no window,
+// 1500 frames) is slower here, 26.0 -> 29.5, at 4000 frames even; the line does
+// not look at the mask, so that a tensor and the implicit mask it equals give
+// the same bits.
+inline bool prefill_group_takes(const AttnArgs& a, int head_dim) {
+    const int nw = head_dim == 128 ? 8 : 4;
+    const uint32_t hl = prefill_group_heads_log2(a, nw);
+    if (head_dim == 128) return ((((int64_t)a.nq + 31) / 32) << hl) >= 4;
+    if (!(a.mask || a.im_causal) || a.rope_pos) return false;
+    const int64_t bm = 32 * (nw >> hl);
+    return (a.nq + bm - 1) / bm * (a.hq >> hl) * (int64_t)a.b >= kGroup64Min;
 }
 hipError_t launch_zero(float* dst, int64_t n, hipStream_t stream);
 hipError_t launch_kv_append(const AppendArgs& a, hipStream_t stream);

@@ -824,7 +824,7 @@ static hipError_t launch_pw(const AttnArgs& a, hipStream_t st) {
 // a mask (tensor or implicit) always 2.
 hipError_t launch_prefill(const AttnArgs& a, int head_dim, int waves, hipStream_t st) {
     const int mm = a.im_causal ? 2 : (a.mask != nullptr ? 1 : 0);
-    if (head_dim == 128 && (mm != 1 || a.mask_rows) && prefill128_takes(a)) return launch_prefill128(a, st);
+    if (head_dim == 128 && (mm != 1 || a.mask_rows) && prefill_group_takes(a, 128)) return launch_prefill_group(a, 128, st);
     if (head_dim == 64) {
         if (mm == 1) return launch_pw<64, 2, 4, 1>(a, st);
         if (mm == 2) return launch_pw<64, 2, 4, 2>(a, st);

@@ -1,4 +1,4 @@
-// fa_prefill128.hip — hd 128 prefill for gfx950: the query heads of one kv
+// fa_prefill_group.hip — hd 128 prefill for gfx950: the query heads of one kv
 // head share each K/V block, the KV range is cut into pieces when the query
 // rows alone leave the chip idle.
 //
@@ -17,7 +17,7 @@
 //   workgroup each (piece p of a tile with fewer pieces ends at once). A tile
 //   of one piece writes its output; otherwise every piece leaves its
 //   unnormalised O with the rows' running max and sum in the workspace, and
-//   fa_prefill128_combine merges them in piece order.
+//   fa_prefill_group_combine merges them in piece order.
 // What bounds it: per wavefront and block 16 MFMAs (512 cycles of its SIMD's
 //   matrix pipe) against ~130 VALU instructions of softmax, so the two pipes
 //   are about even and have to overlap. PV runs one block behind:
@@ -45,23 +45,26 @@
 
 namespace vxfa {
 
-namespace p128 {
-constexpr int D = 128;
-constexpr int KS = D / 16;             // S-MFMA k-steps
-constexpr int DB = D / 32;             // O^T row blocks
-constexpr int BK = 32;                 // positions per block
-constexpr int ROW = D * 2;             // bytes per K/V row
-constexpr int BLK = BK * ROW;          // bytes of one matrix block (8 KiB)
-constexpr int STEP = 2 * BLK;          // one matrix of a 64-position step
-constexpr int NS = 4;                  // ring slots
-constexpr int NW = 8;
-constexpr int NT = 64 * NW;
-constexpr int REC = 64 * 64 + 64;      // floats of a wavefront's record: O, then (m, l) of 32 rows
-constexpr float TAU_SUM = 256.0f;      // 2^8
-constexpr float TAU = 8.0f;
-// 1/sqrt(128) in log2 units, as the host computes it from ggml's float scale
-constexpr float kC128 = 0.08838834764831845f * kLog2e;
-}  // namespace p128
+template <int HD>
+struct PG {
+    static constexpr int D = HD;
+    static constexpr int KS = D / 16;             // S-MFMA k-steps
+    static constexpr int DB = D / 32;             // O^T row blocks
+    static constexpr int BK = 32;                 // positions per block
+    static constexpr int ROW = D * 2;             // bytes per K/V row
+    static constexpr int BLK = BK * ROW;          // bytes of one matrix block
+    static constexpr int STEP = 2 * BLK;          // one matrix of a 64-position step
+    static constexpr int NS = 4;                  // ring slots
+    static constexpr int NW = D / 16;             // wavefronts (8 or 4)
+    static constexpr int LOGR = D == 128 ? 8 : 7; // log2 of a workgroup's rows (32 per wavefront)
+    static constexpr int NT = 64 * NW;
+    static constexpr int RECO = 64 * 16 * DB;     // floats of O in a wavefront's record
+    static constexpr int REC = RECO + 64;         // and (m, l) of 32 rows
+    // 1/sqrt(hd) in log2 units, as the host computes it from ggml's float scale
+    static constexpr float C = (D == 128 ? 0.08838834764831845f : 0.125f) * kLog2e;
+};
+constexpr float PG_TAU_SUM = 256.0f;              // 2^8
+constexpr float PG_TAU = 8.0f;
 
 struct Pieces {
     uint32_t hpw_log2;                 // log2 of the query heads per workgroup
@@ -91,14 +94,17 @@ __device__ __forceinline__ int wave_max32(int x) {
 }
 
 // MM: 0 no mask, 1 a mask tensor (intervals in a.mask_rows), 2 implicit.
-// CL: the scale is exactly 1/sqrt(128) (c is a literal, see exps below).
+// CL: the scale is exactly 1/sqrt(hd) (c is a literal, see exps below).
 // QT: 0 F32 rows, 1 f16 rows, 2 F32 rows to rotate (a call whose rotated rows
 // do not fit the scratch; 14 KB of code that the others do not fetch).
-template <int QT, bool CL, int MM>
-__global__ __launch_bounds__(p128::NT) void fa_prefill128(AttnArgs a, GridMap gm, Pieces pc) {
-    using namespace p128;
-    // K steps, V steps, and half of the Q staging (160 KiB: all of a CU's LDS)
-    __shared__ __attribute__((aligned(16))) char smem[NS * 2 * STEP + (QT == 2 ? 0 : 4 * BLK)];
+template <int HD, int QT, bool CL, int MM>
+__global__ __launch_bounds__(PG<HD>::NT, 2) void fa_prefill_group(AttnArgs a, GridMap gm, Pieces pc) {
+    using P = PG<HD>;
+    constexpr int D = P::D, KS = P::KS, DB = P::DB, BK = P::BK, ROW = P::ROW, BLK = P::BLK, STEP = P::STEP,
+                  NS = P::NS, NW = P::NW, REC = P::REC;
+    // K steps, V steps, and with 8 wavefronts half of the Q staging (160 KiB, all
+    // of a CU's LDS; 64 KiB with 4)
+    __shared__ __attribute__((aligned(16))) char smem[NS * 2 * STEP + (QT == 2 || NW == 4 ? 0 : 4 * BLK)];
 
     int idx, hg, b, hk, bkv;
     gm.locate(blockIdx.x, idx, hg, b, hk, bkv);
@@ -123,25 +129,25 @@ __global__ __launch_bounds__(p128::NT) void fa_prefill128(AttnArgs a, GridMap gm
     const char* vb = (const char*)a.v + (int64_t)hk * a.v_nb2 + (int64_t)bkv * a.v_nb3;
 
     // ---- live interval of the lane's row, union over the workgroup ----------
-    // (MM = 1: 4 table entries per lane cover the workgroup's 256 rows; every
+    // (MM = 1: NW / 2 table entries per lane cover the workgroup's rows; every
     // wavefront reduces them itself, no barrier)
     int rlo = 0, rhi = a.nkv - 1;                         // the lane's row
     int lo = 0, hi = a.nkv;                               // the workgroup
     bool slow = false;
     if constexpr (MM == 1) {
         const int2* tab = a.mask_rows + (int64_t)(b % a.bm) * a.hm * a.nq;
-        int2 iv[4];
+        int2 iv[NW / 2];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < NW / 2; ++u) {
             const int i = 64 * u + lane;                  // head i / bm of the workgroup, row i % bm
-            const int hi_ = i >> (8 - pc.hpw_log2), row = min(q0 + (i & (bm - 1)), a.nq - 1);
+            const int hi_ = i >> (P::LOGR - (int)pc.hpw_log2), row = min(q0 + (i & (bm - 1)), a.nq - 1);
             iv[u] = tab[(int64_t)((hg * hpw + hi_) % a.hm) * a.nq + row];
         }
         const int2 mine = tab[(int64_t)(h % a.hm) * a.nq + qld];
         int tlo = 0x7fffffff, thi = -1;
         bool non = false;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < NW / 2; ++u) {
             non = non || iv[u].x == -2;
             if (iv[u].x >= 0 && iv[u].x <= iv[u].y) {
                 tlo = min(tlo, iv[u].x);
@@ -186,8 +192,8 @@ __global__ __launch_bounds__(p128::NT) void fa_prefill128(AttnArgs a, GridMap gm
     // touches 32 rows per instruction, and its 16 instructions of 8 wavefronts
     // kept the CU's address unit busy for ~2 us. QT 2 (rotation) needs a row's
     // pairs together and loads the operand layout.
-    constexpr int QL = QT == 2 ? 2 * KS : (QT == 1 ? KS : 2 * KS);   // 16-byte loads per lane
-    constexpr int QCH = QT == 1 ? 16 : 32;                            // 16-byte chunks per row
+    constexpr int QL = QT == 1 ? KS : 2 * KS;        // 16-byte loads per lane
+    constexpr int QCH = QT == 1 ? D / 8 : D / 4;     // 16-byte chunks per row
     floatx4 qraw[QL];
     int qpos = 0;
     {
@@ -207,17 +213,19 @@ __global__ __launch_bounds__(p128::NT) void fa_prefill128(AttnArgs a, GridMap gm
     }
 
     // ---- step loads: global -> LDS ring ----------------------------------------
-    // Instruction i (0, 1) of wavefront w fills rows [4 (w + 8 i), + 4) of the
-    // step; lane l writes LDS chunk l % 16 of row + l / 16, which holds the
-    // row's chunk (l % 16) ^ swizzle(row). Rows at or past n_kv read row
+    // Instruction i (0, 1) of wavefront w fills rows [RPI (w + NW i), + RPI) of
+    // the step; lane l writes LDS chunk l % CH of row + l / CH, which holds the
+    // row's chunk (l % CH) ^ swizzle(row). Rows at or past n_kv read row
     // n_kv - 1.
+    constexpr int CH = D / 8, RPI = 64 / CH;
+    static_assert(2 * NW * RPI == 2 * BK, "two instructions per matrix and step");
     const int nstep = (nb + 1) >> 1;
     uint32_t ldk[2], ldv[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        const int r = 4 * (wave + NW * i) + (lane >> 4);
-        ldk[i] = (uint32_t)r * (uint32_t)a.k_nb1 + ((lane & 15) ^ swz_k<D>(r)) * 16;
-        ldv[i] = (uint32_t)r * (uint32_t)a.v_nb1 + ((lane & 15) ^ swz_v<D>(r)) * 16;
+        const int r = RPI * (wave + NW * i) + lane / CH;
+        ldk[i] = (uint32_t)r * (uint32_t)a.k_nb1 + ((lane % CH) ^ swz_k<D>(r)) * 16;
+        ldv[i] = (uint32_t)r * (uint32_t)a.v_nb1 + ((lane % CH) ^ swz_v<D>(r)) * 16;
     }
     const uint32_t lds0 = lds_offset(smem);
     auto issue = [&](int u) {
@@ -227,9 +235,9 @@ __global__ __launch_bounds__(p128::NT) void fa_prefill128(AttnArgs a, GridMap gm
         const char* vst = vb + (int64_t)kv0 * a.v_nb1;
         if (kv0 + 2 * BK <= a.nkv) {
 #pragma unroll
-            for (int i = 0; i < 2; ++i) dma16(kst, ldk[i], kd + 4 * (wave + NW * i) * ROW);
+            for (int i = 0; i < 2; ++i) dma16(kst, ldk[i], kd + RPI * (wave + NW * i) * ROW);
 #pragma unroll
-            for (int i = 0; i < 2; ++i) dma16(vst, ldv[i], vd + 4 * (wave + NW * i) * ROW);
+            for (int i = 0; i < 2; ++i) dma16(vst, ldv[i], vd + RPI * (wave + NW * i) * ROW);
         } else {
             // (recomputed here rather than held across the loop; the empty asm
             // keeps it here)
@@ -238,15 +246,15 @@ __global__ __launch_bounds__(p128::NT) void fa_prefill128(AttnArgs a, GridMap gm
             const int rmax = a.nkv - 1 - kv0;   // kv0 < n_kv
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
-                const int r = 4 * (wave + NW * i) + (ln >> 4);
-                dma16(kst, (uint32_t)min(r, rmax) * (uint32_t)a.k_nb1 + ((ln & 15) ^ swz_k<D>(r)) * 16,
-                      kd + 4 * (wave + NW * i) * ROW);
+                const int r = RPI * (wave + NW * i) + ln / CH;
+                dma16(kst, (uint32_t)min(r, rmax) * (uint32_t)a.k_nb1 + ((ln % CH) ^ swz_k<D>(r)) * 16,
+                      kd + RPI * (wave + NW * i) * ROW);
             }
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
-                const int r = 4 * (wave + NW * i) + (ln >> 4);
-                dma16(vst, (uint32_t)min(r, rmax) * (uint32_t)a.v_nb1 + ((ln & 15) ^ swz_v<D>(r)) * 16,
-                      vd + 4 * (wave + NW * i) * ROW);
+                const int r = RPI * (wave + NW * i) + ln / CH;
+                dma16(vst, (uint32_t)min(r, rmax) * (uint32_t)a.v_nb1 + ((ln % CH) ^ swz_v<D>(r)) * 16,
+                      vd + RPI * (wave + NW * i) * ROW);
             }
         }
     };
@@ -278,7 +286,7 @@ __global__ __launch_bounds__(p128::NT) void fa_prefill128(AttnArgs a, GridMap gm
                 for (int e = 0; e < 8; ++e) qb[ks][e] = (_Float16)(x[e] * sg);
             }
         } else {
-            // the wavefront's 8 KiB: row r at 256 r, 16-byte chunk j at j ^ (r & 15);
+            // the wavefront's 32 rows, 16-byte chunk j of row r at j ^ (r % CH);
             // wavefronts 0-3 in ring slot 3 (filled from iteration 0 on), 4-7 past
             // the ring
             char* qs = smem + (wave < 2 ? 3 * STEP + wave * BLK
@@ -288,18 +296,18 @@ __global__ __launch_bounds__(p128::NT) void fa_prefill128(AttnArgs a, GridMap gm
             for (int u = 0; u < QL; ++u) {
                 const int r = (64 / QCH) * u + lane / QCH, j = lane % QCH;
                 if constexpr (QT == 1) {
-                    *(half8*)(qs + r * ROW + ((j ^ (r & 15)) * 16)) = __builtin_bit_cast(half8, qraw[u]) * (_Float16)sg;
+                    *(half8*)(qs + r * ROW + ((j ^ (r % CH)) * 16)) = __builtin_bit_cast(half8, qraw[u]) * (_Float16)sg;
                 } else {
                     half4 y;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) y[e] = (_Float16)(qraw[u][e] * sg);
-                    *(half4*)(qs + r * ROW + (((j >> 1) ^ (r & 15)) * 16) + (j & 1) * 8) = y;
+                    *(half4*)(qs + r * ROW + (((j >> 1) ^ (r % CH)) * 16) + (j & 1) * 8) = y;
                 }
             }
             __builtin_amdgcn_wave_barrier();   // (one wavefront's LDS accesses run in order)
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks)
-                qb[ks] = *(const half8*)(qs + nl * ROW + (((2 * ks + hh) ^ (nl & 15)) * 16));
+                qb[ks] = *(const half8*)(qs + nl * ROW + (((2 * ks + hh) ^ (nl % CH)) * 16));
         }
     }
 
@@ -393,7 +401,7 @@ __global__ __launch_bounds__(p128::NT) void fa_prefill128(AttnArgs a, GridMap gm
         for (int cc = 0; cc < 2; ++cc) {
 #pragma unroll
             for (int i = 0; i < 8; ++i)
-                p[cc][i] = (_Float16)exp2_fast(fmaf(sc[8 * cc + i], CL ? kC128 : c, nm));
+                p[cc][i] = (_Float16)exp2_fast(fmaf(sc[8 * cc + i], CL ? P::C : c, nm));
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const half2 p2 = {p[cc][2 * i], p[cc][2 * i + 1]};
@@ -423,7 +431,7 @@ __global__ __launch_bounds__(p128::NT) void fa_prefill128(AttnArgs a, GridMap gm
     // take no part in the choice)
     auto softmax = [&](const floatx16& sc, half8 (&p)[2]) {
         float ls = exps(sc, p);
-        bool up = !(ls <= TAU_SUM);
+        bool up = !(ls <= PG_TAU_SUM);
         if constexpr (MM != 0) up = (up || m == -INFINITY) && qvalid;
         if (__any(up)) {
             raise(block_max(sc));
@@ -484,7 +492,7 @@ __global__ __launch_bounds__(p128::NT) void fa_prefill128(AttnArgs a, GridMap gm
                     for (int j = 0; j < 16; ++j)
                         sa[j] = mv[j] == kF16NegInf ? -INFINITY : fmaf(f16_bits_to_f32(mv[j]), inv_c, sa[j]);
                     const float mx = block_max(sa);
-                    if (__any(mx > m + TAU && qvalid)) raise(mx);
+                    if (__any(mx > m + PG_TAU && qvalid)) raise(mx);
                     l += exps(sa, pa);
                     pv_mfma(pa, vr);
                 }
@@ -562,7 +570,7 @@ __global__ __launch_bounds__(p128::NT) void fa_prefill128(AttnArgs a, GridMap gm
             for (int a4 = 0; a4 < 4; ++a4)
                 *(floatx4*)(rec + (4 * db + a4) * 256 + 4 * lane) =
                     floatx4{o[db][4 * a4], o[db][4 * a4 + 1], o[db][4 * a4 + 2], o[db][4 * a4 + 3]};
-        if (hh == 0) *(float2*)(rec + 4096 + 2 * nl) = float2{m, lt};
+        if (hh == 0) *(float2*)(rec + P::RECO + 2 * nl) = float2{m, lt};
     }
 }
 
@@ -572,8 +580,9 @@ __global__ __launch_bounds__(p128::NT) void fa_prefill128(AttnArgs a, GridMap gm
 // workgroup then merge through LDS (SP = 1: a workgroup is the four dim
 // groups of a wavefront tile).
 template <int SP, int UP>
-__global__ __launch_bounds__(256) void fa_prefill128_combine(AttnArgs a, Pieces pc) {
-    using namespace p128;
+__global__ __launch_bounds__(256) void fa_prefill_group_combine(AttnArgs a, Pieces pc) {
+    using P = PG<128>;
+    constexpr int D = P::D, DB = P::DB, NW = P::NW, REC = P::REC;
     static_assert(SP == 1 || SP == 4, "wavefronts per tile and dims");
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -602,7 +611,7 @@ __global__ __launch_bounds__(256) void fa_prefill128_combine(AttnArgs a, Pieces 
 #pragma unroll
         for (int i = 0; i < UP; ++i) {
             const float* r = rec + min(p0 + SP * i, n - 1) * stride;
-            ml[i] = *(const float2*)(r + 4096 + 2 * nl);
+            ml[i] = *(const float2*)(r + P::RECO + 2 * nl);
 #pragma unroll
             for (int a4 = 0; a4 < 4; ++a4) v[i][a4] = *(const floatx4*)(r + (4 * db + a4) * 256 + 4 * lane);
         }
@@ -667,20 +676,20 @@ __global__ __launch_bounds__(256) void fa_prefill128_combine(AttnArgs a, Pieces 
 // Blocks per piece and pieces per tile. `len(t)` is the block count of tile t.
 // (Any mask is taken for a causal one that ends at n_kv, as voxtral's are;
 // another only balances worse. An implicit mask and the tensor that it stands
-// for so get the same pieces, and the same bits.) Time in units of a block (~0.75 us):
-// a workgroup costs its blocks plus kWg, and 256 run at once; merging costs
-// a launch and the records' traffic.
+// for so get the same pieces, and the same bits.) Time in units of a block
+// (~0.9 us): a workgroup costs its blocks plus kWg, and 256 run at once;
+// merging costs a launch and the records' traffic.
 static void choose_pieces(const AttnArgs& a, int bm, int nqt, int64_t groups, size_t ws_bytes, uint32_t& lp,
                           uint32_t& np) {
     constexpr double kWg = 4.0, kLaunch = 4.0, kRecord = 0.05;
-    const int nblk = (a.nkv + p128::BK - 1) / p128::BK;
+    const int nblk = (a.nkv + PG<128>::BK - 1) / PG<128>::BK;
     auto len = [&](int t) -> int {
         int64_t hi = a.nkv;
         if ((a.mask || a.im_causal) && a.nkv >= a.nq) {
             const int64_t q1 = (int64_t)(t + 1) * bm < a.nq ? (int64_t)(t + 1) * bm : a.nq;
             hi = q1 + (a.nkv - a.nq);
         }
-        return (int)((hi + p128::BK - 1) / p128::BK);
+        return (int)((hi + PG<128>::BK - 1) / PG<128>::BK);
     };
     lp = (uint32_t)nblk;
     np = 1;
@@ -694,7 +703,7 @@ static void choose_pieces(const AttnArgs& a, int bm, int nqt, int64_t groups, si
         const int l = ((longest + P - 1) / P + 1) & ~1;
         // pieces per tile: the kernel's own count for the longest possible tile
         const int pn = P == 1 ? 1 : (nblk + l - 1) / l;
-        const size_t need = (size_t)groups * nqt * (sizeof(int) + (size_t)pn * p128::NW * p128::REC * sizeof(float)) + 256;
+        const size_t need = (size_t)groups * nqt * (sizeof(int) + (size_t)pn * PG<128>::NW * PG<128>::REC * sizeof(float)) + 256;
         if (P > 1 && need > ws_bytes) break;
         int64_t total = 0, count = 0, recs = 0;
         for (int t = 0; t < nqt; ++t) {
@@ -719,51 +728,64 @@ static void choose_pieces(const AttnArgs& a, int bm, int nqt, int64_t groups, si
     }
 }
 
-template <int QT, bool CL>
-static void launch_p128(const AttnArgs& a, const GridMap& gm, const Pieces& pc, unsigned nwg, hipStream_t st) {
-    const dim3 grid(nwg), block(p128::NT);
-    if (a.mask) hipLaunchKernelGGL((fa_prefill128<QT, CL, 1>), grid, block, 0, st, a, gm, pc);
-    else if (a.im_causal) hipLaunchKernelGGL((fa_prefill128<QT, CL, 2>), grid, block, 0, st, a, gm, pc);
-    else hipLaunchKernelGGL((fa_prefill128<QT, CL, 0>), grid, block, 0, st, a, gm, pc);
+template <int HD, int QT, bool CL>
+static void launch_pg(const AttnArgs& a, const GridMap& gm, const Pieces& pc, unsigned nwg, hipStream_t st) {
+    const dim3 grid(nwg), block(PG<HD>::NT);
+    if (a.mask) hipLaunchKernelGGL((fa_prefill_group<HD, QT, CL, 1>), grid, block, 0, st, a, gm, pc);
+    else if (a.im_causal) hipLaunchKernelGGL((fa_prefill_group<HD, QT, CL, 2>), grid, block, 0, st, a, gm, pc);
+    else if constexpr (HD == 128) hipLaunchKernelGGL((fa_prefill_group<HD, QT, CL, 0>), grid, block, 0, st, a, gm, pc);
 }
 
-hipError_t launch_prefill128(const AttnArgs& a, hipStream_t st) {
+template <int HD>
+static hipError_t launch_group(const AttnArgs& a, hipStream_t st) {
+    using P = PG<HD>;
     if (a.mask && !a.mask_rows) return hipErrorInvalidValue;
-    if (!prefill128_takes(a) || a.nkv <= 0) return hipErrorInvalidValue;
+    if (a.nkv <= 0 || a.nq <= 0) return hipErrorInvalidValue;
+    const bool masked = a.mask || a.im_causal;
+    if (HD == 64 && (!masked || a.rope_pos)) return hipErrorInvalidValue;
     Pieces pc;
-    pc.hpw_log2 = prefill128_heads_log2(a);
-    const int hpw = 1 << pc.hpw_log2, bm = 32 * (p128::NW >> pc.hpw_log2);
+    pc.hpw_log2 = prefill_group_heads_log2(a, P::NW);
+    const int hpw = 1 << pc.hpw_log2, bm = 32 * (P::NW >> pc.hpw_log2);
     const int nqt = (a.nq + bm - 1) / bm, nhg = a.hq / hpw;
     const int64_t groups = (int64_t)nhg * a.b;
     uint32_t np = 1;
-    choose_pieces(a, bm, nqt, groups, a.ws ? a.ws_bytes : 0, pc.lp, np);
+    pc.lp = (uint32_t)(a.nkv + P::BK - 1) / P::BK;
+    if (HD == 128) choose_pieces(a, bm, nqt, groups, a.ws ? a.ws_bytes : 0, pc.lp, np);
     pc.np = DivMod::make(np);
     pc.nqt = nqt;
     pc.nhg = nhg;
     pc.count = reinterpret_cast<int*>(a.ws);
-    pc.rec = a.ws + (((size_t)groups * nqt + 63) & ~(size_t)63);
+    pc.rec = np > 1 ? a.ws + (((size_t)groups * nqt + 63) & ~(size_t)63) : nullptr;
     const int64_t nwg = groups * nqt * np;
     if (nwg <= 0 || nwg > 0x7fffffff) return hipErrorInvalidValue;
-    const bool masked = a.mask || a.im_causal;
     const GridMap gm = masked ? GridMap::make_tiles_desc((int)nwg, nqt * (int)np, nhg, a.hkv, a.b, a.bk)
                               : GridMap::make((int)nwg, nqt * (int)np, nhg, a.hkv, a.b, a.bk);
-    const bool cl = fabsf(a.scale_log2) == p128::kC128;
+    const bool cl = fabsf(a.scale_log2) == P::C;
+    const unsigned n = (unsigned)nwg;
     if (a.q_f16) {
-        if (cl) launch_p128<1, true>(a, gm, pc, (unsigned)nwg, st);
-        else launch_p128<1, false>(a, gm, pc, (unsigned)nwg, st);
-    } else if (a.rope_pos) {
-        if (cl) launch_p128<2, true>(a, gm, pc, (unsigned)nwg, st);
-        else launch_p128<2, false>(a, gm, pc, (unsigned)nwg, st);
+        if (cl) launch_pg<HD, 1, true>(a, gm, pc, n, st);
+        else launch_pg<HD, 1, false>(a, gm, pc, n, st);
+    } else if (HD == 128 && a.rope_pos) {
+        if (cl) launch_pg<128, 2, true>(a, gm, pc, n, st);
+        else launch_pg<128, 2, false>(a, gm, pc, n, st);
     } else {
-        if (cl) launch_p128<0, true>(a, gm, pc, (unsigned)nwg, st);
-        else launch_p128<0, false>(a, gm, pc, (unsigned)nwg, st);
+        if (cl) launch_pg<HD, 0, true>(a, gm, pc, n, st);
+        else launch_pg<HD, 0, false>(a, gm, pc, n, st);
     }
-    hipError_t e = hipGetLastError();
+    const hipError_t e = hipGetLastError();
     if (e != hipSuccess || np == 1) return e;
-    const unsigned nwt = (unsigned)(groups * nqt * p128::NW);
-    if (np <= 4) hipLaunchKernelGGL((fa_prefill128_combine<1, 4>), dim3(nwt), dim3(256), 0, st, a, pc);
-    else hipLaunchKernelGGL((fa_prefill128_combine<4, 4>), dim3(nwt * p128::DB), dim3(256), 0, st, a, pc);
+    if constexpr (HD == 128) {
+        const unsigned nwt = (unsigned)(groups * nqt * P::NW);
+        if (np <= 4) hipLaunchKernelGGL((fa_prefill_group_combine<1, 4>), dim3(nwt), dim3(256), 0, st, a, pc);
+        else hipLaunchKernelGGL((fa_prefill_group_combine<4, 4>), dim3(nwt * P::DB), dim3(256), 0, st, a, pc);
+    }
     return hipGetLastError();
+}
+
+hipError_t launch_prefill_group(const AttnArgs& a, int head_dim, hipStream_t st) {
+    if (head_dim == 128) return prefill_group_takes(a, 128) ? launch_group<128>(a, st) : hipErrorInvalidValue;
+    if (head_dim == 64) return launch_group<64>(a, st);
+    return hipErrorInvalidValue;
 }
 
 }  // namespace vxfa

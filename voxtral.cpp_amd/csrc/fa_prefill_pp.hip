@@ -854,12 +854,14 @@ hipError_t launch_prefill64_pp(const AttnArgs& a, const StageReq* stage, hipStre
             const hipError_t e = launch_mask_prep(a, stage, st);
             if (e != hipSuccess) return e;
         }
+        if (prefill_group_takes(a, 64)) return launch_prefill_group(a, 64, st);
         launch_pp_mm<1>(a, gm, nblk, ni, is_c8, grid, block, st);
     } else {
         if (stage) {
             const hipError_t e = launch_to_f16_kv(*stage, st);
             if (e != hipSuccess) return e;
         }
+        if (prefill_group_takes(a, 64)) return launch_prefill_group(a, 64, st);
         if (a.im_causal) launch_pp_mm<2>(a, gm, nblk, ni, is_c8, grid, block, st);
         else launch_pp_mm<0>(a, gm, nblk, ni, is_c8, grid, block, st);
     }

@@ -590,7 +590,7 @@ int run(Workspace& w, const vxfa_tensor* q, const vxfa_tensor* k, const vxfa_ten
         // hd 128 beyond the short masked prefill: the kernel whose workgroups
         // share K/V blocks among the heads of a kv group (a mask tensor needs
         // its intervals table)
-        const bool grouped = D == 128 && !pair && (!mask || mrows) && vxfa::prefill128_takes(a);
+        const bool grouped = D == 128 && !pair && (!mask || mrows) && vxfa::prefill_group_takes(a, 128);
         const bool pp = D == 64 && (!mask || mrows) && scale != 0.0f && w.tune.pp_enabled;
         if (separate) {
             // the append launch also rotates Q into scratch as f16 (else the
