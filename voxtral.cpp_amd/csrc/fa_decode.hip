@@ -40,7 +40,7 @@
 // of 32 would leave the grid short of workgroups; software pipelined: the
 // next tile's K/V loads are in flight while the current tile is computed):
 //   QK^T  v_mfma_f32_16x16x32_f16 per (16 positions, 32 dims); against F32
-//         K, v_mfma_f32_16x16x4f32 per (16 positions, 4 dims) with F32 Q.
+//         K, v_mfma_f32_4x4x1_16b_f32 per (16 positions, 4 dims) with F32 Q.
 //         The A operand holds the G query heads replicated 16/G times, so
 //         every lane gets the scores of all G heads for one position: no
 //         cross-lane dot reduction.
@@ -500,7 +500,7 @@ __device__ __forceinline__ void decode_body(const AttnArgs& a, const DecodeDivs&
     }
     __syncthreads();
     // MFMA A operands. f16 K: head (lane & 15) % G, dims 32 ks + 8 (lane / 16)
-    // .. + 7 of step ks. F32 K (v_mfma_f32_16x16x4f32, one dim per lane and
+    // .. + 7 of step ks. F32 K (v_mfma_f32_4x4x1_16b_f32, one dim per lane and
     // step): lane l takes dim (D / 4) (l / 16) + s at step s, so its D / 4
     // values of Q (and of each K row) are contiguous.
     half8 qa[KS];
@@ -539,9 +539,14 @@ __device__ __forceinline__ void decode_body(const AttnArgs& a, const DecodeDivs&
         if constexpr (KV32) {
             // F32 rows, 16-byte chunk c of row r at chunk c ^ (r % 16): the 16
             // rows of one operand read (one chunk each) fall on 16 bank groups.
-            // S^T in F32: v_mfma_f32_16x16x4f32, D / 4 steps, the products and
-            // their sums in F32 as ggml's F32 dot (the matrix pipe has time to
-            // spare in an HBM-bound kernel).
+            // S^T in F32, products and sums, as ggml's F32 dot:
+            // v_mfma_f32_4x4x1_16b_f32, whose 16 blocks of 4 heads x 4 positions
+            // are here 4 position groups x 4 quarters of the dims (block l / 4,
+            // so lane l's quarter is l / 16 and its position l % 16), D / 4 steps
+            // of 8 matrix cycles; the quarters' sums are added across the lanes.
+            // (A 16x16x4 step takes 32 cycles, three quarters of them for the
+            // group's 4 heads repeated: 1024 cycles a tile on the path from the
+            // tile's arrival to its softmax.)
 #pragma unroll
             for (int i = 0; i < NV; ++i) {
                 const int r = vrow + i * RPI, c0 = 2 * (lane % CH);
@@ -552,13 +557,20 @@ __device__ __forceinline__ void decode_body(const AttnArgs& a, const DecodeDivs&
 #pragma unroll
             for (int grp = 0; grp < NG; ++grp) {
                 const int r = 16 * grp + (lane & 15);
-                sc[grp] = floatx4{0.f, 0.f, 0.f, 0.f};
+                floatx4 acc2[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
                 for (int cq = 0; cq < D / 16; ++cq) {
                     const floatx4 kv = *(const floatx4*)(ktf + r * D + 4 * (((D / 16) * (lane >> 4) + cq) ^ (r & 15)));
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        sc[grp] = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[4 * cq + e], kv[e], sc[grp], 0, 0, 0);
+                        acc2[e & 1] = __builtin_amdgcn_mfma_f32_4x4x1f32(qf[4 * cq + e], kv[e], acc2[e & 1], 0, 0, 0);
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float x = acc2[0][i] + acc2[1][i];
+                    const int xi = __builtin_bit_cast(int, x);
+                    const auto r = __builtin_amdgcn_permlane16_swap(xi, xi, false, false);
+                    sc[grp][i] = pair32_sum(__builtin_bit_cast(float, (int)r[0]) + __builtin_bit_cast(float, (int)r[1]));
                 }
             }
         } else {
@@ -636,7 +648,7 @@ __device__ __forceinline__ void decode_body(const AttnArgs& a, const DecodeDivs&
 
     // The new row's F32 loads: with the 16-position tiles of short spans ahead
     // of the main loop, where they cost no round trip of their own (the larger
-    // tiles have no registers left for them). With its own turn among the
+    // tiles and the masked ones have no registers left for them). With its own turn among the
     // wavefronts, n_kv 435 in 8 splits: append 6.96 -> 6.14 us per layer, rope
     // + append 7.64 -> 6.73 (it was wavefront 0 of the last split's fifth tile,
     // its loads after the loop).
@@ -650,7 +662,8 @@ __device__ __forceinline__ void decode_body(const AttnArgs& a, const DecodeDivs&
             new_v[u] = vn[u];
         }
     };
-    if constexpr (!KV32 && T16) {
+    constexpr bool NEW_EARLY = T16 && !KV32 && !masked;
+    if constexpr (NEW_EARLY) {
         if (appends) load_new();
     }
 
@@ -684,7 +697,7 @@ __device__ __forceinline__ void decode_body(const AttnArgs& a, const DecodeDivs&
     if constexpr (!KV32) {
         if (appends) {
             const int pn = a.nkv - 1;
-            if constexpr (!T16) load_new();
+            if constexpr (!NEW_EARLY) load_new();
             auto cvt8 = [&](const floatx4 (&r)[2], int d0, bool rot) {
                 float x[8] = {r[0][0], r[0][1], r[0][2], r[0][3], r[1][0], r[1][1], r[1][2], r[1][3]};
                 if (rot) rope8_tab(x, d0, lds_rope, a.rope_dims);
