@@ -33,12 +33,14 @@ struct AttnArgs {
     int64_t v_nb1, v_nb2, v_nb3;   // bytes
     int64_t m_nb1, m_nb2, m_nb3;   // bytes
     int32_t nq, nkv, hq, hkv, b, bk, hm, bm;
-    int32_t q_f16;        // q element type is f16
-    int32_t kv_f32;       // k and v element type is F32 (else f16)
-    int32_t n_split;      // decode: workgroups per (batch, kv head)
-    int32_t dec_t16;      // decode, f16 K/V: 16-position tiles (short spans) instead of 32
+    uint8_t q_f16;        // q element type is f16
+    uint8_t kv_f32;       // k and v element type is F32 (else f16)
+    uint8_t dec_t16;      // decode, f16 K/V: 16-position tiles (short spans) instead of 32
+    uint8_t mask_vec;     // mask data and strides 16-byte aligned (128-bit mask loads)
     int32_t dec_chunk;    // decode with mask_rows: positions per split at most
-    int32_t mask_vec;     // mask data and strides 16-byte aligned (128-bit mask loads)
+    int32_t n_split;      // decode: workgroups per (batch, kv head)
+    uint32_t ws_bytes;    // prefill: bytes at ws
+    int32_t mask_rows_ready;   // host: mask_rows has been filled by an earlier launch of this call
     float scale_log2;     // scale * log2(e)
     // implicit causal / window mask (instead of a mask tensor): query row i
     // attends kv j iff j <= i + im_offset and, when im_window > 0,
@@ -72,9 +74,10 @@ struct AttnArgs {
     // {-2, -2}; written by a pre-pass launch into workspace scratch.
     // Batched decode with a mask tensor: the rows' live ranges (fa_decode.hip)
     int2* mask_rows;
-    int32_t mask_rows_ready;   // host: mask_rows has been filled by an earlier launch of this call
-    size_t ws_bytes;      // prefill: bytes at ws
 };
+// (one more cache line of launch arguments is one more cold scalar load before a
+// decode kernel's first tile load)
+static_assert(sizeof(AttnArgs) == 296, "launch arguments");
 
 // n / d for 0 <= n < 2^31 by a multiply-high, an add and a shift, with the
 // constants computed on the host (Granlund and Montgomery, "Division by

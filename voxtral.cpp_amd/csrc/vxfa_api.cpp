@@ -651,7 +651,7 @@ int run(Workspace& w, const vxfa_tensor* q, const vxfa_tensor* k, const vxfa_ten
                 e = vxfa::launch_prefill_pair(a, st);
             } else {
                 a.ws = reinterpret_cast<float*>(w.base + used);
-                a.ws_bytes = w.bytes - used;
+                a.ws_bytes = (uint32_t)(w.bytes - used);
                 // query-row wavefronts per workgroup (each with its KV partner
                 // wavefronts): 4 shares every staged K/V step among 128 query rows;
                 // hd 128 and small grids (fewer than 128 workgroups of 128 rows) use 2
