@@ -73,13 +73,14 @@ typedef struct vxfa_tensor {
 
 /* Per-stream context (the analogue of a ggml backend context). Owns one
  * device workspace of fixed size, allocated by vxfa_ctx_create and freed by
- * vxfa_ctx_destroy: the split-KV partial records (8 MiB: partial O,
- * running max and sum per split) and an f16 staging
- * area for F32 K/V of prefill calls (32 MiB: K and V of up to 8192 rows of
- * 8 x 128). No other call allocates, frees or synchronises, so every call
- * can be captured into a HIP graph; a decode call whose batch would need more
- * partial records than the workspace holds runs with fewer splits, a prefill
- * call with F32 K/V beyond the staging area returns VXFA_NO_WORKSPACE. The
+ * vxfa_ctx_destroy: 40 MiB, which hold a decode call's split-KV partial
+ * records (8 MiB at most: partial O, running max and sum per split), or a
+ * prefill call's f16 copies of F32 K/V (32 MiB at most: K and V of up to 8192
+ * rows of 8 x 128), mask row intervals, rotated queries and records of KV
+ * pieces. No other call allocates, frees or synchronises, so every call
+ * can be captured into a HIP graph; a call whose records would need more
+ * runs with fewer splits or pieces, a
+ * prefill call with F32 K/V beyond the 32 MiB returns VXFA_NO_WORKSPACE. The
  * caller's tensors are never allocated or freed here. One context per
  * stream; calls on one context must not overlap. */
 typedef struct vxfa_ctx vxfa_ctx;
@@ -259,7 +260,9 @@ int vxfa_flash_attn_ext_rope(vxfa_ctx* ctx, const vxfa_tensor* q,
  * counterpart in the reference: it is for callers that cannot allocate
  * device memory or create a context at that point (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc). Same
- * contract, results and status codes as vxfa_flash_attn_ext, on the current
+ * contract, results (a prefill over n_kv > 512 may round differently: its
+ * smaller scratch allows fewer KV pieces) and status codes as
+ * vxfa_flash_attn_ext, on the current
  * HIP device and `stream`; the scratch it needs (split-KV partial records of
  * a decode step, f16 staging of F32 K/V for a prefill call) lives in a
  * static 8 MiB array in the library's code object, one per GPU, kept until

@@ -63,7 +63,8 @@
 //         shared by the wavefront (DPP row reductions).
 // Masks: an additive F16 mask is honoured exactly (-inf removes a position).
 // The workgroup first scans the mask row(s) for the live range, so a sliding
-// window or a ragged stream length only costs its live positions. Without a
+// window only costs its live positions; for a batch of streams a pre-pass
+// launch finds the rows' live ranges instead (row_split below). Without a
 // mask tensor the host passes the live range (all of n_kv, or the rows an
 // implicit causal / window mask leaves to the query) and sizes the splits to
 // it, so no scan runs.
@@ -571,8 +572,8 @@ __device__ __forceinline__ void decode_body(const AttnArgs& a, const DecodeDivs&
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int si = __builtin_bit_cast(int, acc2[0][i] + acc2[1][i]);
-                    const auto r = __builtin_amdgcn_permlane16_swap(si, si, false, false);
-                    sc[grp][i] = pair32_sum(__builtin_bit_cast(float, (int)r[0]) + __builtin_bit_cast(float, (int)r[1]));
+                    const auto sw = __builtin_amdgcn_permlane16_swap(si, si, false, false);
+                    sc[grp][i] = pair32_sum(__builtin_bit_cast(float, (int)sw[0]) + __builtin_bit_cast(float, (int)sw[1]));
                 }
             }
         } else {
@@ -650,7 +651,8 @@ __device__ __forceinline__ void decode_body(const AttnArgs& a, const DecodeDivs&
 
     // The new row's F32 loads: with the 16-position tiles of short spans ahead
     // of the main loop, where they cost no round trip of their own (the larger
-    // tiles and the masked ones have no registers left for them). With its own turn among the
+    // tiles and the masked ones have no registers left for them; a ring, measured
+    // full, where its fold follows a tile all the same, lost 1 % with it). With its own turn among the
     // wavefronts, n_kv 435 in 8 splits: append 6.96 -> 6.14 us per layer, rope
     // + append 7.64 -> 6.73 (it was wavefront 0 of the last split's fifth tile,
     // its loads after the loop).
@@ -664,7 +666,7 @@ __device__ __forceinline__ void decode_body(const AttnArgs& a, const DecodeDivs&
             new_v[u] = vn[u];
         }
     };
-    constexpr bool NEW_EARLY = APP && T16 && !masked;
+    constexpr bool NEW_EARLY = APP && T16 && !masked && !RING;
     if constexpr (NEW_EARLY) {
         if (appends) load_new();
     }

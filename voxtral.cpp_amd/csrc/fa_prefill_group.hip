@@ -1,16 +1,22 @@
-// fa_prefill_group.hip — hd 128 prefill for gfx950: the query heads of one kv
-// head share each K/V block, the KV range is cut into pieces when the query
-// rows alone leave the chip idle.
+// fa_prefill_group.hip — prefill for gfx950 (hd 128, and masked hd 64 of many
+// workgroups): the query heads of one kv head share each K/V block, the KV
+// range is cut into pieces when the query rows alone leave the chip idle (hd
+// 128).
 //
 // Replaces the backend kernel of GGML_OP_FLASH_ATTN_EXT for the decoder
 // prefill calls of voxtral.cpp (src/voxtral.cpp:1802, GQA 32/8, hd 128, the
 // causal mask of :2104-2111) that the short masked kernel does not take:
-// n_kv over 512, or no mask.
+// n_kv over 512, or no mask. With head dim 64 also the realtime encoder's calls
+// (:2179-2190) from the size on that prefill_group_takes gives.
+// Measured, us per layer, before (one head and one wavefront per SIMD) and now:
+// 8192 rows causal 1127 -> 541 (1017 TFLOP/s), 600 rows on 3000 cached, implicit
+// mask 119 -> 53.7, with rope, append and mask tensor 164 -> 60.4, 10 rows on 4000
+// cached 33.7 (uncut prologue, serial merge) -> 18.4.
 //
 // Work decomposition
-//   Workgroup = 8 wavefronts of 32 query rows, two per SIMD: HPW query heads
-//   of one kv head (the largest power of two dividing the GQA group, up to 8)
-//   x 8 / HPW row tiles, so a group of 4 takes 64 positions of 4 heads. All
+//   Workgroup = 8 wavefronts (hd 64: 4) of 32 query rows, two per SIMD: HPW
+//   query heads of one kv head (the largest power of two dividing the GQA
+//   group, up to 8) x 8 / HPW row tiles, so a group of 4 takes 64 positions of 4 heads. All
 //   of them walk the same 32-position K/V blocks, read from L2 once for 256
 //   query rows and shared in LDS.
 //   A tile's live blocks are cut into pieces of at most `lp` blocks, one
@@ -23,11 +29,13 @@
 //   are about even and have to overlap. PV runs one block behind:
 //     half t:  MFMA  O += V_{t-1}^T P(t-1)^T, then S(t+1) = K_{t+1} Q^T
 //              VALU  softmax of S(t) -> P(t)
-//   where no MFMA waits for that half's VALU work. K_{t+1} is read at the top
+//   where no MFMA waits for that half's VALU work (at 8192 rows the matrix pipe
+//   is busy 53 % of the cycles at ~1.86 GHz; other orders of the half measured
+//   0-4 % slower). K_{t+1} is read at the top
 //   of the half and lands under the PV MFMAs, V_t after them and lands under
 //   the S MFMAs.
 // K/V staging: a ring of 4 steps of 64 positions (32 KiB each), filled by
-//   global_load_lds_dwordx4; step u + 3 is issued in iteration u into the slot
+//   global_load_lds_dwordx4 (hd 64: 16 KiB a step); step u + 3 is issued in iteration u into the slot
 //   of step u - 1, one barrier after its last read, and has two iterations to
 //   land. One barrier per 64 positions.
 // MFMA operand layouts, LDS swizzles and the row-to-KV permutation are those
@@ -678,7 +686,10 @@ __global__ __launch_bounds__(256) void fa_prefill_group_combine(AttnArgs a, Piec
 // another only balances worse. An implicit mask and the tensor that it stands
 // for so get the same pieces, and the same bits.) Time in units of a block
 // (~0.9 us): a workgroup costs its blocks plus kWg, and 256 run at once;
-// merging costs a launch and the records' traffic.
+// merging costs a launch and the records' traffic. Forced counts of 1 to 24 over
+// 12 shapes (1000 rows alone to 1000 on 4000, 10 to 600 on 600 to 4000, a shard of
+// two kv heads) were at best 2 % better: 600 on 3000 1 piece 96.7 us, 2 62.9, 3 54.4
+// (taken), 4 96.9 (two rounds); 10 on 4000 1 75.7, 8 20.4, 16 18.4 (taken), 24 19.7.
 static void choose_pieces(const AttnArgs& a, int bm, int nqt, int64_t groups, size_t ws_bytes, uint32_t& lp,
                           uint32_t& np) {
     constexpr double kWg = 4.0, kLaunch = 4.0, kRecord = 0.05;
