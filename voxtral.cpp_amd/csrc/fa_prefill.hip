@@ -1,10 +1,11 @@
 // fa_prefill.hip — multi-query attention (prefill) for gfx950 with f16 MFMA.
 //
-// Replaces the backend kernel of GGML_OP_FLASH_ATTN_EXT for the prefill
-// calls voxtral.cpp makes:
-//   encoder self-attention, hd 64, no mask offline    (src/voxtral.cpp:1611)
-//   decoder prefill, GQA 32/8, hd 128, causal mask     (src/voxtral.cpp:1802,
-//       mask built by fill_causal_mask :2104-2111)
+// The general kernel behind GGML_OP_FLASH_ATTN_EXT's prefill calls
+// (src/voxtral.cpp:1611, :1802): those that fa_prefill_pp.hip (hd 64),
+// fa_prefill_pair.hip (masked hd 128, n_kv <= 512) and fa_prefill_group.hip
+// (other hd 128, large masked hd 64) leave: hd 64 with scale 0, or with a
+// rotary embedding whose rotated rows do not fit the scratch; hd 128 with few
+// rows in GQA groups of 1 or 2; a mask tensor whose interval table does not fit.
 //
 // Work decomposition
 //   One workgroup per (block of BM = 32 * NQW query rows, query head, batch)
