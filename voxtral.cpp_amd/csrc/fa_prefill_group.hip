@@ -47,6 +47,12 @@
 // wholly live for a wavefront's rows get their dead scores set to -inf. A
 // workgroup with a row that is no interval (finite values, holes) reads the
 // mask per block and skips the blocks that are dead for its rows.
+// A block that is dead for all 32 rows of a wavefront (the second of a step at
+// the end of an odd walk, a part of the union that only other rows attend)
+// takes a block of zeros for V, so an infinity or NaN at positions that the
+// mask removes from those rows cannot reach them as 0 x V. (8192 rows causal
+// 544 -> 550 us, the realtime encoder's layer 34.8 -> 35.4, with no mask 82.2 ->
+// 79.9 at 2000 rows.)
 #include "fa_common.h"
 
 #include <type_traits>
@@ -111,8 +117,11 @@ __global__ __launch_bounds__(PG<HD>::NT, 2) void fa_prefill_group(AttnArgs a, Gr
     constexpr int D = P::D, KS = P::KS, DB = P::DB, BK = P::BK, ROW = P::ROW, BLK = P::BLK, STEP = P::STEP,
                   NS = P::NS, NW = P::NW, REC = P::REC;
     // K steps, V steps, and with 8 wavefronts half of the Q staging (160 KiB, all
-    // of a CU's LDS; 64 KiB with 4)
-    __shared__ __attribute__((aligned(16))) char smem[NS * 2 * STEP + (QT == 2 || NW == 4 ? 0 : 4 * BLK)];
+    // of a CU's LDS; 68 KiB with 4). The first block past the ring is zeros from
+    // iteration 0 on: what a wavefront reads for V of a block dead for its rows.
+    constexpr bool QPAST = QT != 2 && NW == 8;            // Q staging past the ring
+    constexpr int ZERO = 2 * NS * STEP;
+    __shared__ __attribute__((aligned(16))) char smem[ZERO + (QPAST ? 4 : 1) * BLK];
 
     int idx, hg, b, hk, bkv;
     gm.locate(blockIdx.x, idx, hg, b, hk, bkv);
@@ -316,7 +325,18 @@ __global__ __launch_bounds__(PG<HD>::NT, 2) void fa_prefill_group(AttnArgs a, Gr
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks)
                 qb[ks] = *(const half8*)(qs + nl * ROW + (((2 * ks + hh) ^ (nl % CH)) * 16));
+            __builtin_amdgcn_wave_barrier();
         }
+    }
+    // the block of zeros (past the ring: by the wavefront whose rows it held)
+    if constexpr (QPAST) {
+        if (wave == 4) {
+#pragma unroll
+            for (int i = 0; i < BLK / 1024; ++i) *(half8*)(smem + ZERO + 1024 * i + 16 * lane) = half8{};
+        }
+    } else {
+        static_assert(QPAST || BLK == 16 * P::NT, "one 16-byte store per thread");
+        *(half8*)(smem + ZERO + 16 * tid) = half8{};
     }
 
     // ---- operand reads ------------------------------------------------------------
@@ -343,8 +363,9 @@ __global__ __launch_bounds__(PG<HD>::NT, 2) void fa_prefill_group(AttnArgs a, Gr
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) kr[ks] = *(const half8*)(smem + (base ^ (32 * ks)));
     };
-    auto read_v = [&](int t, half8 (&vr)[2][DB]) {
-        const int base = vbase + (t & (2 * NS - 1)) * BLK;
+    auto v_at = [&](int t) -> int { return (t & (2 * NS - 1)) * BLK; };
+    auto read_v = [&](int at, half8 (&vr)[2][DB]) {
+        const int base = vbase + at;
 #pragma unroll
         for (int cc = 0; cc < 2; ++cc)
 #pragma unroll
@@ -383,9 +404,24 @@ __global__ __launch_bounds__(PG<HD>::NT, 2) void fa_prefill_group(AttnArgs a, Gr
         hlo = __builtin_amdgcn_readlane(rlo, 31);
         hhi = __builtin_amdgcn_readlane(rhi, 0);
     }
-    auto mask_fix = [&](floatx16& sc, int t) {
+    int dlo = 0, dhi = last;                              // MM = 2: the union of its rows' intervals
+    if constexpr (MM == 2) {
+        dlo = __builtin_amdgcn_readlane(rlo, 0);
+        dhi = __builtin_amdgcn_readlane(rhi, 31);
+    }
+    // (returns where block t's V is read: the zeros when the block is dead for all
+    // of the wavefront's rows, as P x V has to be 0 there whatever V holds)
+    auto mask_fix = [&](floatx16& sc, int t) -> int {
         const int kv0 = (bs + t) * BK;
+        int at = v_at(t);
         if (!(kv0 >= hlo && kv0 + BK - 1 <= hhi)) {
+            if constexpr (MM == 0) {
+                if (kv0 > last) at = ZERO - NS * STEP;
+            } else if constexpr (MM == 1) {
+                if (!__any(kv0 <= rhi && kv0 + BK > rlo && rlo <= rhi)) at = ZERO - NS * STEP;
+            } else {
+                if (kv0 > dhi || kv0 + BK <= dlo) at = ZERO - NS * STEP;
+            }
 #pragma unroll
             for (int j = 0; j < 16; ++j) {
                 const int kv = kv0 + pf_kv_of(hh, j);
@@ -393,6 +429,7 @@ __global__ __launch_bounds__(PG<HD>::NT, 2) void fa_prefill_group(AttnArgs a, Gr
                 else sc[j] = (kv < rlo || kv > rhi) ? -INFINITY : sc[j];
             }
         }
+        return at;
     };
 
     // ---- softmax ------------------------------------------------------------------
@@ -495,7 +532,7 @@ __global__ __launch_bounds__(PG<HD>::NT, 2) void fa_prefill_group(AttnArgs a, Gr
                     if (!__any(live && qvalid)) continue;
                     read_k(t, kr);
                     s_mfma(sa, kr);
-                    read_v(t, vr);
+                    read_v(v_at(t), vr);
 #pragma unroll
                     for (int j = 0; j < 16; ++j)
                         sa[j] = mv[j] == kF16NegInf ? -INFINITY : fmaf(f16_bits_to_f32(mv[j]), inv_c, sa[j]);
@@ -522,11 +559,11 @@ __global__ __launch_bounds__(PG<HD>::NT, 2) void fa_prefill_group(AttnArgs a, Gr
             m = block_max(sa);
             // half t: PV(t - 1), S(t + 1) and the softmax of S(t)
             auto half = [&](int t, floatx16& scur, floatx16& snext, half8 (&pcur)[2], half8 (&pprev)[2]) {
-                mask_fix(scur, t);
+                const int va = mask_fix(scur, t);
                 read_k(t + 1, kr);
                 pv_mfma(pprev, vr);
                 __builtin_amdgcn_sched_barrier(0x6);   // VALU and SALU may cross
-                read_v(t, vr);
+                read_v(va, vr);
                 s_mfma(snext, kr);
                 softmax(scur, pcur);
             };
