@@ -285,6 +285,25 @@ struct AppendArgs {
     int2* m_out;
 };
 
+// Workgroups of the append launch, grid (mx + n_new, bk): batch y's row holds its
+// share of the nmb mask blocks first, then one workgroup per new row. (Two
+// dimensions, as a launch takes fewer than 2^32 threads along x: 256 per
+// workgroup leave 2^24 - 1 of them, which new rows x batches may exceed.)
+struct AppendGrid {
+    uint32_t nmb, mx;
+    static AppendGrid make(uint32_t mask_blocks, uint32_t bk) {
+        return AppendGrid{mask_blocks, (mask_blocks + bk - 1) / bk};
+    }
+    // workgroup (x, y): its mask block (< nmb), or -1 and its new row t of batch y;
+    // false: nothing to do
+    __host__ __device__ __forceinline__ bool unit(uint32_t x, uint32_t y, int& mask_block, int& t) const {
+        t = (int)(x - mx);
+        mask_block = x < mx ? (int)(y * mx + x) : -1;
+        return x >= mx || y * mx + x < nmb;
+    }
+};
+constexpr uint32_t kMaxGridX = (1u << 24) - 1;   // workgroups of 256 threads along x
+
 // Rotary embedding as ggml_rope_ext computes it for mode 0 with
 // freq_scale 1, ext_factor 0, attn_factor 1 (the arguments voxtral.cpp
 // passes at src/voxtral.cpp:1746-1749 and :1595-1598): pair j = (x[2j],

@@ -23,15 +23,16 @@
 
 namespace vxfa {
 
-// blocks [0, nmb): four mask rows each; then one block per (new row t, batch b)
-__global__ __launch_bounds__(256) void kv_append_kernel(AppendArgs a, uint32_t nmb, DivMod nnew) {
-    if (blockIdx.x < nmb) {
+// a mask block takes four mask rows
+__global__ __launch_bounds__(256) void kv_append_kernel(AppendArgs a, AppendGrid g) {
+    int mb, t;
+    if (!g.unit(blockIdx.x, blockIdx.y, mb, t)) return;
+    if (mb >= 0) {
         const MaskRowArgs m{a.mask, a.m_nb1, a.m_nb2, a.m_nb3, a.m_n, a.m_nq, a.m_hm, a.m_rows, a.m_out};
-        mask_rows_block(m, blockIdx.x, (int)threadIdx.x);
+        mask_rows_block(m, (uint32_t)mb, (int)threadIdx.x);
         return;
     }
-    const uint32_t bx = blockIdx.x - nmb;
-    const int b = (int)nnew.div(bx), t = (int)nnew.mod(bx);
+    const int b = blockIdx.y;
     const int per = a.hkv * a.d / 8;   // 8-element chunks per matrix row
     const int perq = a.q_out ? a.hq * a.d / 8 : 0;
     // the token's rotary cos / sin per pair, shared by its heads
@@ -71,11 +72,9 @@ hipError_t launch_kv_append(const AppendArgs& a, hipStream_t st) {
     if (a.n_new <= 0 || a.bk <= 0) return hipSuccess;
     if (a.d % 8 || a.d > 256 || a.bk > 65535) return hipErrorInvalidValue;
     if (a.m_out && a.m_rows <= 0) return hipErrorInvalidValue;
-    const uint32_t nmb = a.m_out ? ((uint32_t)a.m_rows + 3) / 4 : 0;
-    const int64_t nwg = (int64_t)a.n_new * a.bk + nmb;
-    if (nwg > 0x7fffffff) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(kv_append_kernel, dim3((unsigned)nwg), dim3(256), 0, st, a, nmb,
-                       DivMod::make((uint32_t)a.n_new));
+    const AppendGrid g = AppendGrid::make(a.m_out ? ((uint32_t)a.m_rows + 3) / 4 : 0, (uint32_t)a.bk);
+    if ((int64_t)a.n_new + g.mx > kMaxGridX) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(kv_append_kernel, dim3((unsigned)a.n_new + g.mx, (unsigned)a.bk), dim3(256), 0, st, a, g);
     return hipGetLastError();
 }
 

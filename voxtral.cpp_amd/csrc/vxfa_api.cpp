@@ -614,8 +614,9 @@ int run(Workspace& w, const vxfa_tensor* q, const vxfa_tensor* k, const vxfa_ten
                     a.rope_pos = nullptr;
                 }
             }
-            const int64_t nrows = Nq * a.hm * a.bm;
-            if (mask && mrows && (grouped || pp || (pair && w.tune.pair_intervals)) && nrows < 0x7fffffff - 15) {
+            const int64_t nrows = Nq * a.hm * a.bm;   // (the table fits the workspace: a few million)
+            if (mask && mrows && (grouped || pp || (pair && w.tune.pair_intervals)) &&
+                ap.n_new + (nrows + 3) / 4 <= (int64_t)vxfa::kMaxGridX) {
                 ap.mask = a.mask;
                 ap.m_nb1 = a.m_nb1; ap.m_nb2 = a.m_nb2; ap.m_nb3 = a.m_nb3;
                 ap.m_n = a.nkv; ap.m_nq = a.nq; ap.m_hm = a.hm; ap.m_rows = (int32_t)nrows;
