@@ -582,12 +582,14 @@ int run(Workspace& w, const vxfa_tensor* q, const vxfa_tensor* k, const vxfa_ten
         // hd 128 one, the short masked prefill when F32 K/V are staged): the
         // live interval of each mask row (8 bytes a row), after the staged K/V
         int2* mrows = nullptr;
-        if (mask) {
-            const size_t need = ((size_t)(Nq * a.hm * a.bm) * sizeof(int2) + 255) & ~(size_t)255;
-            if (used + need <= w.bytes) {
-                mrows = reinterpret_cast<int2*>(w.base + used);
-                used += need;
-            }
+        constexpr int64_t kFar = (int64_t)1 << 40;   // (no workspace holds it)
+        auto table_bytes = [&](int64_t rows) { 
+            return ((size_t)(rows < kFar ? rows : kFar) * sizeof(int2) + 255) & ~(size_t)255;
+        };
+        const size_t table_max = table_bytes(Nq * Hq * B), table = mask ? table_bytes(Nq * a.hm * a.bm) : 0;
+        if (mask && used + table <= w.bytes) {
+            mrows = reinterpret_cast<int2*>(w.base + used);
+            used += table;
         }
         const bool pair = D == 128 && (mask || implicit) && Nkv <= 512 && w.tune.pair_enabled &&
                           vxfa::prefill_pair_fits(a);
@@ -656,7 +658,11 @@ int run(Workspace& w, const vxfa_tensor* q, const vxfa_tensor* k, const vxfa_ten
                 e = vxfa::launch_prefill_pair(a, st);
             } else {
                 a.ws = reinterpret_cast<float*>(w.base + used);
-                a.ws_bytes = (uint32_t)(w.bytes - used);
+                // the records' room does not depend on the mask's form: beside a table
+                // of a row per query row, head and batch, the largest there can be (calls
+                // of up to 2^18 of those rows are cut into pieces)
+                const size_t rest = (mask && mrows ? used - table : used) + table_max;
+                a.ws_bytes = rest < w.bytes ? (uint32_t)(w.bytes - rest) : 0u;
                 // query-row wavefronts per workgroup (each with its KV partner
                 // wavefronts): 4 shares every staged K/V step among 128 query rows;
                 // hd 128 and small grids (fewer than 128 workgroups of 128 rows) use 2
