@@ -260,16 +260,13 @@ int vxfa_flash_attn_ext_rope(vxfa_ctx* ctx, const vxfa_tensor* q,
  * counterpart in the reference: it is for callers that cannot allocate
  * device memory or create a context at that point (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc). Same
- * contract, results (a prefill over n_kv > 512 may round differently: its
- * smaller scratch allows fewer KV pieces) and status codes as
- * vxfa_flash_attn_ext, on the current
- * HIP device and `stream`; the scratch it needs (split-KV partial records of
- * a decode step, f16 staging of F32 K/V for a prefill call) lives in a
- * static 8 MiB array in the library's code object, one per GPU, kept until
- * the process ends. Limits: F32 K/V prefill calls whose f16 K and V exceed
- * 8 MiB return VXFA_NO_WORKSPACE; decode steps always run (with fewer
- * splits if their records would not fit, which the call shapes of voxtral
- * never reach). Every call on one GPU shares the array, so calls that
+ * contract, results (the same bits) and status codes as vxfa_flash_attn_ext,
+ * on the current HIP device and `stream`; the scratch it needs (what a
+ * context's workspace holds, above) lives in a static 40 MiB array in the
+ * library's code object, one per GPU, kept until the process ends. Limits:
+ * F32 K/V prefill calls whose f16 K and V exceed 8 MiB return
+ * VXFA_NO_WORKSPACE; decode steps always run (with fewer splits if their
+ * records would not fit, which the call shapes of voxtral never reach). Every call on one GPU shares the array, so calls that
  * overlap on one GPU race. Its messages are read with vxfa_last_error(NULL)
  * (per calling thread). */
 int vxfa_flash_attn_ext_noalloc(const vxfa_tensor* q, const vxfa_tensor* k,

@@ -82,7 +82,10 @@ struct vxfa_ctx {
 // code uses only that address, never the array's name, which on the host is
 // a stand-in symbol, not device memory. Every call on one GPU shares the
 // array: calls that overlap on one GPU (two streams, two threads) race.
-constexpr size_t kScratchBytes = (size_t)8 << 20;
+// As large as a context's workspace, so that every call is cut into the same
+// pieces as there and gives the same bits; F32 K/V are staged in 8 MiB of it.
+constexpr size_t kScratchBytes = kRecordBytes + kStageBytes;
+constexpr size_t kScratchStageBytes = (size_t)8 << 20;
 static __device__ __align__(256) float scratch[kScratchBytes / sizeof(float)];
 
 constexpr int kMaxDevices = 64;
@@ -812,7 +815,7 @@ int vxfa_flash_attn_ext_noalloc(const vxfa_tensor* q, const vxfa_tensor* k, cons
         t.read_env();
         return t;
     }();
-    Workspace w{device, static_cast<char*>(ptr), kScratchBytes, kScratchBytes, kScratchBytes, t_noalloc_err,
+    Workspace w{device, static_cast<char*>(ptr), kScratchBytes, kRecordBytes, kScratchStageBytes, t_noalloc_err,
                 sizeof(t_noalloc_err), tune};
     return run(w, q, k, v, mask, nullptr, dst, scale, max_bias, logit_softcap, stream);
 }
