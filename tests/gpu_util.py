@@ -9,6 +9,8 @@ must be intact, and the inputs the op only reads (q, k, v, mask) must still
 hold their host bytes."""
 from __future__ import annotations
 
+import os
+
 import numpy as np
 import torch
 
@@ -65,10 +67,20 @@ def new_rows(rows):
 
 
 class Runner:
-    """Owns one vxfa context on the current torch stream."""
+    """Owns one vxfa context on the current torch stream. env: route switches
+    (VXFA_*), which a context reads once, at creation."""
 
-    def __init__(self):
-        self.ctx = vxfa.Context(0)
+    def __init__(self, **env):
+        old = {k: os.environ.get(k) for k in env}
+        os.environ.update({k: str(v) for k, v in env.items()})
+        try:
+            self.ctx = vxfa.Context(0)
+        finally:
+            for k, v in old.items():
+                if v is None:
+                    del os.environ[k]
+                else:
+                    os.environ[k] = v
 
     def _dst(self, case):
         B, Nq, Hq, D = case.out_shape

@@ -1,0 +1,117 @@
+// Host check of the routes of vxfa_api.cpp (linked in, no GPU): the HIP calls a
+// run makes are stand-ins and the launchers note which one was called, so the
+// lines between kernels are held on both sides at sizes where both were timed.
+// Built and run by tests/test_routes.py.
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <string>
+
+#include "../../include/vxfa.h"
+#include "../../voxtral.cpp_amd/csrc/fa_common.h"
+
+extern "C" {
+hipError_t hipGetDeviceCount(int* n) { *n = 1; return hipSuccess; }
+hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipMalloc(void** p, size_t n) { *p = std::malloc(n); return *p ? hipSuccess : hipErrorOutOfMemory; }
+hipError_t hipFree(void* p) { std::free(p); return hipSuccess; }
+hipError_t hipDeviceSynchronize(void) { return hipSuccess; }
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* s) { *s = hipStreamCaptureStatusNone; return hipSuccess; }
+hipError_t hipGetSymbolAddress(void** p, const void*) { *p = nullptr; return hipErrorInvalidValue; }
+}
+
+static std::string g_route;
+static void note(const char* s) { g_route += (g_route.empty() ? "" : " ") + std::string(s); }
+namespace vxfa {
+hipError_t launch_decode(const AttnArgs& a, int, int, hipStream_t) { note(a.mask_rows ? "decode+rows" : "decode"); return hipSuccess; }
+hipError_t launch_prefill(const AttnArgs&, int, int, hipStream_t) { note("general"); return hipSuccess; }
+hipError_t launch_prefill64_pp(const AttnArgs&, const StageReq*, hipStream_t) { note("pipelined"); return hipSuccess; }
+hipError_t launch_prefill_pair(const AttnArgs&, hipStream_t) { note("pair"); return hipSuccess; }
+bool prefill_pair_fits(const AttnArgs&) { return true; }
+hipError_t launch_mask_prep(const AttnArgs&, const StageReq*, hipStream_t) { note("prep"); return hipSuccess; }
+hipError_t launch_to_f16_kv(const StageReq&, hipStream_t) { note("stage"); return hipSuccess; }
+hipError_t launch_zero(float*, int64_t, hipStream_t) { note("zero"); return hipSuccess; }
+hipError_t launch_kv_append(const AppendArgs&, hipStream_t) { note("append"); return hipSuccess; }
+}  // namespace vxfa
+
+static vxfa_tensor tensor(int type, int64_t n0, int64_t n1, int64_t n2, int64_t n3, size_t nb1, size_t nb2, size_t nb3) {
+    vxfa_tensor t;
+    std::memset(&t, 0, sizeof(t));
+    t.data = reinterpret_cast<void*>(0x7e0000000000ull);   // (never dereferenced)
+    t.type = type;
+    t.ne[0] = n0; t.ne[1] = n1; t.ne[2] = n2; t.ne[3] = n3;
+    t.nb[0] = type == VXFA_TYPE_F32 ? 4 : 2;
+    t.nb[1] = nb1; t.nb[2] = nb2; t.nb[3] = nb3;
+    return t;
+}
+
+enum Mask { NONE, TENSOR, CAUSAL };
+struct Call {
+    int hq, hkv, hd;
+    int64_t nq, nkv;
+    int batch;
+    Mask mask;
+    int window;
+    bool f32, rope;
+};
+static vxfa_ctx* g_ctx;
+static std::string route(const Call& c) {
+    const size_t e = c.f32 ? 4 : 2, D = c.hd;
+    vxfa_tensor q = tensor(VXFA_TYPE_F32, c.hd, c.nq, c.hq, c.batch, c.hq * D * 4, D * 4, c.nq * c.hq * D * 4);
+    vxfa_tensor k = tensor(c.f32 ? VXFA_TYPE_F32 : VXFA_TYPE_F16, c.hd, c.nkv, c.hkv, c.batch, c.hkv * D * e, D * e,
+                           c.nkv * c.hkv * D * e);
+    vxfa_tensor v = k;
+    vxfa_tensor dst = tensor(VXFA_TYPE_F32, c.hd, c.hq, c.nq, c.batch, D * 4, c.hq * D * 4, c.nq * c.hq * D * 4);
+    const int64_t bm = c.nq == 1 ? c.batch : 1;   // a decode step's streams have a row each
+    vxfa_tensor m = tensor(VXFA_TYPE_F16, c.nkv, c.nq, 1, bm, c.nkv * 2, c.nkv * c.nq * 2, c.nkv * c.nq * 2);
+    g_route.clear();
+    int rc;
+    if (c.rope) {
+        vxfa_tensor n = tensor(VXFA_TYPE_F32, c.hkv * c.hd, c.nq, 1, c.batch, c.hkv * D * 4, c.nq * c.hkv * D * 4,
+                               c.nq * c.hkv * D * 4);
+        vxfa_rope rp{reinterpret_cast<const int32_t*>(0x7e0000000000ull), c.hd, 0, 1e6f, 1.0f};
+        rc = vxfa_flash_attn_ext_rope(g_ctx, &q, &k, &v, &n, &n, &rp, c.mask == TENSOR ? &m : nullptr, &dst, 0.125f, 0.f,
+                                      0.f, nullptr);
+    } else if (c.mask == CAUSAL) {
+        vxfa_mask_desc md{VXFA_MASK_CAUSAL, c.window, c.nkv - c.nq};
+        rc = vxfa_flash_attn_ext_implicit(g_ctx, &q, &k, &v, &md, &dst, 0.125f, 0.f, 0.f, nullptr);
+    } else {
+        rc = vxfa_flash_attn_ext(g_ctx, &q, &k, &v, c.mask == TENSOR ? &m : nullptr, &dst, 0.125f, 0.f, 0.f, nullptr);
+    }
+    return rc == VXFA_OK ? g_route : "status " + std::to_string(rc);
+}
+
+int main() {
+    g_ctx = vxfa_ctx_create(0);
+    if (!g_ctx) return 1;
+    struct { Call c; const char* want; } t[] = {
+        // batched decode under a mask row per stream: {hq, hkv, hd, nq, n_kv, streams}
+        {{32, 8, 128, 1, 300, 2, TENSOR}, "decode"},
+        {{32, 8, 128, 1, 8192, 2, TENSOR}, "decode"},
+        {{32, 8, 128, 1, 1500, 4, TENSOR}, "decode"},
+        {{32, 8, 128, 1, 2048, 4, TENSOR}, "decode+rows"},
+        {{32, 8, 128, 1, 500, 8, TENSOR}, "decode"},
+        {{32, 8, 128, 1, 1000, 8, TENSOR}, "decode+rows"},
+        {{32, 8, 128, 1, 8192, 32, TENSOR}, "decode+rows"},
+        {{32, 8, 128, 1, 1000, 3, TENSOR, 0, true}, "decode"},
+        {{32, 8, 128, 1, 1500, 3, TENSOR, 0, true}, "decode+rows"},
+        {{32, 8, 128, 1, 256, 24, TENSOR, 0, true}, "decode"},
+        {{32, 8, 128, 1, 300, 16, TENSOR, 0, true}, "decode+rows"},
+        {{8, 2, 128, 1, 8192, 4, TENSOR}, "decode"},
+        {{32, 8, 128, 1, 8192, 1, TENSOR}, "decode"},
+    };
+    int bad = 0;
+    for (const auto& x : t) {
+        const std::string got = route(x.c);
+        if (got != x.want) {
+            std::printf("FAIL %d/%d hd %d nq %lld n_kv %lld batch %d mask %d window %d f32 %d rope %d: %s, not %s\n", x.c.hq,
+                        x.c.hkv, x.c.hd, (long long)x.c.nq, (long long)x.c.nkv, x.c.batch, x.c.mask, x.c.window, x.c.f32,
+                        x.c.rope, got.c_str(), x.want);
+            bad = 1;
+        }
+    }
+    vxfa_ctx_destroy(g_ctx);
+    if (!bad) std::printf("ok\n");
+    return bad;
+}

@@ -1,5 +1,6 @@
 """Batched decode with a mask tensor: the rows' live ranges found by a
-pre-pass, splits sized to each stream (fa_decode.hip). Stream lengths at the
+pre-pass and splits sized to each stream, or by a scan in every workgroup
+(fa_decode.hip). Stream lengths at the
 edges of tiles, rounds and splits, rows that are no range of zeros, appended
 rows, F32 caches and hd 64, against the exact float64 reference.
 
@@ -15,10 +16,12 @@ from oracle import oracle
 pytestmark = pytest.mark.gpu
 
 
-@pytest.fixture(scope="module")
-def runner():
+# every test with the pre-pass, and with a scan in each workgroup (what a call
+# takes by itself depends on its size)
+@pytest.fixture(scope="module", params=[1, 0], ids=["pre-pass", "scan"])
+def runner(request):
     import gpu_util
-    r = gpu_util.Runner()
+    r = gpu_util.Runner(VXFA_DECODE_ROWS=request.param)
     yield r
     r.close()
 

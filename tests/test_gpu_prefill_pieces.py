@@ -1,8 +1,6 @@
 """KV pieces of the grouped hd 128 prefill at the workspace's limit: the
 number of pieces depends on the call's sizes alone, so calls that stand for
 each other give the same bits."""
-import os
-
 import numpy as np
 import pytest
 
@@ -16,11 +14,7 @@ vx = cases.load_package().vxfa
 @pytest.fixture(scope="module")
 def runner():
     import gpu_util
-    os.environ["VXFA_PREFILL_GROUP"] = "1"   # read once, by the context's creation
-    try:
-        r = gpu_util.Runner()
-    finally:
-        del os.environ["VXFA_PREFILL_GROUP"]
+    r = gpu_util.Runner(VXFA_PREFILL_GROUP=1)
     yield r
     r.close()
 

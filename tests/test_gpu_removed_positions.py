@@ -2,8 +2,6 @@
 and NaN in K and V: the grouped prefill kernel's workgroups walk the union of
 their rows' live blocks in pairs, so they meet blocks that are dead for a
 wavefront's 32 rows, or past the last live one; none may reach an output."""
-import os
-
 import numpy as np
 import pytest
 
@@ -17,11 +15,7 @@ vx = cases.load_package().vxfa
 @pytest.fixture(scope="module")
 def runner():
     import gpu_util
-    os.environ["VXFA_PREFILL_GROUP"] = "1"   # read once, by the context's creation
-    try:
-        r = gpu_util.Runner()
-    finally:
-        del os.environ["VXFA_PREFILL_GROUP"]
+    r = gpu_util.Runner(VXFA_PREFILL_GROUP=1)
     yield r
     r.close()
 

@@ -27,8 +27,8 @@ constexpr size_t kRecordBytes = (size_t)8 << 20;        // decode records: e.g. 
 constexpr size_t kStageBytes = (size_t)32 << 20;        // F32 K and V of 8192 rows x 1024 as f16
 
 // Launch-shape overrides for tuning sweeps (VXFA_DECODE_SPLIT,
-// VXFA_PREFILL_WAVES, VXFA_PREFILL_PP, VXFA_PREFILL_PAIR), read from the
-// environment; 0 = heuristic.
+// VXFA_PREFILL_WAVES; 0 = heuristic) and route switches for tests and
+// measurements, read from the environment when a context is created.
 struct Tuning {
     int split_override = 0;
     int waves_override = 0;
@@ -40,12 +40,16 @@ struct Tuning {
     // prefill classifies its blocks from the mask itself rather than from the
     // intervals a pre-pass finds in the staging launch
     bool pair_intervals = true;
+    // VXFA_DECODE_ROWS: batched decode with a mask tensor of one head plane
+    // finds its rows' live ranges by a pre-pass always (1) or never (0)
+    int decode_rows = -1;
     void read_env() {
         if (const char* e = getenv("VXFA_DECODE_SPLIT")) split_override = atoi(e);
         if (const char* e = getenv("VXFA_PREFILL_WAVES")) waves_override = atoi(e);
         if (const char* e = getenv("VXFA_PREFILL_PP")) pp_enabled = atoi(e) != 0;
         if (const char* e = getenv("VXFA_PREFILL_PAIR")) pair_enabled = atoi(e) != 0;
         if (const char* e = getenv("VXFA_PAIR_INTERVALS")) pair_intervals = atoi(e) != 0;
+        if (const char* e = getenv("VXFA_DECODE_ROWS")) decode_rows = atoi(e) != 0;
     }
 };
 
@@ -276,6 +280,26 @@ int choose_split(int64_t pairs, int64_t nkv, bool kv_f32, bool* t16) {
     if (s > vxfa::kDecodeMaxSplit) s = vxfa::kDecodeMaxSplit;
     if (s < 1) s = 1;
     return (int)s;
+}
+
+// Whether a batched decode call with a mask row per stream finds the rows' live
+// ranges by a pre-pass launch (which costs ~2 us and a table load ahead of each
+// workgroup's first tile) rather than by a scan in every workgroup: where the
+// positions are more than one tile for each of choose_split's wavefronts, so
+// that splits sized to each stream gain more than the launch costs, and from 24
+// (batch, kv head) pairs on. Measured, us per call, scan -> pre-pass, 8 kv heads,
+// ragged streams: f16 2 streams up to 8192 rows 11.4 -> 12.6, 4 up to 1500 10.7
+// -> 12.1, 2048 15.9 -> 12.7, 8 up to 700 11.1 -> 13.0, 1000 16.1 -> 13.5, 32 up to
+// 256 17.1 -> 16.4, 8192 135 -> 118; F32 3 up to 1000 11.9 -> 14.2, 1500 16.5 ->
+// 14.7, 16 up to 256 13.8 -> 15.5, 300 18.2 -> 16.2, 24 up to 256 (as many
+// splits either way) 20.3 -> 21.2. Where the scan is kept, the pre-pass was 7 to
+// 23 % slower; where it is not, at most 5 % (24 pairs of long rows in many
+// streams of one or two kv heads) and mostly 5 to 50 % faster.
+bool rows_by_prepass(const Workspace& w, int64_t nkv, int64_t pairs, bool kv_f32, bool t16) {
+    if (w.tune.decode_rows >= 0) return w.tune.decode_rows != 0;
+    if (pairs < 24) return false;
+    // (f16: choose_split's own line between tiles of 16 and of 32)
+    return kv_f32 ? nkv > 256 && nkv * pairs > 2048 * 16 : !t16;
 }
 
 // The split count a workspace of rec_bytes can hold: pairs * S records of
@@ -513,14 +537,14 @@ int run(Workspace& w, const vxfa_tensor* q, const vxfa_tensor* k, const vxfa_ten
         // 32 splits: 10.29 -> 9.83 us)
         if (mask && B == 1 && !a.kv_f32) t16 = true;
         size_t used = 0;
-        if (mask && B > 1 && a.hm == 1 && Nkv < (1 << 30)) {
+        const int64_t pairs = B * Hkv;
+        if (mask && B > 1 && a.hm == 1 && Nkv < (1 << 30) && rows_by_prepass(w, Nkv, pairs, a.kv_f32 != 0, t16)) {
             // streams of ragged lengths (a mask row each): the rows' live ranges
             // by a pre-pass, then splits of up to `chunk` positions, about
             // 4096 workgroups in all if every stream were full: the streams'
             // lengths differ, so the splits have to be fine for the last round (32
             // streams of up to 8192 rows: 4, 8, 12 and 16 splits a stream 132, 125,
             // 120.3 and 119.8 us; with every workgroup scanning its row, 133.4)
-            const int64_t pairs = B * Hkv;
             int64_t s2 = w.tune.split_override > 0 ? w.tune.split_override : (4096 + pairs - 1) / pairs;
             if (s2 > vxfa::kDecodeMaxSplit) s2 = vxfa::kDecodeMaxSplit;
             used = ((size_t)a.bm * sizeof(int2) + 255) & ~(size_t)255;
@@ -534,8 +558,8 @@ int run(Workspace& w, const vxfa_tensor* q, const vxfa_tensor* k, const vxfa_ten
             a.dec_chunk = (int32_t)chunk;
             a.mask_rows = reinterpret_cast<int2*>(w.base);
         } else {
-            // (several head planes: each stream's workgroups scan them; the longest
-            // stream sets the time, so about 2048 workgroups in all)
+            // (each stream's workgroups scan its row, or its head planes' rows; the
+            // longest stream sets the time, so about 2048 workgroups in all)
             if (mask && B > 1) {
                 const int64_t s2 = (2048 + B * Hkv - 1) / (B * Hkv);
                 if (s2 > S) S = (int)(s2 < (Nkv + 63) / 64 ? s2 : (Nkv + 63) / 64);
