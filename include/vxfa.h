@@ -260,10 +260,12 @@ int vxfa_flash_attn_ext_rope(vxfa_ctx* ctx, const vxfa_tensor* q,
  * counterpart in the reference: it is for callers that cannot allocate
  * device memory or create a context at that point (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc). Same
- * contract, results (the same bits) and status codes as vxfa_flash_attn_ext,
+ * contract, results (the same bits, unless staged F32 K/V leave a mask
+ * tensor's row intervals no room) and status codes as vxfa_flash_attn_ext,
  * on the current HIP device and `stream`; the scratch it needs (what a
- * context's workspace holds, above) lives in a static 40 MiB array in the
- * library's code object, one per GPU, kept until the process ends. Limits:
+ * context's workspace holds, above) lives in static arrays in the library's
+ * code object (8 MiB, and 40 MiB for the records of KV pieces), one of each per
+ * GPU, kept until the process ends. Limits:
  * F32 K/V prefill calls whose f16 K and V exceed 8 MiB return
  * VXFA_NO_WORKSPACE; decode steps always run (with fewer splits if their
  * records would not fit, which the call shapes of voxtral never reach). Every call on one GPU shares the array, so calls that

@@ -32,7 +32,7 @@ struct Alloc {
     uintptr_t lo, hi;
 };
 std::vector<Alloc> g_allocs;
-alignas(256) unsigned char g_scratch_stand_in[(size_t)40 << 20];
+alignas(256) unsigned char g_scratch_stand_in[(size_t)8 << 20];
 int g_fail = 0;
 size_t g_launches = 0;
 

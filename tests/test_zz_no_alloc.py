@@ -71,6 +71,7 @@ def test_noalloc_mask_tensor_after_staging(runner):
     _same(runner, cases.encoder_case(600, 20, 64, seed=309, window=300, kv_f32=True), oracle=True)
     _same(runner, cases.encoder_case(200, 4, 64, seed=310, window=50), oracle=True)
 
+
 @pytest.mark.parametrize("kw", [dict(n=600, kv_offset=3000), dict(n=200, kv_offset=4000, hq=8, hkv=2),
                                 dict(n=64, kv_offset=2000, causal=False), dict(n=500, kv_offset=1000, kv_f32=True)])
 def test_noalloc_pieces(runner, kw):
@@ -81,8 +82,7 @@ def test_noalloc_pieces(runner, kw):
 
 def test_noalloc_rejects_staging_beyond_the_scratch(runner):
     """F32 K and V of 16384 rows x 8 x 128 need 64 MiB of f16 staging: beyond
-    the 8 MiB that the scratch gives it, the call returns VXFA_NO_WORKSPACE and
-    launches nothing."""
+    the 8 MiB scratch, the call returns VXFA_NO_WORKSPACE and launches nothing."""
     from conftest import load_package
     vx = load_package().vxfa
     c = cases.prefill_case(2, seed=308, causal=False, kv_offset=16382, kv_f32=True)

@@ -25,6 +25,7 @@
 // staging for F32 K/V of prefill calls.
 constexpr size_t kRecordBytes = (size_t)8 << 20;        // decode records: e.g. 256 (batch, kv head) pairs x 8 splits, or 8 x 64
 constexpr size_t kStageBytes = (size_t)32 << 20;        // F32 K and V of 8192 rows x 1024 as f16
+constexpr size_t kWorkspaceBytes = kRecordBytes + kStageBytes;
 
 // Launch-shape overrides for tuning sweeps (VXFA_DECODE_SPLIT,
 // VXFA_PREFILL_WAVES; 0 = heuristic) and route switches for tests and
@@ -61,6 +62,8 @@ struct Workspace {
     char* base;           // one area, 256-byte aligned: a decode call's split-KV
     size_t bytes;         // records, or a prefill call's staged K/V, mask row
                           // intervals and piece records, in that order
+    char* pieces;         // prefill piece records, where they have an area of their own (of
+                          // kWorkspaceBytes) rather than what is left at base
     size_t rec_bytes;     // of it, most that decode records take
     size_t stage_bytes;   // of it, most that staged F32 K/V take
     char* err;            // message of the last failure
@@ -70,11 +73,11 @@ struct Workspace {
 
 struct vxfa_ctx {
     int device = 0;
-    char* ws = nullptr;           // kRecordBytes + kStageBytes of device memory
+    char* ws = nullptr;           // kWorkspaceBytes of device memory
     char last_error[256] = {0};
     Tuning tune;                  // read once when the context is created
     Workspace view() {
-        return Workspace{device, ws, kRecordBytes + kStageBytes, kRecordBytes, kStageBytes, last_error,
+        return Workspace{device, ws, kWorkspaceBytes, nullptr, kRecordBytes, kStageBytes, last_error,
                          sizeof(last_error), tune};
     }
 };
@@ -86,15 +89,16 @@ struct vxfa_ctx {
 // code uses only that address, never the array's name, which on the host is
 // a stand-in symbol, not device memory. Every call on one GPU shares the
 // array: calls that overlap on one GPU (two streams, two threads) race.
-// As large as a context's workspace, so that every call is cut into the same
-// pieces as there and gives the same bits; F32 K/V are staged in 8 MiB of it.
-constexpr size_t kScratchBytes = kRecordBytes + kStageBytes;
-constexpr size_t kScratchStageBytes = (size_t)8 << 20;
+// Piece records of prefill calls have an array of their own, so that every call
+// is cut into the same pieces as with a context and gives the same bits.
+constexpr size_t kScratchBytes = (size_t)8 << 20;
 static __device__ __align__(256) float scratch[kScratchBytes / sizeof(float)];
+static __device__ __align__(256) float piece_scratch[kWorkspaceBytes / sizeof(float)];
 
 constexpr int kMaxDevices = 64;
 static std::mutex g_scratch_mu;
 static void* g_scratch_ptr[kMaxDevices] = {nullptr};
+static void* g_piece_ptr[kMaxDevices] = {nullptr};
 static thread_local char t_noalloc_err[256] = {0};   // message of this thread's last failing no-alloc call
 
 namespace {
@@ -324,7 +328,7 @@ vxfa_ctx* vxfa_ctx_create(int device) {
     c->tune.read_env();
     int prev = 0;
     (void)hipGetDevice(&prev);
-    const bool ok = hipSetDevice(device) == hipSuccess && hipMalloc(&c->ws, kRecordBytes + kStageBytes) == hipSuccess;
+    const bool ok = hipSetDevice(device) == hipSuccess && hipMalloc(&c->ws, kWorkspaceBytes) == hipSuccess;
     (void)hipSetDevice(prev);
     if (!ok) {
         delete c;
@@ -684,12 +688,12 @@ int run(Workspace& w, const vxfa_tensor* q, const vxfa_tensor* k, const vxfa_ten
                 // tiles, every live block on its own wavefront
                 e = vxfa::launch_prefill_pair(a, st);
             } else {
-                a.ws = reinterpret_cast<float*>(w.base + used);
+                a.ws = reinterpret_cast<float*>(w.pieces ? w.pieces : w.base + used);
                 // the records' room does not depend on the mask's form: beside a table
                 // of a row per query row, head and batch, the largest there can be (calls
                 // of up to 2^18 of those rows are cut into pieces)
                 const size_t rest = (mask && mrows ? used - table : used) + table_max;
-                a.ws_bytes = rest < w.bytes ? (uint32_t)(w.bytes - rest) : 0u;
+                a.ws_bytes = rest < kWorkspaceBytes ? (uint32_t)(kWorkspaceBytes - rest) : 0u;
                 // query-row wavefronts per workgroup (each with its KV partner
                 // wavefronts): 4 shares every staged K/V step among 128 query rows;
                 // hd 128 and small grids (fewer than 128 workgroups of 128 rows) use 2
@@ -808,7 +812,7 @@ int vxfa_flash_attn_ext_noalloc(const vxfa_tensor* q, const vxfa_tensor* k, cons
         snprintf(t_noalloc_err, sizeof(t_noalloc_err), "no usable current HIP device");
         return VXFA_HIP_ERROR;
     }
-    void* ptr = nullptr;
+    void *ptr = nullptr, *pieces = nullptr;
     {
         // first call on this device (the device is current): the array's
         // device address, once. hipGetSymbolAddress may load the code object,
@@ -823,8 +827,9 @@ int vxfa_flash_attn_ext_noalloc(const vxfa_tensor* q, const vxfa_tensor* k, cons
                          "the first no-alloc call on a device must be made outside stream capture");
                 return VXFA_HIP_ERROR;
             }
-            e = hipGetSymbolAddress(&g_scratch_ptr[device], HIP_SYMBOL(scratch));
-            if (e != hipSuccess || !g_scratch_ptr[device]) {
+            e = hipGetSymbolAddress(&g_piece_ptr[device], HIP_SYMBOL(piece_scratch));
+            if (e == hipSuccess) e = hipGetSymbolAddress(&g_scratch_ptr[device], HIP_SYMBOL(scratch));
+            if (e != hipSuccess || !g_scratch_ptr[device] || !g_piece_ptr[device]) {
                 g_scratch_ptr[device] = nullptr;
                 snprintf(t_noalloc_err, sizeof(t_noalloc_err), "hipGetSymbolAddress(scratch): %s",
                          hipGetErrorString(e));
@@ -832,6 +837,7 @@ int vxfa_flash_attn_ext_noalloc(const vxfa_tensor* q, const vxfa_tensor* k, cons
             }
         }
         ptr = g_scratch_ptr[device];
+        pieces = g_piece_ptr[device];
     }
     // the tuning variables, read once per process
     static const Tuning tune = [] {
@@ -839,8 +845,8 @@ int vxfa_flash_attn_ext_noalloc(const vxfa_tensor* q, const vxfa_tensor* k, cons
         t.read_env();
         return t;
     }();
-    Workspace w{device, static_cast<char*>(ptr), kScratchBytes, kRecordBytes, kScratchStageBytes, t_noalloc_err,
-                sizeof(t_noalloc_err), tune};
+    Workspace w{device, static_cast<char*>(ptr), kScratchBytes, static_cast<char*>(pieces), kScratchBytes, kScratchBytes,
+                t_noalloc_err, sizeof(t_noalloc_err), tune};
     return run(w, q, k, v, mask, nullptr, dst, scale, max_bias, logit_softcap, stream);
 }
 
