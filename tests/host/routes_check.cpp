@@ -25,7 +25,10 @@ static std::string g_route;
 static void note(const char* s) { g_route += (g_route.empty() ? "" : " ") + std::string(s); }
 namespace vxfa {
 hipError_t launch_decode(const AttnArgs& a, int, int, hipStream_t) { note(a.mask_rows ? "decode+rows" : "decode"); return hipSuccess; }
-hipError_t launch_prefill(const AttnArgs&, int, int, hipStream_t) { note("general"); return hipSuccess; }
+hipError_t launch_prefill(const AttnArgs& a, int, int, hipStream_t) {
+    note(a.n_split > 1 ? "grouped, cut" : (a.n_split == 1 ? "grouped" : "general"));
+    return hipSuccess;
+}
 hipError_t launch_prefill64_pp(const AttnArgs&, const StageReq*, hipStream_t) { note("pipelined"); return hipSuccess; }
 hipError_t launch_prefill_pair(const AttnArgs&, hipStream_t) { note("pair"); return hipSuccess; }
 bool prefill_pair_fits(const AttnArgs&) { return true; }
@@ -100,6 +103,34 @@ int main() {
         {{32, 8, 128, 1, 300, 16, TENSOR, 0, true}, "decode+rows"},
         {{8, 2, 128, 1, 8192, 4, TENSOR}, "decode"},
         {{32, 8, 128, 1, 8192, 1, TENSOR}, "decode"},
+        // hd 128 prefill: {hq, hkv, hd, nq, n_kv, batch}
+        {{32, 8, 128, 8192, 8192, 1, CAUSAL}, "grouped"},
+        {{32, 8, 128, 600, 3600, 1, CAUSAL}, "grouped, cut"},
+        {{32, 8, 128, 10, 4000, 1, CAUSAL}, "grouped, cut"},
+        {{32, 8, 128, 64, 1000, 1, CAUSAL}, "grouped, cut"},
+        {{32, 8, 128, 200, 520, 1, CAUSAL}, "general"},
+        {{32, 8, 128, 512, 600, 1, CAUSAL}, "general"},
+        {{32, 8, 128, 700, 700, 1, CAUSAL}, "general"},
+        {{32, 8, 128, 1500, 1700, 1, CAUSAL}, "grouped"},
+        {{8, 2, 128, 200, 700, 1, CAUSAL}, "grouped, cut"},
+        {{8, 2, 128, 2200, 2200, 1, CAUSAL}, "general"},
+        {{8, 8, 128, 1634, 1634, 1, CAUSAL, 373}, "general"},
+        {{32, 32, 128, 128, 520, 1, CAUSAL}, "general"},
+        {{32, 32, 128, 64, 4000, 1, CAUSAL}, "general"},
+        {{32, 8, 128, 200, 720, 1, TENSOR}, "general"},
+        {{32, 8, 128, 100, 900, 1, TENSOR}, "prep grouped, cut"},
+        {{32, 8, 128, 600, 3600, 1, TENSOR, 0, true}, "prep grouped, cut"},
+        {{32, 8, 128, 600, 3600, 1, TENSOR, 0, false, true}, "append grouped, cut"},
+        {{32, 8, 128, 300, 439, 1, CAUSAL}, "pair"},
+        {{8, 2, 128, 3000, 3000, 1, TENSOR}, "prep grouped, cut"},
+        {{32, 8, 128, 64, 520, 1, CAUSAL}, "grouped, cut"},
+        {{32, 8, 128, 512, 2200, 1, CAUSAL}, "general"},
+        {{32, 8, 128, 700, 1300, 1, CAUSAL}, "grouped, cut"},
+        {{32, 8, 128, 64, 512, 1, NONE}, "general"},
+        {{32, 8, 128, 400, 400, 1, NONE}, "general"},
+        {{32, 8, 128, 400, 400, 4, NONE}, "grouped"},
+        {{32, 8, 128, 2000, 2000, 1, NONE}, "grouped"},
+        {{32, 8, 128, 8, 3000, 1, NONE}, "grouped, cut"},
     };
     int bad = 0;
     for (const auto& x : t) {

@@ -9,8 +9,13 @@
 //   * decode: 1 <= n_split <= 64, and the split records of every (batch,
 //     kv head) pair inside one workspace allocation;
 //   * F32 staging: both f16 copies inside one allocation, disjoint;
-//   * pipelined hd 64 prefill with a mask tensor: the interval table inside
-//     one allocation and clear of the staged K/V;
+//     a batch's row ranges clear of them, their splits holding the whole row;
+//   * append: rotated query rows and the mask interval table inside one
+//     allocation, clear of each other and of staged K/V;
+//   * pipelined hd 64 and grouped prefill with a mask tensor: the interval
+//     table inside one allocation and clear of the staged K/V and the queries;
+//   * grouped prefill: piece records inside one allocation and clear of all of
+//     those, as many pieces as the walk needs;
 //   * every launch: positive sizes, non-null operands.
 // Descriptors are voxtral-shaped (decode, decoder prefill, encoder, realtime
 // encoder, batched streams) with random sizes, types, strides, alignments,
@@ -25,6 +30,7 @@
 
 #include "../../include/vxfa.h"
 #include "../../voxtral.cpp_amd/csrc/fa_common.h"
+#include "../../voxtral.cpp_amd/csrc/fa_prefill_route.h"
 
 // ---- host stand-ins for the HIP runtime --------------------------------------
 namespace {
@@ -33,6 +39,7 @@ struct Alloc {
 };
 std::vector<Alloc> g_allocs;
 alignas(256) unsigned char g_scratch_stand_in[(size_t)8 << 20];
+alignas(256) unsigned char g_pieces_stand_in[(size_t)40 << 20];   // the no-alloc piece records' array
 int g_fail = 0;
 size_t g_launches = 0;
 
@@ -46,8 +53,17 @@ bool inside_one(const void* p, size_t bytes) {
         if (a >= r.lo && a + bytes <= r.hi) return true;
     return false;
 }
-// byte ranges written by the last F32 staging launch (cleared per call)
-uintptr_t g_stage_lo = 0, g_stage_hi = 0;
+// byte ranges written by the last F32 staging launch and, rotated query rows, by
+// the append launch (cleared per call)
+uintptr_t g_stage_lo = 0, g_stage_hi = 0, g_q_lo = 0, g_q_hi = 0;
+void overlap(const void* p, size_t bytes, const char* what) {
+    const uintptr_t lo = reinterpret_cast<uintptr_t>(p);
+    if ((g_stage_hi > g_stage_lo && lo < g_stage_hi && g_stage_lo < lo + bytes) ||
+        (g_q_hi > g_q_lo && lo < g_q_hi && g_q_lo < lo + bytes)) {
+        std::printf("%s: ", what);
+        fail("overlaps the staged K/V or the rotated queries");
+    }
+}
 }  // namespace
 
 extern "C" {
@@ -77,12 +93,14 @@ hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* s) {
     *s = hipStreamCaptureStatusNone;
     return hipSuccess;
 }
-hipError_t hipGetSymbolAddress(void** p, const void*) {
-    *p = g_scratch_stand_in;
-    const uintptr_t lo = reinterpret_cast<uintptr_t>(g_scratch_stand_in);
+hipError_t hipGetSymbolAddress(void** p, const void* symbol) {
+    static const void* const pieces = symbol;   // (looked up first)
+    unsigned char* const at = symbol == pieces ? g_pieces_stand_in : g_scratch_stand_in;
+    *p = at;
+    const uintptr_t lo = reinterpret_cast<uintptr_t>(at);
     bool known = false;
     for (const Alloc& r : g_allocs) known = known || r.lo == lo;
-    if (!known) g_allocs.push_back({lo, lo + sizeof(g_scratch_stand_in)});
+    if (!known) g_allocs.push_back({lo, lo + (symbol == pieces ? sizeof(g_pieces_stand_in) : sizeof(g_scratch_stand_in))});
     return hipSuccess;
 }
 }
@@ -113,22 +131,48 @@ hipError_t launch_decode(const AttnArgs& a, int D, int G, hipStream_t) {
     common(a);
     if (a.n_split < 1 || a.n_split > kDecodeMaxSplit) fail("n_split out of range");
     if (G != a.hq / a.hkv) fail("group");
-    if (a.n_split > 1) {
-        const size_t bytes = (size_t)a.b * a.hkv * a.n_split * dec_record_floats(D, G) * sizeof(float);
-        if (!a.ws || !inside_one(a.ws, bytes)) fail("decode records outside the workspace");
+    const size_t bytes = (size_t)a.b * a.hkv * a.n_split * dec_record_floats(D, G) * sizeof(float);
+    if (a.n_split > 1 && (!a.ws || !inside_one(a.ws, bytes))) fail("decode records outside the workspace");
+    if (a.mask_rows) {
+        // a batch's row ranges: one head plane, ahead of the records, n_split
+        // splits of dec_chunk positions (whole rounds) hold the whole row
+        const size_t table = (size_t)a.bm * 8;
+        if (!a.mask || a.hm != 1 || !inside_one(a.mask_rows, table)) fail("row ranges");
+        const uintptr_t t = reinterpret_cast<uintptr_t>(a.mask_rows), r = reinterpret_cast<uintptr_t>(a.ws);
+        if (a.n_split > 1 && r < t + table && t < r + bytes) fail("row ranges overlap the decode records");
+        const int round = kDecodeWaves * (a.dec_t16 || a.kv_f32 ? 16 : 32);
+        if (a.dec_chunk < 1 || a.dec_chunk % round || (int64_t)a.dec_chunk * a.n_split < a.nkv) fail("dec_chunk");
     }
-    return hipSuccess;
-}
-hipError_t launch_prefill(const AttnArgs& a, int, int, hipStream_t) {
-    common(a);
     return hipSuccess;
 }
 void check_mask_table(const AttnArgs& a) {
     const size_t bytes = (size_t)a.nq * a.hm * a.bm * 8;
     if (!a.mask_rows || !inside_one(a.mask_rows, bytes)) fail("mask interval table outside the workspace");
-    const uintptr_t lo = reinterpret_cast<uintptr_t>(a.mask_rows);
-    if (g_stage_hi > g_stage_lo && lo < g_stage_hi && g_stage_lo < lo + bytes)
-        fail("mask interval table overlaps the staged K/V");
+    overlap(a.mask_rows, bytes, "mask interval table");
+}
+void overlap_table(const AttnArgs& a, const void* p, size_t bytes, const char* what) {
+    const uintptr_t lo = reinterpret_cast<uintptr_t>(a.mask_rows), x = reinterpret_cast<uintptr_t>(p);
+    const size_t table = (size_t)a.nq * a.hm * a.bm * 8;
+    if (x < lo + table && lo < x + bytes) {
+        std::printf("%s: ", what);
+        fail("overlaps the mask interval table");
+    }
+}
+hipError_t launch_prefill(const AttnArgs& a, int hd, int, hipStream_t) {
+    common(a);
+    if (a.n_split == 0) return hipSuccess;   // the general kernel
+    if (a.mask) check_mask_table(a);
+    if (hd != 128 || a.n_split < 0 || (int64_t)a.dec_chunk * a.n_split * 32 < a.nkv) fail("pieces do not hold the walk");
+    if (a.n_split > 1) {
+        // counts, then records of n_split pieces of every tile
+        const GroupTiles g(a);
+        const size_t tiles = (size_t)g.groups * g.n, bytes = ((tiles + 63) & ~(size_t)63) * 4 +
+                             tiles * a.n_split * kGroupWaves * kGroupRecord * sizeof(float);
+        if (bytes > a.ws_bytes || !inside_one(a.ws, a.ws_bytes)) fail("piece records outside the workspace");
+        overlap(a.ws, bytes, "piece records");
+        if (a.mask) overlap_table(a, a.ws, bytes, "piece records");
+    }
+    return hipSuccess;
 }
 hipError_t launch_mask_prep(const AttnArgs& a, const StageReq* stage, hipStream_t) {
     ++g_launches;
@@ -158,8 +202,21 @@ hipError_t launch_zero(float* p, int64_t n, hipStream_t) {
     if (!p || n <= 0) fail("zero fill");
     return hipSuccess;
 }
-hipError_t launch_kv_append(const AppendArgs&, hipStream_t) {
+hipError_t launch_kv_append(const AppendArgs& a, hipStream_t) {
     ++g_launches;
+    if (a.n_new <= 0 || a.bk <= 0 || a.pos0 < 0 || !a.k_new || !a.v_new || !a.k || !a.v) fail("append operands");
+    if (a.q_out) {   // rotated query rows
+        const size_t bytes = (size_t)a.bk * a.n_new * a.hq * a.d * 2;
+        if (!a.q || !a.rope_pos || a.hq <= 0 || !inside_one(a.q_out, bytes)) fail("rotated queries outside the workspace");
+        g_q_lo = reinterpret_cast<uintptr_t>(a.q_out);
+        g_q_hi = g_q_lo + bytes;
+    }
+    if (a.m_out) {   // mask row intervals
+        const size_t bytes = (size_t)a.m_rows * 8;
+        if (!a.mask || a.m_rows <= 0 || a.m_n <= 0 || a.m_nq <= 0 || a.m_rows % (a.m_nq * a.m_hm)) fail("append mask rows");
+        if (!inside_one(a.m_out, bytes)) fail("mask interval table outside the workspace");
+        overlap(a.m_out, bytes, "append's mask interval table");
+    }
     return hipSuccess;
 }
 }  // namespace vxfa
@@ -195,14 +252,14 @@ int main(int argc, char** argv) {
     if (!ctx) { std::printf("no context\n"); return 1; }
     int counts[8] = {0};
     for (int it = 0; it < iters; ++it) {
-        g_stage_lo = g_stage_hi = 0;
+        g_stage_lo = g_stage_hi = g_q_lo = g_q_hi = 0;
         const int64_t D = pick<int64_t>(g, {64, 128, 128, 80});
         const int64_t Hkv = pick<int64_t>(g, {1, 2, 8, 20, 32});
         const int64_t G = pick<int64_t>(g, {1, 2, 4, 3});
         const int64_t Hq = Hkv * G;
-        const int64_t B = pick<int64_t>(g, {1, 1, 2, 3});
+        const int64_t B = pick<int64_t>(g, {1, 1, 2, 3, 24});
         const int64_t Bk = (g() % 2) ? 1 : B;
-        const int64_t Nq = pick<int64_t>(g, {0, 1, 1, 2, 31, 64, 130, 439, 1500});
+        const int64_t Nq = pick<int64_t>(g, {0, 1, 1, 2, 31, 64, 130, 439, 1500, 5200});
         const int64_t Nkv = pick<int64_t>(g, {0, 1, 33, 300, 439, 1500, 8192, 16384});
         const int64_t cap = Nkv + (int64_t)(g() % 3) * 64;
         const int kvt = (g() % 3) ? VXFA_TYPE_F16 : VXFA_TYPE_F32;

@@ -17,10 +17,11 @@ pytestmark = pytest.mark.gpu
 vx = cases.load_package().vxfa
 
 
+# (hd 128 wherever it can: which kernel a call takes by itself depends on its size)
 @pytest.fixture(scope="module")
 def runner():
     import gpu_util
-    r = gpu_util.Runner()
+    r = gpu_util.Runner(VXFA_PREFILL_GROUP=1)
     yield r
     r.close()
 
@@ -129,7 +130,7 @@ def test_f32_kv(runner):
 
 
 def test_scratch_of_a_call_without_context(runner):
-    """8 MiB of scratch: fewer pieces, or none next to staged F32 K/V."""
+    """8 MiB of scratch, and the piece records' own array."""
     for kw in ({}, {"kv_f32": True}):
         c = cases.prefill_case(128, kv_offset=1800, seed=2800, name=f"no-alloc {kw}", **kw)
         print(f"[case] {c.name}", flush=True)

@@ -37,8 +37,8 @@ struct AttnArgs {
     uint8_t kv_f32;       // k and v element type is F32 (else f16)
     uint8_t dec_t16;      // decode, f16 K/V: 16-position tiles (short spans) instead of 32
     uint8_t mask_vec;     // mask data and strides 16-byte aligned (128-bit mask loads)
-    int32_t dec_chunk;    // decode with mask_rows: positions per split at most
-    int32_t n_split;      // decode: workgroups per (batch, kv head)
+    int32_t dec_chunk;    // decode with mask_rows: positions per split at most; grouped prefill: blocks per piece at most
+    int32_t n_split;      // decode: workgroups per (batch, kv head); grouped prefill: pieces per tile (0: another kernel)
     uint32_t ws_bytes;    // prefill: bytes at ws
     int32_t mask_rows_ready;   // host: mask_rows has been filled by an earlier launch of this call
     float scale_log2;     // scale * log2(e)
@@ -607,14 +607,13 @@ __device__ __forceinline__ float pair32_sum(float x) {
 // Host-side launchers (implemented in the kernel translation units).
 namespace vxfa {
 hipError_t launch_decode(const AttnArgs& a, int head_dim, int group, hipStream_t stream);
-constexpr int64_t kGroup64Min = 384;   // hd 64: workgroups from which launch_prefill_group is the better
 constexpr int kDecodeMaxSplit = 64;  // split workgroups per (batch, kv head)
 constexpr int kDecodeWaves = 4;      // wavefronts per decode workgroup
 // Floats per decode partial record: O [G][D], then m [G] and l [G], padded to
 // a multiple of 4 so every record starts 16-byte aligned.
 constexpr int dec_record_floats(int D, int G) { return G * D + ((2 * G + 3) & ~3); }
-// prefill beyond the kernels below; hd 128 with prefill_group_takes (and
-// a.mask_rows set if there is a mask tensor) goes to launch_prefill_group
+// prefill beyond the kernels below; with a.n_split > 0 (fa_prefill_route.h, hd 128)
+// the grouped kernel, else the general one
 hipError_t launch_prefill(const AttnArgs& a, int head_dim, int waves, hipStream_t stream);
 // hd 64 prefill on the pipelined kernel: no mask, an implicit mask, or a mask
 // tensor (a.mask_rows: workspace for nq * hm * bm intervals, filled first by
@@ -636,35 +635,14 @@ bool prefill_pair_fits(const AttnArgs& a);
 // Prefill with a workgroup's wavefronts (32 query rows each, of the heads of a
 // kv group) sharing K/V blocks. hd 128: no mask, an implicit mask, or a mask
 // tensor (a.mask_rows filled first); a.ws: scratch for the records of tiles
-// cut into KV pieces (any size; with less, fewer pieces). hd 64: masked calls
-// without a rotary embedding.
+// cut into a.n_split KV pieces of a.dec_chunk blocks (fa_prefill_route.h). hd 64:
+// masked calls without a rotary embedding, whole tiles.
 hipError_t launch_prefill_group(const AttnArgs& a, int head_dim, hipStream_t stream);
-// its query heads per workgroup of nw wavefronts (log2): the largest power of
-// two, up to nw, that divides the GQA group
-inline uint32_t prefill_group_heads_log2(const AttnArgs& a, int nw) {
-    uint32_t l = 0;
-    while ((2 << l) <= nw && (a.hq / a.hkv) % (2 << l) == 0) ++l;
-    return l;
-}
-// Whether the launchers take a call there. hd 128: at least half of a
-// workgroup's 8 wavefronts have rows. hd 64 (4 wavefronts, two workgroups a CU,
-// each walking its whole range): masked calls of 384 workgroups or more, which
-// the pipelined kernel (one workgroup of 128 rows and 4 KV groups a CU, ~8 us of
-// it outside the loop) runs in two rounds. Measured, us per layer, pipelined ->
-// this: 32 heads, window 750, mask tensor and F32 K/V, 1500 frames 38.3 -> 34.4;
-// implicit mask 1500 frames 26.5 -> 25.1, 4000 70.9 -> 56.2; below the line 1400
-// frames 23.7 -> 24.8, 1200 20.9 -> 23.6. A walk of 47 blocks (causal, no window,
-// 1500 frames) is slower here, 26.0 -> 29.5, at 4000 frames even; the line does
-// not look at the mask, so that a tensor and the implicit mask it equals give
-// the same bits.
-inline bool prefill_group_takes(const AttnArgs& a, int head_dim) {
-    const int nw = head_dim == 128 ? 8 : 4;
-    const uint32_t hl = prefill_group_heads_log2(a, nw);
-    if (head_dim == 128) return ((((int64_t)a.nq + 31) / 32) << hl) >= 4;
-    if (!(a.mask || a.im_causal) || a.rope_pos) return false;
-    const int64_t bm = 32 * (nw >> hl);
-    return (a.nq + bm - 1) / bm * (a.hq >> hl) * (int64_t)a.b >= kGroup64Min;
-}
+// hd 64: whether the pipelined kernel's launcher hands a call on. Masked calls of
+// 384 workgroups of this kernel or more (4 wavefronts, two workgroups a CU, each
+// walking its whole range), which the pipelined one (one workgroup of 128
+// rows and 4 KV groups a CU, ~8 us of it outside the loop) runs in two rounds.
+bool prefill_group64_takes(const AttnArgs& a);
 hipError_t launch_zero(float* dst, int64_t n, hipStream_t stream);
 hipError_t launch_kv_append(const AppendArgs& a, hipStream_t stream);
 // F32 -> f16 copies of K and V (StageReq above), one launch of their own

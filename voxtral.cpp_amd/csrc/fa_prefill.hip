@@ -3,9 +3,11 @@
 // The general kernel behind GGML_OP_FLASH_ATTN_EXT's prefill calls
 // (src/voxtral.cpp:1611, :1802): those that fa_prefill_pp.hip (hd 64),
 // fa_prefill_pair.hip (masked hd 128, n_kv <= 512) and fa_prefill_group.hip
-// (other hd 128, large masked hd 64) leave: hd 64 with scale 0, or with a
-// rotary embedding whose rotated rows do not fit the scratch; hd 128 with few
-// rows in GQA groups of 1 or 2; a mask tensor whose interval table does not fit.
+// (large hd 128 and masked hd 64) leave: hd 128 calls of middling size, for which
+// this one's split of the KV range inside a workgroup beats pieces that have
+// to be merged (fa_prefill_route.h); hd 64 with scale 0, or with a rotary
+// embedding whose rotated rows do not fit the scratch; a mask tensor whose
+// interval table does not fit.
 //
 // Work decomposition
 //   One workgroup per (block of BM = 32 * NQW query rows, query head, batch)
@@ -824,8 +826,8 @@ static hipError_t launch_pw(const AttnArgs& a, hipStream_t st) {
 // always runs 2 (8 wavefronts). hd 128: 4 or 2 with one KV partner each; with
 // a mask (tensor or implicit) always 2.
 hipError_t launch_prefill(const AttnArgs& a, int head_dim, int waves, hipStream_t st) {
+    if (a.n_split > 0) return head_dim == 128 ? launch_prefill_group(a, 128, st) : hipErrorInvalidValue;
     const int mm = a.im_causal ? 2 : (a.mask != nullptr ? 1 : 0);
-    if (head_dim == 128 && (mm != 1 || a.mask_rows) && prefill_group_takes(a, 128)) return launch_prefill_group(a, 128, st);
     if (head_dim == 64) {
         if (mm == 1) return launch_pw<64, 2, 4, 1>(a, st);
         if (mm == 2) return launch_pw<64, 2, 4, 2>(a, st);

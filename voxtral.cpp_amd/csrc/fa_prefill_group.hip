@@ -5,9 +5,10 @@
 //
 // Replaces the backend kernel of GGML_OP_FLASH_ATTN_EXT for the decoder
 // prefill calls of voxtral.cpp (src/voxtral.cpp:1802, GQA 32/8, hd 128, the
-// causal mask of :2104-2111) that the short masked kernel does not take:
-// n_kv over 512, or no mask. With head dim 64 also the realtime encoder's calls
-// (:2179-2190) from the size on that prefill_group_takes gives.
+// causal mask of :2104-2111) that the short masked kernel does not take (n_kv
+// over 512, or no mask), where it is faster than the general one
+// (prefill_group128 in fa_prefill_route.h). With head dim 64 also the realtime encoder's calls
+// (:2179-2190) of many workgroups (prefill_group64_takes).
 // Measured, us per layer, before (one head and one wavefront per SIMD) and now:
 // 8192 rows causal 1127 -> 541 (1017 TFLOP/s), 600 rows on 3000 cached, implicit
 // mask 119 -> 53.7, with rope, append and mask tensor 164 -> 60.4, 10 rows on 4000
@@ -54,6 +55,7 @@
 // 544 -> 550 us, the realtime encoder's layer 34.8 -> 35.4, with no mask 82.2 ->
 // 79.9 at 2000 rows.)
 #include "fa_common.h"
+#include "fa_prefill_route.h"
 
 #include <type_traits>
 
@@ -718,64 +720,6 @@ __global__ __launch_bounds__(256) void fa_prefill_group_combine(AttnArgs a, Piec
     }
 }
 
-// Blocks per piece and pieces per tile. `len(t)` is the block count of tile t.
-// (Any mask is taken for a causal one that ends at n_kv, as voxtral's are;
-// another only balances worse. An implicit mask and the tensor that it stands
-// for so get the same pieces, and the same bits.) Time in units of a block
-// (~0.9 us): a workgroup costs its blocks plus kWg, and 256 run at once;
-// merging costs a launch and the records' traffic. Forced counts of 1 to 24 over
-// 12 shapes (1000 rows alone to 1000 on 4000, 10 to 600 on 600 to 4000, a shard of
-// two kv heads) were at best 2 % better: 600 on 3000 1 piece 96.7 us, 2 62.9, 3 54.4
-// (taken), 4 96.9 (two rounds); 10 on 4000 1 75.7, 8 20.4, 16 18.4 (taken), 24 19.7.
-static void choose_pieces(const AttnArgs& a, int bm, int nqt, int64_t groups, size_t ws_bytes, uint32_t& lp,
-                          uint32_t& np) {
-    constexpr double kWg = 4.0, kLaunch = 4.0, kRecord = 0.05;
-    const int nblk = (a.nkv + PG<128>::BK - 1) / PG<128>::BK;
-    auto len = [&](int t) -> int {
-        int64_t hi = a.nkv;
-        if ((a.mask || a.im_causal) && a.nkv >= a.nq) {
-            const int64_t q1 = (int64_t)(t + 1) * bm < a.nq ? (int64_t)(t + 1) * bm : a.nq;
-            hi = q1 + (a.nkv - a.nq);
-        }
-        return (int)((hi + PG<128>::BK - 1) / PG<128>::BK);
-    };
-    lp = (uint32_t)nblk;
-    np = 1;
-    if (groups * nqt >= 1024) return;
-    int longest = 1;
-    for (int t = 0; t < nqt; ++t) { const int n = len(t); longest = n > longest ? n : longest; }
-    double best = 1e30;
-    static const int cand[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32, 48, 64};
-    for (int P : cand) {
-        if (P > 1 && longest < 2 * P) break;
-        const int l = ((longest + P - 1) / P + 1) & ~1;
-        // pieces per tile: the kernel's own count for the longest possible tile
-        const int pn = P == 1 ? 1 : (nblk + l - 1) / l;
-        const size_t need = (size_t)groups * nqt * (sizeof(int) + (size_t)pn * PG<128>::NW * PG<128>::REC * sizeof(float)) + 256;
-        if (P > 1 && need > ws_bytes) break;
-        int64_t total = 0, count = 0, recs = 0;
-        for (int t = 0; t < nqt; ++t) {
-            const int n = len(t), k = n > l ? (n + l - 1) / l : 1;
-            total += n;
-            count += k;
-            if (k > 1) recs += k;
-        }
-        total *= groups;
-        count *= groups;
-        recs *= groups;
-        const double rounds = (double)((count + 255) / 256);
-        const double mean = (double)total / (double)count;
-        double cost = rounds * (mean + kWg);
-        if (cost < l + kWg) cost = l + kWg;
-        if (recs) cost += kLaunch + kRecord * (double)recs;
-        if (cost < best) {
-            best = cost;
-            lp = (uint32_t)(P == 1 ? nblk : l);
-            np = (uint32_t)pn;
-        }
-    }
-}
-
 template <int HD, int QT, bool CL>
 static void launch_pg(const AttnArgs& a, const GridMap& gm, const Pieces& pc, unsigned nwg, hipStream_t st) {
     const dim3 grid(nwg), block(PG<HD>::NT);
@@ -796,14 +740,19 @@ static hipError_t launch_group(const AttnArgs& a, hipStream_t st) {
     const int hpw = 1 << pc.hpw_log2, bm = 32 * (P::NW >> pc.hpw_log2);
     const int nqt = (a.nq + bm - 1) / bm, nhg = a.hq / hpw;
     const int64_t groups = (int64_t)nhg * a.b;
-    uint32_t np = 1;
-    pc.lp = (uint32_t)(a.nkv + P::BK - 1) / P::BK;
-    if (HD == 128) choose_pieces(a, bm, nqt, groups, a.ws ? a.ws_bytes : 0, pc.lp, np);
-    pc.np = DivMod::make(np);
+    // (the kernel cuts a tile into ceil(blocks / lp) pieces: np has to hold them)
+    const int32_t np = a.n_split;
+    if (np < 1 || a.dec_chunk < 1 || (np > 1 && HD != 128) || (int64_t)a.dec_chunk * np * P::BK < a.nkv)
+        return hipErrorInvalidValue;
+    pc.lp = (uint32_t)a.dec_chunk;
+    pc.np = DivMod::make((uint32_t)np);
     pc.nqt = nqt;
     pc.nhg = nhg;
     pc.count = reinterpret_cast<int*>(a.ws);
-    pc.rec = np > 1 ? a.ws + (((size_t)groups * nqt + 63) & ~(size_t)63) : nullptr;
+    const size_t counts = ((size_t)groups * nqt + 63) & ~(size_t)63;
+    pc.rec = np > 1 ? a.ws + counts : nullptr;
+    if (np > 1 && (!a.ws || (counts + (size_t)groups * nqt * np * P::NW * P::REC) * sizeof(float) > a.ws_bytes))
+        return hipErrorInvalidValue;
     const int64_t nwg = groups * nqt * np;
     if (nwg <= 0 || nwg > 0x7fffffff) return hipErrorInvalidValue;
     const GridMap gm = masked ? GridMap::make_tiles_desc((int)nwg, nqt * (int)np, nhg, a.hkv, a.b, a.bk)
@@ -831,9 +780,17 @@ static hipError_t launch_group(const AttnArgs& a, hipStream_t st) {
 }
 
 hipError_t launch_prefill_group(const AttnArgs& a, int head_dim, hipStream_t st) {
-    if (head_dim == 128) return prefill_group_takes(a, 128) ? launch_group<128>(a, st) : hipErrorInvalidValue;
+    static_assert(PG<128>::NW == kGroupWaves && PG<128>::REC == kGroupRecord, "the plan's sizes");
+    if (head_dim == 128) return launch_group<128>(a, st);
     if (head_dim == 64) return launch_group<64>(a, st);
     return hipErrorInvalidValue;
+}
+
+bool prefill_group64_takes(const AttnArgs& a) {
+    if (!(a.mask || a.im_causal) || a.rope_pos) return false;
+    const uint32_t hl = prefill_group_heads_log2(a, PG<64>::NW);
+    const int64_t bm = 32 * (PG<64>::NW >> hl);
+    return (a.nq + bm - 1) / bm * (a.hq >> hl) * (int64_t)a.b >= 384;
 }
 
 }  // namespace vxfa

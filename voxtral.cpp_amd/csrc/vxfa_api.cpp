@@ -19,6 +19,7 @@
 
 #include "../../include/vxfa.h"
 #include "fa_common.h"
+#include "fa_prefill_route.h"
 
 // Device workspace of a context, allocated once by vxfa_ctx_create (no call
 // allocates, frees or synchronises): the split-KV partial records and f16
@@ -44,12 +45,16 @@ struct Tuning {
     // VXFA_DECODE_ROWS: batched decode with a mask tensor of one head plane
     // finds its rows' live ranges by a pre-pass always (1) or never (0)
     int decode_rows = -1;
+    // VXFA_PREFILL_GROUP: hd 128 prefill on the grouped kernel wherever it can (1)
+    // or never (0)
+    int group = -1;
     void read_env() {
         if (const char* e = getenv("VXFA_DECODE_SPLIT")) split_override = atoi(e);
         if (const char* e = getenv("VXFA_PREFILL_WAVES")) waves_override = atoi(e);
         if (const char* e = getenv("VXFA_PREFILL_PP")) pp_enabled = atoi(e) != 0;
         if (const char* e = getenv("VXFA_PREFILL_PAIR")) pair_enabled = atoi(e) != 0;
         if (const char* e = getenv("VXFA_PAIR_INTERVALS")) pair_intervals = atoi(e) != 0;
+        if (const char* e = getenv("VXFA_PREFILL_GROUP")) group = atoi(e) != 0;
         if (const char* e = getenv("VXFA_DECODE_ROWS")) decode_rows = atoi(e) != 0;
     }
 };
@@ -624,23 +629,31 @@ int run(Workspace& w, const vxfa_tensor* q, const vxfa_tensor* k, const vxfa_ten
         }
         const bool pair = D == 128 && (mask || implicit) && Nkv <= 512 && w.tune.pair_enabled &&
                           vxfa::prefill_pair_fits(a);
+        const size_t q_bytes = rope ? ((size_t)(B * Nq * Hq * D) * sizeof(_Float16) + 255) & ~(size_t)255 : 0;
+        const bool q_fits = rope && used + q_bytes <= w.bytes;
         // hd 128 beyond the short masked prefill: the kernel whose workgroups
-        // share K/V blocks among the heads of a kv group (a mask tensor needs
-        // its intervals table)
-        const bool grouped = D == 128 && !pair && (!mask || mrows) && vxfa::prefill_group_takes(a, 128);
+        // share K/V blocks among the heads of a kv group, where that is the
+        // faster one (a mask tensor needs its intervals table). The records' room
+        // does not depend on the mask's form: beside a table of a row per query row,
+        // head and batch, the largest there can be (calls of up to 2^18 of those
+        // rows are cut into pieces)
+        const size_t rest = (mask && mrows ? used - table : used) + (q_fits ? q_bytes : 0) + table_max;
+        const size_t record_bytes = rest < kWorkspaceBytes ? kWorkspaceBytes - rest : 0;
+        vxfa::GroupPlan plan{};
+        const bool grouped = D == 128 && !pair && (!mask || mrows) &&
+                             vxfa::prefill_group128(a, record_bytes, !staged && !separate, w.tune.group, plan);
         const bool pp = D == 64 && (!mask || mrows) && scale != 0.0f && w.tune.pp_enabled;
         if (separate) {
             // the append launch also rotates Q into scratch as f16 (else the
             // attention kernel rotates it in each workgroup, and hd 64 goes to
             // the general kernel), and finds the mask rows' intervals
             if (rope) {
-                const size_t need = ((size_t)(B * Nq * Hq * D) * sizeof(_Float16) + 255) & ~(size_t)255;
-                if (used + need <= w.bytes && (pair || grouped || pp)) {
+                if (q_fits && (pair || grouped || pp)) {
                     ap.q = static_cast<const float*>(q->data);
                     ap.q_nb1 = a.q_nb1; ap.q_nb2 = a.q_nb2; ap.q_nb3 = a.q_nb3;
                     ap.q_out = reinterpret_cast<_Float16*>(w.base + used);
                     ap.hq = (int32_t)Hq;
-                    used += need;
+                    used += q_bytes;
                     a.q = ap.q_out;
                     a.q_f16 = 1;
                     a.q_nb1 = Hq * D * 2; a.q_nb2 = D * 2; a.q_nb3 = Nq * Hq * D * 2;
@@ -688,12 +701,12 @@ int run(Workspace& w, const vxfa_tensor* q, const vxfa_tensor* k, const vxfa_ten
                 // tiles, every live block on its own wavefront
                 e = vxfa::launch_prefill_pair(a, st);
             } else {
-                a.ws = reinterpret_cast<float*>(w.pieces ? w.pieces : w.base + used);
-                // the records' room does not depend on the mask's form: beside a table
-                // of a row per query row, head and batch, the largest there can be (calls
-                // of up to 2^18 of those rows are cut into pieces)
-                const size_t rest = (mask && mrows ? used - table : used) + table_max;
-                a.ws_bytes = rest < kWorkspaceBytes ? (uint32_t)(kWorkspaceBytes - rest) : 0u;
+                if (grouped) {
+                    a.n_split = (int32_t)plan.np;
+                    a.dec_chunk = (int32_t)plan.lp;
+                    a.ws = reinterpret_cast<float*>(w.pieces ? w.pieces : w.base + used);
+                    a.ws_bytes = (uint32_t)record_bytes;
+                }
                 // query-row wavefronts per workgroup (each with its KV partner
                 // wavefronts): 4 shares every staged K/V step among 128 query rows;
                 // hd 128 and small grids (fewer than 128 workgroups of 128 rows) use 2
