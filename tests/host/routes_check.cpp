@@ -29,7 +29,10 @@ hipError_t launch_prefill(const AttnArgs& a, int, int, hipStream_t) {
     note(a.n_split > 1 ? "grouped, cut" : (a.n_split == 1 ? "grouped" : "general"));
     return hipSuccess;
 }
-hipError_t launch_prefill64_pp(const AttnArgs&, const StageReq*, hipStream_t) { note("pipelined"); return hipSuccess; }
+hipError_t launch_prefill64_pp(const AttnArgs& a, const StageReq*, hipStream_t) {
+    note(a.n_split > 0 ? "grouped" : "pipelined");
+    return hipSuccess;
+}
 hipError_t launch_prefill_pair(const AttnArgs&, hipStream_t) { note("pair"); return hipSuccess; }
 bool prefill_pair_fits(const AttnArgs&) { return true; }
 hipError_t launch_mask_prep(const AttnArgs&, const StageReq*, hipStream_t) { note("prep"); return hipSuccess; }
@@ -131,6 +134,22 @@ int main() {
         {{32, 8, 128, 400, 400, 4, NONE}, "grouped"},
         {{32, 8, 128, 2000, 2000, 1, NONE}, "grouped"},
         {{32, 8, 128, 8, 3000, 1, NONE}, "grouped, cut"},
+        // hd 64
+        {{20, 20, 64, 1500, 1500, 1, NONE}, "pipelined"},
+        {{32, 32, 64, 1400, 1400, 1, CAUSAL, 750}, "pipelined"},
+        {{32, 32, 64, 1500, 1500, 1, CAUSAL, 750}, "grouped"},
+        {{32, 32, 64, 1500, 1500, 1, CAUSAL}, "pipelined"},
+        {{32, 32, 64, 4000, 4000, 1, CAUSAL, 750}, "grouped"},
+        {{20, 20, 64, 4000, 4000, 1, CAUSAL}, "pipelined"},
+        {{64, 64, 64, 1500, 1500, 1, CAUSAL}, "grouped"},
+        {{32, 32, 64, 2500, 2500, 1, CAUSAL}, "grouped"},
+        {{28, 28, 64, 3000, 3000, 1, CAUSAL}, "pipelined"},
+        {{80, 80, 64, 513, 513, 1, CAUSAL}, "grouped"},
+        {{32, 32, 64, 1500, 1500, 1, TENSOR, 0, true}, "grouped"},
+        {{24, 24, 64, 2048, 2048, 1, TENSOR}, "pipelined"},
+        {{32, 32, 64, 2, 4000, 12, TENSOR}, "grouped"},
+        {{32, 32, 64, 32, 8192, 12, CAUSAL}, "pipelined"},
+        {{32, 8, 64, 1530, 1600, 1, TENSOR}, "grouped"},
     };
     int bad = 0;
     for (const auto& x : t) {

@@ -620,7 +620,8 @@ hipError_t launch_prefill(const AttnArgs& a, int head_dim, int waves, hipStream_
 // a pre-pass launch)
 // stage: F32 K/V to convert first (a.k / a.v already point at the f16
 // copies), or null; with a mask tensor the conversion and the pre-pass share
-// one launch
+// one launch. With a.n_split > 0 (fa_prefill_route.h) the grouped kernel follows
+// them instead.
 hipError_t launch_prefill64_pp(const AttnArgs& a, const StageReq* stage, hipStream_t stream);
 // the mask pre-pass: the live interval of each of the nq * hm * bm rows of
 // a.mask into a.mask_rows, in one launch with the F32 -> f16 staging of
@@ -638,11 +639,6 @@ bool prefill_pair_fits(const AttnArgs& a);
 // cut into a.n_split KV pieces of a.dec_chunk blocks (fa_prefill_route.h). hd 64:
 // masked calls without a rotary embedding, whole tiles.
 hipError_t launch_prefill_group(const AttnArgs& a, int head_dim, hipStream_t stream);
-// hd 64: whether the pipelined kernel's launcher hands a call on. Masked calls of
-// 384 workgroups of this kernel or more (4 wavefronts, two workgroups a CU, each
-// walking its whole range), which the pipelined one (one workgroup of 128
-// rows and 4 KV groups a CU, ~8 us of it outside the loop) runs in two rounds.
-bool prefill_group64_takes(const AttnArgs& a);
 hipError_t launch_zero(float* dst, int64_t n, hipStream_t stream);
 hipError_t launch_kv_append(const AppendArgs& a, hipStream_t stream);
 // F32 -> f16 copies of K and V (StageReq above), one launch of their own

@@ -8,7 +8,7 @@
 // causal mask of :2104-2111) that the short masked kernel does not take (n_kv
 // over 512, or no mask), where it is faster than the general one
 // (prefill_group128 in fa_prefill_route.h). With head dim 64 also the realtime encoder's calls
-// (:2179-2190) of many workgroups (prefill_group64_takes).
+// (:2179-2190) of many workgroups (prefill_group64).
 // Measured, us per layer, before (one head and one wavefront per SIMD) and now:
 // 8192 rows causal 1127 -> 541 (1017 TFLOP/s), 600 rows on 3000 cached, implicit
 // mask 119 -> 53.7, with rope, append and mask tensor 164 -> 60.4, 10 rows on 4000
@@ -784,13 +784,6 @@ hipError_t launch_prefill_group(const AttnArgs& a, int head_dim, hipStream_t st)
     if (head_dim == 128) return launch_group<128>(a, st);
     if (head_dim == 64) return launch_group<64>(a, st);
     return hipErrorInvalidValue;
-}
-
-bool prefill_group64_takes(const AttnArgs& a) {
-    if (!(a.mask || a.im_causal) || a.rope_pos) return false;
-    const uint32_t hl = prefill_group_heads_log2(a, PG<64>::NW);
-    const int64_t bm = 32 * (PG<64>::NW >> hl);
-    return (a.nq + bm - 1) / bm * (a.hq >> hl) * (int64_t)a.b >= 384;
 }
 
 }  // namespace vxfa

@@ -834,12 +834,6 @@ hipError_t launch_mask_prep(const AttnArgs& a, const StageReq* stage, hipStream_
     return hipGetLastError();
 }
 
-static hipError_t launch_group64(AttnArgs a, hipStream_t st) {
-    a.n_split = 1;
-    a.dec_chunk = (int32_t)(((int64_t)a.nkv + 31) / 32);
-    return launch_prefill_group(a, 64, st);
-}
-
 hipError_t launch_prefill64_pp(const AttnArgs& a, const StageReq* stage, hipStream_t st) {
     using namespace pp;
     const int nqg = (a.nq + BM - 1) / BM;
@@ -860,14 +854,14 @@ hipError_t launch_prefill64_pp(const AttnArgs& a, const StageReq* stage, hipStre
             const hipError_t e = launch_mask_prep(a, stage, st);
             if (e != hipSuccess) return e;
         }
-        if (prefill_group64_takes(a)) return launch_group64(a, st);
+        if (a.n_split > 0) return launch_prefill_group(a, 64, st);
         launch_pp_mm<1>(a, gm, nblk, ni, is_c8, grid, block, st);
     } else {
         if (stage) {
             const hipError_t e = launch_to_f16_kv(*stage, st);
             if (e != hipSuccess) return e;
         }
-        if (prefill_group64_takes(a)) return launch_group64(a, st);
+        if (a.n_split > 0) return launch_prefill_group(a, 64, st);
         if (a.im_causal) launch_pp_mm<2>(a, gm, nblk, ni, is_c8, grid, block, st);
         else launch_pp_mm<0>(a, gm, nblk, ni, is_c8, grid, block, st);
     }

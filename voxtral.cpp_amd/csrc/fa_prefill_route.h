@@ -210,4 +210,36 @@ inline bool prefill_group128(const AttnArgs& a, size_t record_bytes, bool own_pr
     return general128_us(a) > 1.04 * (grouped128_us(a, g, plan) + (a.mask && own_prep ? 4.2 : 0.0));
 }
 
+// Whether the grouped kernel takes a masked hd 64 call from the pipelined one
+// (fa_prefill_pp.hip): 4 wavefronts and no pieces, two workgroups a CU, each walking
+// its whole range, against one workgroup of 128 rows and 4 KV groups a CU, ~8 us
+// of it outside the loop, in two rounds from 257 workgroups on. From 384
+// workgroups of this kernel on, where their walks are short or so many (560, dealt
+// to the XCDs longest first; else by the walk) that the longest do not set the
+// time; a tensor's reach is not known here, so it is
+// taken for one that leaves each row a window (the realtime encoder's), unless few
+// rows on a long cache make the walks even. Measured, us per layer, pipelined ->
+// grouped, 32 heads unless said: implicit window 750, 1500 frames 26.6 -> 24.9, 4000
+// 70.5 -> 57.4; causal 1500 26.9 -> 29.6, 2000 35.7 -> 37.6, 24 heads 2000 31.2 ->
+// 36.9, 20 heads 4000 86 -> 98 (there), 24 heads 3000 56.3 ->
+// 51.8, 2500 55.1 -> 46.8, 64 heads 1500 47.4 -> 40.8 (here). Tensor:
+// window 750, 1500 frames 32.7 -> 29.4, F32 K/V 39.3 -> 35.9; causal 1500 31.8 ->
+// 34.1 (here all the same), 2000 46.7 -> 42.9, 24 heads 2048 37.6 -> 43.1 (there); 12
+// batches of 2 rows on 4000 127 -> 106, of 128 on 2000 63.9 -> 59.1.
+inline bool prefill_group64(const AttnArgs& a) {
+    constexpr int kWaves = 4;
+    if (!a.mask && !a.im_causal) return false;
+    const uint32_t hl = prefill_group_heads_log2(a, kWaves);
+    const int64_t rows = 32 * (kWaves >> hl), groups = (int64_t)(a.hq >> hl) * a.b;
+    const int64_t n = ((int64_t)a.nq + rows - 1) / rows * groups;
+    if (n < 384) return false;
+    if (n >= 560 && groups % 8 == 0) return true;
+    int64_t reach = a.nkv;
+    if (a.im_causal && a.im_window > 0 && a.im_window + rows - 1 < reach) reach = a.im_window + rows - 1;
+    const int64_t walk = (reach + 31) / 32;   // blocks of the longest
+    if (walk <= 32) return true;
+    if (!a.mask) return n >= 11 * walk;
+    return n >= 7 * walk || (a.nkv >= a.nq && n * (2 * (int64_t)a.nkv - a.nq) >= 600 * (int64_t)a.nkv);
+}
+
 }  // namespace vxfa

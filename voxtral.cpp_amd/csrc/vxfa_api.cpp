@@ -642,6 +642,8 @@ int run(Workspace& w, const vxfa_tensor* q, const vxfa_tensor* k, const vxfa_ten
         vxfa::GroupPlan plan{};
         const bool grouped = D == 128 && !pair && (!mask || mrows) &&
                              vxfa::prefill_group128(a, record_bytes, !staged && !separate, w.tune.group, plan);
+        // (scale 0 goes to the general kernel: the pipelined one folds the
+        // scale into the exponent and scores the partial block's dead rows -inf)
         const bool pp = D == 64 && (!mask || mrows) && scale != 0.0f && w.tune.pp_enabled;
         if (separate) {
             // the append launch also rotates Q into scratch as f16 (else the
@@ -675,12 +677,15 @@ int run(Workspace& w, const vxfa_tensor* q, const vxfa_tensor* k, const vxfa_ten
         }
         if (pp && !a.rope_pos) {
             a.mask_rows = mrows;
-            // (scale 0 goes to the general kernel: the pipelined one folds the
-            // scale into the exponent and scores the partial block's dead rows -inf)
             // encoder prefill: the software-pipelined hd 64 kernel, also under
             // an implicit causal / window mask or a mask tensor (the realtime
-            // encoder's window); it launches the F32 staging itself, in the mask
-            // pre-pass's launch when there is one
+            // encoder's window), or the grouped kernel after the same launches; the
+            // F32 staging is launched there, in the mask pre-pass's launch when there
+            // is one
+            if (vxfa::prefill_group64(a)) {
+                a.n_split = 1;
+                a.dec_chunk = (int32_t)((Nkv + 31) / 32);
+            }
             e = vxfa::launch_prefill64_pp(a, staged ? &stage : nullptr, st);
         } else {
             if (mask && mrows && !a.mask_rows_ready && ((pair && staged && w.tune.pair_intervals) || grouped)) {
