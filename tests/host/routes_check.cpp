@@ -150,6 +150,11 @@ int main() {
         {{32, 32, 64, 2, 4000, 12, TENSOR}, "grouped"},
         {{32, 32, 64, 32, 8192, 12, CAUSAL}, "pipelined"},
         {{32, 8, 64, 1530, 1600, 1, TENSOR}, "grouped"},
+        {{32, 32, 64, 4, 400, 1, TENSOR, 0, false, true}, "append pipelined"},
+        {{32, 32, 64, 4, 2004, 1, TENSOR, 0, false, true}, "append general"},
+        {{32, 32, 64, 200, 2200, 1, NONE, 0, false, true}, "append general"},
+        {{32, 32, 64, 700, 2200, 1, TENSOR, 0, false, true}, "append pipelined"},
+        {{32, 32, 64, 400, 2200, 1, NONE, 0, false, true}, "append pipelined"},
     };
     int bad = 0;
     for (const auto& x : t) {

@@ -6,8 +6,8 @@
 // (large hd 128 and masked hd 64) leave: hd 128 calls of middling size, for which
 // this one's split of the KV range inside a workgroup beats pieces that have
 // to be merged (fa_prefill_route.h); hd 64 with scale 0, or with a rotary
-// embedding whose rotated rows do not fit the scratch; a mask tensor whose
-// interval table does not fit.
+// embedding on a long cache or whose rotated rows do not fit the scratch; a mask
+// tensor whose interval table does not fit.
 //
 // Work decomposition
 //   One workgroup per (block of BM = 32 * NQW query rows, query head, batch)

@@ -242,4 +242,17 @@ inline bool prefill_group64(const AttnArgs& a) {
     return n >= 7 * walk || (a.nkv >= a.nq && n * (2 * (int64_t)a.nkv - a.nq) >= 600 * (int64_t)a.nkv);
 }
 
+// Whether an hd 64 call with a rotary embedding has its query rows rotated by the
+// append launch, for the pipelined or the grouped kernel; else the general kernel
+// rotates them in each workgroup, and splits a long walk over more of a
+// workgroup. Measured, us per layer, general -> pipelined, causal tensor, 32
+// heads: 4 rows on 300 18.2 -> 16.0, on 700 20.1 -> 20.7, on 2000 32.6 -> 37.9; 100 on
+// 700 24.2 -> 22.9; 200 on 400 22.0 -> 19.5, on 2000 37.2 -> 41.2; 700 on 700 47.2 -> 34.1, on 2300 1.45 times
+// as fast: from more than 256 workgroups on (128 of the unmasked form's 128 rows)
+// the general kernel runs in rounds.
+inline bool prefill_rope64(const AttnArgs& a) {
+    const int64_t rows = a.mask ? 64 : 128, n = ((int64_t)a.nq + rows - 1) / rows * a.hq * a.b;
+    return a.nkv <= (a.mask ? 800 : 900) || (a.mask ? n > 256 : n >= 128);
+}
+
 }  // namespace vxfa

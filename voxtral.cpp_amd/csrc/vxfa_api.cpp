@@ -644,7 +644,8 @@ int run(Workspace& w, const vxfa_tensor* q, const vxfa_tensor* k, const vxfa_ten
                              vxfa::prefill_group128(a, record_bytes, !staged && !separate, w.tune.group, plan);
         // (scale 0 goes to the general kernel: the pipelined one folds the
         // scale into the exponent and scores the partial block's dead rows -inf)
-        const bool pp = D == 64 && (!mask || mrows) && scale != 0.0f && w.tune.pp_enabled;
+        const bool pp = D == 64 && (!mask || mrows) && scale != 0.0f && w.tune.pp_enabled &&
+                        (!rope || vxfa::prefill_rope64(a));
         if (separate) {
             // the append launch also rotates Q into scratch as f16 (else the
             // attention kernel rotates it in each workgroup, and hd 64 goes to
