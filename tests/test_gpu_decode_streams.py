@@ -101,5 +101,6 @@ def test_append(runner):
     res = runner.run_append(c, kn, vn)
     for t, new in (("k", kn), ("v", vn)):
         c.bufs[t].reshape(3, cap, 1024)[:, -1] = cases.f16_bits(new)[:, 0]
+        assert np.array_equal(res[2][t], c.bufs[t].view(np.uint8).reshape(-1)), t
     assert res[0] == 0
     agree(res[1], c)

@@ -188,3 +188,25 @@ def test_hd64_group_and_scale(runner):
     run(runner, c)
     c.scale = cases.f32(-0.2)
     run(runner, c, rel=3e-3)
+
+
+@pytest.mark.parametrize("kind", ["holes", "planes", "batch"])
+def test_hd64_mask_forms(runner, kind):
+    """A third of the entries removed; a plane for each of two heads; two
+    batches with masks of their own."""
+    n, rng = 500, np.random.default_rng(3300)
+    m = cases.implicit_mask(n, n, 0, 130)
+    if kind == "batch":
+        c = cases.decode_case(n, hq=48, hkv=48, hd=64, batch=2, seed=3301, name="hd64 batch")
+        c.bufs.pop("q"); c.views.pop("q")
+        c.add("q", "q", cases.normal(rng, (2, n, 48, 64)), oracle.F32, *cases._batched_q(n, 48, 64, 4, 2))
+        c.add("mask", "mask", np.stack([m, cases.implicit_mask(n, n, 0)]), oracle.F16, *cases.views.mask(n, n, 1, 2))
+    else:
+        c = cases.encoder_case(n, 96, 64, seed=3302, name=f"hd64 {kind}")
+        if kind == "planes":
+            bias = rng.normal(0, 2, m.shape).astype(np.float16).view(np.uint16)
+            planes = np.stack([m, np.where(m == 0, bias, m).astype(np.uint16)])
+            c.add("mask", "mask", planes, oracle.F16, *cases.views.mask(n, n, 2, 1))
+        else:
+            cases.with_mask(c, np.where(rng.random(m.shape) < 0.3, cases.NEG_INF_F16, m).astype(np.uint16))
+    run(runner, c)

@@ -48,12 +48,16 @@ struct Tuning {
     // VXFA_PREFILL_GROUP: hd 128 prefill on the grouped kernel wherever it can (1)
     // or never (0)
     int group = -1;
+    // VXFA_ROPE_Q=0: no scratch for rotated queries, as for a call whose rows do
+    // not fit it
+    bool rope_q = true;
     void read_env() {
         if (const char* e = getenv("VXFA_DECODE_SPLIT")) split_override = atoi(e);
         if (const char* e = getenv("VXFA_PREFILL_WAVES")) waves_override = atoi(e);
         if (const char* e = getenv("VXFA_PREFILL_PP")) pp_enabled = atoi(e) != 0;
         if (const char* e = getenv("VXFA_PREFILL_PAIR")) pair_enabled = atoi(e) != 0;
         if (const char* e = getenv("VXFA_PAIR_INTERVALS")) pair_intervals = atoi(e) != 0;
+        if (const char* e = getenv("VXFA_ROPE_Q")) rope_q = atoi(e) != 0;
         if (const char* e = getenv("VXFA_PREFILL_GROUP")) group = atoi(e) != 0;
         if (const char* e = getenv("VXFA_DECODE_ROWS")) decode_rows = atoi(e) != 0;
     }
@@ -630,7 +634,7 @@ int run(Workspace& w, const vxfa_tensor* q, const vxfa_tensor* k, const vxfa_ten
         const bool pair = D == 128 && (mask || implicit) && Nkv <= 512 && w.tune.pair_enabled &&
                           vxfa::prefill_pair_fits(a);
         const size_t q_bytes = rope ? ((size_t)(B * Nq * Hq * D) * sizeof(_Float16) + 255) & ~(size_t)255 : 0;
-        const bool q_fits = rope && used + q_bytes <= w.bytes;
+        const bool q_fits = rope && used + q_bytes <= w.bytes && w.tune.rope_q;
         // hd 128 beyond the short masked prefill: the kernel whose workgroups
         // share K/V blocks among the heads of a kv group, where that is the
         // faster one (a mask tensor needs its intervals table). The records' room
