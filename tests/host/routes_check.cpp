@@ -124,6 +124,8 @@ int main() {
         {{32, 8, 128, 100, 900, 1, TENSOR}, "prep grouped, cut"},
         {{32, 8, 128, 600, 3600, 1, TENSOR, 0, true}, "prep grouped, cut"},
         {{32, 8, 128, 600, 3600, 1, TENSOR, 0, false, true}, "append grouped, cut"},
+        {{16, 4, 128, 1000, 1000, 1, TENSOR, 0, false, true}, "append grouped, cut"},
+        {{16, 4, 128, 700, 700, 1, TENSOR, 0, false, true}, "append grouped, cut"},
         {{32, 8, 128, 300, 439, 1, CAUSAL}, "pair"},
         {{8, 2, 128, 3000, 3000, 1, TENSOR}, "prep grouped, cut"},
         {{32, 8, 128, 64, 520, 1, CAUSAL}, "grouped, cut"},
