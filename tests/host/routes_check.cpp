@@ -59,7 +59,7 @@ struct Call {
     int batch;
     Mask mask;
     int window;
-    bool f32, rope;
+    bool f32, rope, append;
 };
 static vxfa_ctx* g_ctx;
 static std::string route(const Call& c) {
@@ -73,12 +73,13 @@ static std::string route(const Call& c) {
     vxfa_tensor m = tensor(VXFA_TYPE_F16, c.nkv, c.nq, 1, bm, c.nkv * 2, c.nkv * c.nq * 2, c.nkv * c.nq * 2);
     g_route.clear();
     int rc;
-    if (c.rope) {
+    if (c.rope || c.append) {
         vxfa_tensor n = tensor(VXFA_TYPE_F32, c.hkv * c.hd, c.nq, 1, c.batch, c.hkv * D * 4, c.nq * c.hkv * D * 4,
                                c.nq * c.hkv * D * 4);
         vxfa_rope rp{reinterpret_cast<const int32_t*>(0x7e0000000000ull), c.hd, 0, 1e6f, 1.0f};
-        rc = vxfa_flash_attn_ext_rope(g_ctx, &q, &k, &v, &n, &n, &rp, c.mask == TENSOR ? &m : nullptr, &dst, 0.125f, 0.f,
-                                      0.f, nullptr);
+        const vxfa_tensor* mt = c.mask == TENSOR ? &m : nullptr;
+        rc = c.rope ? vxfa_flash_attn_ext_rope(g_ctx, &q, &k, &v, &n, &n, &rp, mt, &dst, 0.125f, 0.f, 0.f, nullptr)
+                    : vxfa_flash_attn_ext_append(g_ctx, &q, &k, &v, &n, &n, mt, &dst, 0.125f, 0.f, 0.f, nullptr);
     } else if (c.mask == CAUSAL) {
         vxfa_mask_desc md{VXFA_MASK_CAUSAL, c.window, c.nkv - c.nq};
         rc = vxfa_flash_attn_ext_implicit(g_ctx, &q, &k, &v, &md, &dst, 0.125f, 0.f, 0.f, nullptr);
@@ -168,7 +169,31 @@ int main() {
             bad = 1;
         }
     }
+    // appended rows: the same kernel, and so the same bits, as appending and then
+    // attending. (The launches ahead of it are not compared.)
+    const int heads[][2] = {{32, 8}, {8, 2}, {16, 4}, {32, 32}, {8, 8}, {12, 2}};
+    int64_t calls = 0;
+    for (const auto& h : heads)
+        for (int hd : {64, 128})
+            for (int batch : {1, 3})
+                for (int64_t nq : {2, 10, 39, 64, 100, 200, 383, 512, 700, 1000, 1500, 2200})
+                    for (int64_t past = 0; past < 4000; past = past * 5 / 4 + 37)
+                        for (Mask m : {NONE, TENSOR}) {
+                            auto kernel = [](const std::string& r) {
+                                const size_t p = r.find("prep ") == 0 ? 5 : r.find("append ") == 0 ? 7 : 0;
+                                return r.substr(p);
+                            };
+                            Call c{h[0], h[1], hd, nq, past + nq, batch, m};
+                            const std::string op = route(c);
+                            c.append = true;
+                            const std::string ap = route(c);
+                            ++calls;
+                            if (kernel(op) != kernel(ap) && ++bad <= 10)
+                                std::printf("FAIL %d/%d hd %d nq %lld n_kv %lld batch %d mask %d: %s, appended %s\n", h[0], h[1],
+                                            hd, (long long)nq, (long long)(past + nq), batch, m, op.c_str(), ap.c_str());
+                        }
     vxfa_ctx_destroy(g_ctx);
+    if (calls < 3000) bad = 1;
     if (!bad) std::printf("ok\n");
-    return bad;
+    return bad != 0;
 }

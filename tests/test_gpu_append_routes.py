@@ -75,7 +75,24 @@ def test_prefill_append(runner, kind, n, n_kv, batch, hq, hkv, hd):
     k, v = new_rows(c, n, 6200 + n)
     a = _check_append(runner, c, k, v, fused=True)
     b = _check_append(runner, c, k, v, fused=False)
-    assert np.abs(a - b).max() <= 2e-3   # (a mask tensor alone may take the other kernel)
+    assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+@pytest.mark.parametrize("kind,n,n_kv,batch,hq,hkv", [("causal", 100, 654, 1, 32, 8), ("causal", 200, 929, 1, 32, 8),
+                                                      ("window", 39, 593, 3, 32, 8), ("none", 383, 1112, 1, 32, 8)])
+def test_prefill_append_own_route(kind, n, n_kv, batch, hq, hkv):
+    """Near the line between the general and the grouped kernel, as called by
+    default: appending within the call gives the bits of appending before it."""
+    import gpu_util
+    r = gpu_util.Runner()
+    try:
+        c = prefill(n, n_kv, kind, batch, hq, hkv)
+        k, v = new_rows(c, n, 6300 + n)
+        a = _check_append(r, c, k, v, fused=True)
+        b = _check_append(r, c, k, v, fused=False)
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    finally:
+        r.close()
 
 
 def test_prefill_rope_hd64_long_cache():

@@ -117,13 +117,15 @@ inline int reach_blocks(const AttnArgs& a, int64_t q0, int64_t q1) {
 
 // The general kernel (fa_prefill.hip): a workgroup takes 64 rows of one head and
 // splits its walk over four wavefront groups; 256 run at once. A tensor costs each
-// of them the scan of its rows, a rotary embedding the rotation of its queries
-// (the grouped kernel's are rotated by the append launch: 16/4 heads, 700 rows
-// alone 37.6 -> 32.4 us grouped, 1000 42.1 -> 35.4).
+// of them the scan of its rows, more with every CU at it; a rotary embedding the
+// rotation of its queries (the grouped kernel's are rotated by the append launch:
+// 16/4 heads, 700 rows alone 37.6 -> 32.4 us grouped, 1000 42.1 -> 35.4).
 inline double general128_us(const AttnArgs& a) {
-    const double fix = (a.mask ? 12.8 + 0.107 * ((a.nkv + 31) / 32) : (a.im_causal ? 10.2 : 9.4)) + (a.rope_pos ? 4.0 : 0.0);
-    const double blk = a.mask ? 0.513 : (a.im_causal ? 0.495 : 0.347);
     const int64_t nt = ((int64_t)a.nq + 63) / 64, per = (int64_t)a.hq * a.b, n = nt * per;
+    const double full = n < 256 ? (double)n / 256 : 1.0;
+    const double fix = (a.mask ? 12.0 + 3.0 * full + 0.107 * ((a.nkv + 31) / 32) : (a.im_causal ? 10.2 : 9.4)) +
+                       (a.rope_pos ? 4.0 : 0.0);
+    const double blk = a.mask ? 0.513 : (a.im_causal ? 0.495 : 0.347);
     auto wg = [&](int64_t i) {   // of workgroup i, the last rows' first
         const int64_t t = nt - 1 - i / per, q1 = 64 * t + 64 < a.nq ? 64 * t + 64 : a.nq;
         return fix + blk * reach_blocks(a, 64 * t, q1);
@@ -202,14 +204,18 @@ inline double grouped128_us(const AttnArgs& a, const GroupTiles& g, const GroupP
 // 32/8 heads: 600 rows on 3000 implicit 119 -> 53.7, 10 on 4000 33.7 -> 18.4, 8192
 // alone 1127 -> 550 here; 200 on 320 18.6 -> 23.5, 512 on 88 21.3 -> 32.0, 400
 // unmasked 16.2 -> 22.5 (few rows' work, cut into pieces that have to be merged)
-// there. own_prep: a mask tensor's intervals cost a launch (they ride along with
-// F32 staging or an append): 4.2 us.
+// there. own_prep: a mask tensor's intervals cost a launch, ~4 us, which they do not
+// where they ride along with F32 staging or an append. But appending within the
+// call and appending before it have to give the same bits, so one kernel: both are
+// counted at 2.5 us (at most 3.5 % slower than the general kernel, over 284 sizes of
+// four head counts; a plain call of 383 rows on 1017 40.5 -> 36.5, appended 44.7 -> 36.4).
+// A rotated append is counted without (own_prep false).
 inline bool prefill_group128(const AttnArgs& a, size_t record_bytes, bool own_prep, int force, GroupPlan& plan) {
     if (((((int64_t)a.nq + 31) / 32) << prefill_group_heads_log2(a, kGroupWaves)) < 4 || force == 0) return false;
     const GroupTiles g(a);
     plan = group_pieces(a, g, record_bytes);
     if (force > 0 || g.many()) return true;
-    return general128_us(a) > 1.04 * (grouped128_us(a, g, plan) + (a.mask && own_prep ? 4.2 : 0.0));
+    return general128_us(a) > 1.04 * (grouped128_us(a, g, plan) + (a.mask && own_prep ? 2.5 : 0.0));
 }
 
 // Whether the grouped kernel takes a masked hd 64 call from the pipelined one

@@ -306,8 +306,9 @@ int choose_split(int64_t pairs, int64_t nkv, bool kv_f32, bool* t16) {
 // 256 17.1 -> 16.4, 8192 135 -> 118; F32 3 up to 1000 11.9 -> 14.2, 1500 16.5 ->
 // 14.7, 16 up to 256 13.8 -> 15.5, 300 18.2 -> 16.2, 24 up to 256 (as many
 // splits either way) 20.3 -> 21.2. Where the scan is kept, the pre-pass was 7 to
-// 23 % slower; where it is not, at most 5 % (24 pairs of long rows in many
-// streams of one or two kv heads) and mostly 5 to 50 % faster.
+// 23 % slower; where it is not, at most 10 % (24 pairs of long rows: 4 kv heads, 6
+// streams of F32 from 5600 rows on; 3 full streams of 4000 f16 rows) and mostly 5 to
+// 50 % faster.
 bool rows_by_prepass(const Workspace& w, int64_t nkv, int64_t pairs, bool kv_f32, bool t16) {
     if (w.tune.decode_rows >= 0) return w.tune.decode_rows != 0;
     if (pairs < 24) return false;
@@ -645,7 +646,7 @@ int run(Workspace& w, const vxfa_tensor* q, const vxfa_tensor* k, const vxfa_ten
         const size_t record_bytes = rest < kWorkspaceBytes ? kWorkspaceBytes - rest : 0;
         vxfa::GroupPlan plan{};
         const bool grouped = D == 128 && !pair && (!mask || mrows) &&
-                             vxfa::prefill_group128(a, record_bytes, !staged && !separate, w.tune.group, plan);
+                             vxfa::prefill_group128(a, record_bytes, !staged && !rope, w.tune.group, plan);
         // (scale 0 goes to the general kernel: the pipelined one folds the
         // scale into the exponent and scores the partial block's dead rows -inf)
         const bool pp = D == 64 && (!mask || mrows) && scale != 0.0f && w.tune.pp_enabled &&
