@@ -67,12 +67,14 @@ struct AttnArgs {
     const float* k_new;
     const float* v_new;
     int64_t kn_nb3, vn_nb3;
-    // prefill with a mask tensor (the hd 64 pipelined kernel; the short masked
-    // prefill after F32 staging): per mask row (batch bm_i, plane p, row q at
+    // prefill with a mask tensor (the grouped and the hd 64 pipelined kernel; the
+    // short masked one after F32 staging or an append): per mask row (batch bm_i, plane p, row q at
     // (bm_i * hm + p) * nq + q) the live interval {lo, hi} when the row is 0
     // on [lo, hi] and -inf elsewhere ({n_kv, -1}: no live entry), else
-    // {-2, -2}; written by a pre-pass launch into workspace scratch.
-    // Batched decode with a mask tensor: the rows' live ranges (fa_decode.hip)
+    // {-2, -2}; written into workspace scratch by a pre-pass, a launch of its own
+    // or the first blocks of the one that stages or appends K/V. Batched decode
+    // with a mask row per stream: the rows' live ranges, from rows_by_prepass's
+    // line on (fa_decode.hip)
     int2* mask_rows;
 };
 // (one more cache line of launch arguments is one more cold scalar load before a

@@ -1,5 +1,5 @@
 // fa_decode.hip — single-query (decode-step) attention against a KV cache,
-// split over the KV length, for gfx950. One launch per call.
+// split over the KV length, for gfx950. One to three launches per call.
 //
 // Replaces the backend kernel of GGML_OP_FLASH_ATTN_EXT for the decode calls
 // voxtral.cpp makes from build_decoder_layer (src/voxtral.cpp:1802) with
@@ -9,7 +9,8 @@
 // src/voxtral.cpp:1126-1136); against F32 K/V both products are F32, as in
 // ggml's CPU kernel for F32 K (Q is not rounded to f16).
 //
-// Two kernels on the caller's stream:
+// Two kernels on the caller's stream (after a pre-pass over the mask rows where
+// rows_by_prepass in vxfa_api.cpp asks for one):
 //   fa_decode         grid (n_split * Hkv, B), kDecodeWaves wavefronts per
 //                     workgroup, the kv head fastest-varying (neighbouring
 //                     workgroups stream neighbouring head slices of the same

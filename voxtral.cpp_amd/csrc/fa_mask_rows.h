@@ -48,8 +48,9 @@ __device__ __forceinline__ int wave_sum_dpp(int x) {
 // The pre-pass of a mask tensor: one wavefront per mask row
 // w = (batch bm_i, plane p, row q), w = (bm_i * hm + p) * nq + q, four rows
 // per 256-thread block (mask_rows_kernel, and the first blocks of the launch
-// that also stages F32 K/V, prep_kernel, or that appends new rows, append_prep_kernel); writes out[w] = {lo, hi} when the
-// row's entries are 0 (+0 or -0) on [lo, hi] and -inf elsewhere, {n, -1}
+// that also stages F32 K/V, prep_kernel, or of each row of the launch that
+// appends new rows, kv_append_kernel); writes out[w] = {lo, hi} when the row's
+// entries are 0 (+0 or -0) on [lo, hi] and -inf elsewhere, {n, -1}
 // when every entry is -inf, {-2, -2} otherwise. The row is read as the
 // 16-byte-aligned chunks that cover it (any row alignment; a chunk holds at
 // least one byte of the row, so it lies in the same granule as mask data):
