@@ -26,7 +26,12 @@
  * Query head h reads kv head h / (Hq / Hkv) and mask plane h % Hm.
  *
  * Semantics follow ggml's CPU kernel: a mask entry of -inf removes that kv
- * position; a query row with every position removed produces zeros.
+ * position; a query row with every position removed produces zeros. K and V
+ * at removed positions are not skipped one by one: they may be read and
+ * multiplied by zero where a block of 32 positions (128 in the offline and
+ * realtime encoder's kernel, hd 64) holds a position that one of the tile's
+ * rows attends, so they have to be finite there. Blocks that all of a tile's
+ * rows remove, and rows past n_kv, may hold anything.
  *
  * Everything here is plain C: pointers, sizes and status codes. No HIP or
  * torch types cross the boundary. The stream argument is a hipStream_t
@@ -131,7 +136,10 @@ int vxfa_flash_attn_ext(vxfa_ctx* ctx, const vxfa_tensor* q,
  * (Decoder prefill: offset 0, window 0. Realtime encoder: offset 0, window
  * 750. A decode step with a sliding window W over n_kv cached rows:
  * offset n_kv - 1, window W.) The result equals vxfa_flash_attn_ext with an
- * F16 mask [Nkv, Nq, 1, 1] holding 0 at those positions and -inf elsewhere.
+ * F16 mask [Nkv, Nq, 1, 1] holding 0 at those positions and -inf elsewhere,
+ * within rounding: bit for bit where both forms take the same kernel, as hd
+ * 128 prefill of Nkv <= 512 does; larger calls and decode steps take the
+ * kernel or the splits that are faster for the form.
  * The kernels derive live ranges and tile classes from the formula instead
  * of reading a mask, so no mask is filled, copied or scanned. */
 enum vxfa_mask_kind {
@@ -176,12 +184,14 @@ int vxfa_kv_append(vxfa_ctx* ctx, const vxfa_tensor* k_new,
                    void* stream);
 
 /* vxfa_kv_append(k_new, v_new, k, v) followed by vxfa_flash_attn_ext(q, k,
- * v, mask, dst, ...), with the same result bits. For a single-token decode
- * step (Nq = 1, n_new = 1) the append is fused into the attention kernel:
- * the new row is read once from the F32 source, used, and written to the
- * cache by the same launch; otherwise the append kernel runs first on the
- * same stream. No counterpart in ggml's op: it replaces the two ggml_cpy
- * nodes plus the attention node of each decoder layer (:1758-1802). */
+ * v, mask, dst, ...). For a single-token decode step (Nq = 1, n_new = 1) the
+ * append is fused into the attention kernel: the new row is read once from
+ * the F32 source, used, and written to the cache by the same launch, with the
+ * same cache bytes and a result that differs in the order of the F32 sums
+ * (the new row last; within 1e-5); otherwise the append kernel runs first on
+ * the same stream, with the same result bits. No counterpart in ggml's op:
+ * it replaces the two ggml_cpy nodes plus the attention node of each decoder
+ * layer (:1758-1802). */
 int vxfa_flash_attn_ext_append(vxfa_ctx* ctx, const vxfa_tensor* q,
                                vxfa_tensor* k, vxfa_tensor* v,
                                const vxfa_tensor* k_new,
@@ -244,7 +254,8 @@ typedef struct vxfa_rope {
  * rows, append the new rows (k_new, v_new F32 [Hkv * D, Nq, 1, B]: the new
  * rows are the query tokens, at the last Nq rows of the F16 views k, v),
  * then attend. Equals vxfa_flash_attn_ext_append(rope(q), k, v, rope(k_new),
- * v_new, mask, ...) within the rounding of cos / sin. A decode step is one
+ * v_new, mask, ...) within the rounding of cos / sin and, where a prefill
+ * call takes another kernel, of its order of sums. A decode step is one
  * launch; otherwise the append (with K rotation) runs first. No counterpart
  * in ggml's op: it replaces the two rope nodes, their contiguous copies, the
  * two cache copies and the attention node of a layer. */
