@@ -7,12 +7,12 @@
 // prefill calls of voxtral.cpp (src/voxtral.cpp:1802, GQA 32/8, hd 128, the
 // causal mask of :2104-2111) that the short masked kernel does not take (n_kv
 // over 512, or no mask), where it is faster than the general one
-// (prefill_group128 in fa_prefill_route.h). With head dim 64 also the realtime encoder's calls
-// (:2179-2190) of many workgroups (prefill_group64).
-// Measured, us per layer, before (one head and one wavefront per SIMD) and now:
-// 8192 rows causal 1127 -> 541 (1017 TFLOP/s), 600 rows on 3000 cached, implicit
-// mask 119 -> 53.7, with rope, append and mask tensor 164 -> 60.4, 10 rows on 4000
-// cached 33.7 (uncut prologue, serial merge) -> 18.4.
+// (prefill_group128 in fa_prefill_route.h). With head dim 64 also the realtime
+// encoder's calls (:2179-2190) of many workgroups (prefill_group64).
+// Measured, us per layer, on the general kernel (one head and one wavefront per
+// SIMD) and here: 8192 rows causal 1127 -> 555-563 (~980 TFLOP/s), 600 rows on 3000
+// cached, implicit mask 119 -> 54, with rope, append and mask tensor 164 -> 61, 10
+// rows on 4000 cached 33.7 -> 18.5.
 //
 // Work decomposition
 //   Workgroup = 8 wavefronts (hd 64: 4) of 32 query rows, two per SIMD: HPW
@@ -31,7 +31,7 @@
 //     half t:  MFMA  O += V_{t-1}^T P(t-1)^T, then S(t+1) = K_{t+1} Q^T
 //              VALU  softmax of S(t) -> P(t)
 //   where no MFMA waits for that half's VALU work (at 8192 rows the matrix pipe
-//   is busy 53 % of the cycles at ~1.86 GHz; other orders of the half measured
+//   is busy 50 % of the cycles at ~1.88 GHz; other orders of the half measured
 //   0-4 % slower). K_{t+1} is read at the top
 //   of the half and lands under the PV MFMAs, V_t after them and lands under
 //   the S MFMAs.
@@ -52,8 +52,8 @@
 // the end of an odd walk, a part of the union that only other rows attend)
 // takes a block of zeros for V, so an infinity or NaN at positions that the
 // mask removes from those rows cannot reach them as 0 x V. (8192 rows causal
-// 544 -> 550 us, the realtime encoder's layer 34.8 -> 35.4, with no mask 82.2 ->
-// 79.9 at 2000 rows.)
+// 550 -> 560 us, the realtime encoder's layer 34.5 -> 35.1, with no mask 83.7 ->
+// 81.6 at 2000 rows.)
 #include "fa_common.h"
 #include "fa_prefill_route.h"
 
