@@ -103,6 +103,10 @@ int main() {
         {{32, 8, 128, 1, 8192, 32, TENSOR}, "decode+rows"},
         {{32, 8, 128, 1, 1000, 3, TENSOR, 0, true}, "decode"},
         {{32, 8, 128, 1, 1500, 3, TENSOR, 0, true}, "decode+rows"},
+        {{32, 8, 128, 1, 4096, 3, TENSOR, 0, true}, "decode+rows"},
+        {{32, 8, 128, 1, 4097, 3, TENSOR, 0, true}, "decode"},
+        {{32, 8, 128, 1, 8192, 4, TENSOR, 0, true}, "decode"},
+        {{32, 8, 128, 1, 8192, 5, TENSOR, 0, true}, "decode+rows"},
         {{32, 8, 128, 1, 256, 24, TENSOR, 0, true}, "decode"},
         {{32, 8, 128, 1, 300, 16, TENSOR, 0, true}, "decode+rows"},
         {{8, 2, 128, 1, 8192, 4, TENSOR}, "decode"},
@@ -123,6 +127,10 @@ int main() {
         {{32, 32, 128, 64, 4000, 1, CAUSAL}, "general"},
         {{32, 8, 128, 200, 720, 1, TENSOR}, "general"},
         {{32, 8, 128, 100, 900, 1, TENSOR}, "prep grouped, cut"},
+        {{32, 8, 128, 513, 513, 1, TENSOR}, "general"},
+        {{16, 4, 128, 1025, 1025, 1, TENSOR}, "general"},
+        {{32, 8, 128, 383, 1400, 1, TENSOR}, "prep grouped, cut"},
+        {{32, 8, 128, 700, 1000, 1, TENSOR}, "prep grouped, cut"},
         {{32, 8, 128, 600, 3600, 1, TENSOR, 0, true}, "prep grouped, cut"},
         {{32, 8, 128, 600, 3600, 1, TENSOR, 0, false, true}, "append grouped, cut"},
         {{16, 4, 128, 1000, 1000, 1, TENSOR, 0, false, true}, "append grouped, cut"},

@@ -10,8 +10,9 @@
     choice, workspace and scratch placement, F32 staging, implicit masks,
     ring, append, rope, no-alloc) by tests/sanitize/run_fuzz.cpp: the HIP
     runtime calls replaced by host stand-ins and the launchers by stubs that
-    check the kernels' argument assumptions (records and staging inside one
-    workspace allocation, the mask interval table clear of staged K/V);
+    check the kernels' argument assumptions (records, piece records, staging,
+    rotated queries and mask tables inside one workspace allocation and clear
+    of each other);
   * ThreadSanitizer over the oracle's threaded routines (the scalar
     restatement and the vectorised baseline's thread pool) by
     tests/sanitize/oracle_threads.c.

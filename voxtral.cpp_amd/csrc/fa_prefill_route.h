@@ -122,8 +122,8 @@ inline int reach_blocks(const AttnArgs& a, int64_t q0, int64_t q1) {
 // 16/4 heads, 700 rows alone 37.6 -> 32.4 us grouped, 1000 42.1 -> 35.4).
 inline double general128_us(const AttnArgs& a) {
     const int64_t nt = ((int64_t)a.nq + 63) / 64, per = (int64_t)a.hq * a.b, n = nt * per;
-    const double full = n < 256 ? (double)n / 256 : 1.0;
-    const double fix = (a.mask ? 12.0 + 3.0 * full + 0.107 * ((a.nkv + 31) / 32) : (a.im_causal ? 10.2 : 9.4)) +
+    const double scan = n <= 256 ? 12.0 + 3.0 * (double)n / 256 : 12.8;   // (later rounds start apart)
+    const double fix = (a.mask ? scan + 0.107 * ((a.nkv + 31) / 32) : (a.im_causal ? 10.2 : 9.4)) +
                        (a.rope_pos ? 4.0 : 0.0);
     const double blk = a.mask ? 0.513 : (a.im_causal ? 0.495 : 0.347);
     auto wg = [&](int64_t i) {   // of workgroup i, the last rows' first
@@ -207,15 +207,17 @@ inline double grouped128_us(const AttnArgs& a, const GroupTiles& g, const GroupP
 // there. own_prep: a mask tensor's intervals cost a launch, ~4 us, which they do not
 // where they ride along with F32 staging or an append. But appending within the
 // call and appending before it have to give the same bits, so one kernel: both are
-// counted at 2.5 us (at most 3.5 % slower than the general kernel, over 284 sizes of
-// four head counts; a plain call of 383 rows on 1017 40.5 -> 36.5, appended 44.7 -> 36.4).
-// A rotated append is counted without (own_prep false).
+// counted at 2.5 us, or 4.5 where the general kernel has more than a round of
+// workgroups (over 424 sizes of four head counts the plain call is then at most 3.8 %
+// slower than on the general kernel; 383 rows on 1017 40.6 -> 36.5, appended 44.7 ->
+// 36.4). A rotated append is counted without (own_prep false).
 inline bool prefill_group128(const AttnArgs& a, size_t record_bytes, bool own_prep, int force, GroupPlan& plan) {
     if (((((int64_t)a.nq + 31) / 32) << prefill_group_heads_log2(a, kGroupWaves)) < 4 || force == 0) return false;
     const GroupTiles g(a);
     plan = group_pieces(a, g, record_bytes);
     if (force > 0 || g.many()) return true;
-    return general128_us(a) > 1.04 * (grouped128_us(a, g, plan) + (a.mask && own_prep ? 2.5 : 0.0));
+    const bool one_round = ((int64_t)a.nq + 63) / 64 * a.hq * a.b <= 256;
+    return general128_us(a) > 1.04 * (grouped128_us(a, g, plan) + (a.mask && own_prep ? (one_round ? 2.5 : 4.5) : 0.0));
 }
 
 // Whether the grouped kernel takes a masked hd 64 call from the pipelined one

@@ -306,14 +306,17 @@ int choose_split(int64_t pairs, int64_t nkv, bool kv_f32, bool* t16) {
 // 256 17.1 -> 16.4, 8192 135 -> 118; F32 3 up to 1000 11.9 -> 14.2, 1500 16.5 ->
 // 14.7, 16 up to 256 13.8 -> 15.5, 300 18.2 -> 16.2, 24 up to 256 (as many
 // splits either way) 20.3 -> 21.2. Where the scan is kept, the pre-pass was 7 to
-// 23 % slower; where it is not, at most 10 % (24 pairs of long rows: 4 kv heads, 6
-// streams of F32 from 5600 rows on; 3 full streams of 4000 f16 rows) and mostly 5 to
-// 50 % faster.
+// 23 % slower; where it is not, mostly 5 to 50 % faster. With few long streams it
+// goes by their lengths: 3 F32 streams of up to 8192 rows 25 % faster, 16 and 10 %
+// slower (three draws; 12 to 48 splits a stream instead no better), 4 even to 10 %
+// slower, 5 13 % faster to 8 % slower: F32 of less than 40 pairs over more than 4096
+// rows keeps the scan. Left: up to 10 % slower at 3 F32 streams of 2000 to 4096 rows
+// and 3 full f16 ones of 4000.
 bool rows_by_prepass(const Workspace& w, int64_t nkv, int64_t pairs, bool kv_f32, bool t16) {
     if (w.tune.decode_rows >= 0) return w.tune.decode_rows != 0;
     if (pairs < 24) return false;
     // (f16: choose_split's own line between tiles of 16 and of 32)
-    return kv_f32 ? nkv > 256 && nkv * pairs > 2048 * 16 : !t16;
+    return kv_f32 ? nkv > 256 && nkv * pairs > 2048 * 16 && (pairs >= 40 || nkv <= 4096) : !t16;
 }
 
 // The split count a workspace of rec_bytes can hold: pairs * S records of
