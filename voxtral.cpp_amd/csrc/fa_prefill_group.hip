@@ -10,7 +10,7 @@
 // (prefill_group128 in fa_prefill_route.h). With head dim 64 also the realtime
 // encoder's calls (:2179-2190) of many workgroups (prefill_group64).
 // Measured, us per layer, on the general kernel (one head and one wavefront per
-// SIMD) and here: 8192 rows causal 1127 -> 555-563 (~980 TFLOP/s), 600 rows on 3000
+// SIMD) and here: 8192 rows causal 1127 -> 546-567 (~980 TFLOP/s), 600 rows on 3000
 // cached, implicit mask 119 -> 54, with rope, append and mask tensor 164 -> 61, 10
 // rows on 4000 cached 33.7 -> 18.5.
 //
